@@ -31,6 +31,7 @@ enum FmGemmFlags {
   FM_EPI_RES_SCALE = 32, // y = res + scale[n] * acc
   FM_WEIGHTS_X6 = 64,    // weight_packed is followed by its three bf16 planes (fm_split_weights)
   FM_ACT_EXP = 128,      // residual blocks: ELUs as e^x - 1 (fm_elu_exp), for decoder-side calls
+  FM_WEIGHTS_H3 = 512,   // the bf16 planes are followed by the fp16 planes (fm_split_weights_h3)
   FM_EPI_ROPE = 256      // internal (fm_linear_rope): RoPE on the first rope_cols output columns
 };
 
@@ -119,6 +120,31 @@ FM_DEVICE void split3(floatx4 v, bf16x4& h0, bf16x4& h1, bf16x4& h2) {
   h0 = __builtin_bit_cast(bf16x4, (uintx2_t{p0[0], p0[1]}));
   h1 = __builtin_bit_cast(bf16x4, (uintx2_t{p1[0], p1[1]}));
   h2 = __builtin_bit_cast(bf16x4, (uintx2_t{p2[0], p2[1]}));
+}
+
+// h3 primitives: one v_mfma_f32_32x32x16_f16 (lane layout of fm_mfma32_bf16)
+// and the two-piece fp16 split of eight FP32 values scaled by a power of two:
+// v * sc = h0 + h1 to within 2^-23 |v * sc| (|v * sc| below 2^16).
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
+
+FM_DEVICE floatx16 fm_mfma32_f16(halfx8 a, halfx8 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+FM_DEVICE void split2(floatx4 lo, floatx4 hi, float sc, halfx8& h0, halfx8& h1) {
+  typedef _Float16 halfx2_t __attribute__((ext_vector_type(2)));
+  typedef float floatx2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float a = q < 2 ? lo[2 * q] : hi[2 * q - 4], b = q < 2 ? lo[2 * q + 1] : hi[2 * q - 3];
+    const halfx2_t p = __builtin_convertvector((floatx2_t{a * sc, b * sc}), halfx2_t);
+    // The residual a sc - h0 is exact in FP32.
+    const halfx2_t r = __builtin_convertvector(
+        (floatx2_t{fmaf(a, sc, -(float)p[0]), fmaf(b, sc, -(float)p[1])}), halfx2_t);
+    h0[2 * q] = p[0], h0[2 * q + 1] = p[1];
+    h1[2 * q] = r[0], h1[2 * q + 1] = r[1];
+  }
 }
 
 static inline int fm_ceil_div(long a, long b) { return (int)((a + b - 1) / b); }

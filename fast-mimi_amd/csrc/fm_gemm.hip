@@ -1112,6 +1112,112 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restr
 }
 
 // ---------------------------------------------------------------------------
+// Epilogue of the 16-bit MFMA tiles, straight from the accumulators (no LDS
+// pass, no barrier): lane
+// l of a 32x32 accumulator holds column l % 32 of rows
+// 8 (r / 4) + 4 (l / 32) + r % 4, so each store instruction writes two
+// 128-byte row segments.  Stores and residual loads go through buffer
+// resources over this tile's rows, so past-M rows and past-N columns
+// (offset INT_MIN) are dropped / read as zero without a branch.  An
+// accumulator's residuals are all loaded before its first store, its RoPE
+// factors eight rows at a time: the compiler does not move a load above a
+// store to y (which may alias the residual), so each would otherwise wait
+// out a memory round trip.  RoPE's partner column c ^ 32 of a 64-column head is the same
+// lane's accumulator of the neighbouring 32-column tile (wave tiles start
+// on 64-column boundaries).
+enum TileRope { ROPE_NEVER, ROPE_FLAG, ROPE_ALWAYS };  // whether the tile rotates: p.flags says, or the kernel
+template <int BM, int FM, int FN, TileRope ROT>
+FM_DEVICE void tile_epilogue(const GemmArgs& p, floatx16 (&acc)[FM][FN], long M, long m0, int n0, int wm0,
+                             int wn0, int lane) {
+  const int lcol = lane & 31;
+  float* part = p.partial ? p.partial + (long)blockIdx.y * M * p.N : nullptr;
+  const bool has_res = (p.flags & (FM_EPI_RES_ADD | FM_EPI_RES_SCALE)) && !part;
+  const bool scaled = (p.flags & FM_EPI_RES_SCALE) && !part;
+  const int tile_bytes = (int)min((long)BM, M - m0) * p.N * 4;
+  const __amdgpu_buffer_rsrc_t ry = fm_buffer((part ? part : p.y) + m0 * p.N, tile_bytes);
+  const __amdgpu_buffer_rsrc_t rr = fm_buffer(has_res ? p.res + m0 * p.N : p.y, has_res ? tile_bytes : 0);
+  // Cropped outputs: row m = b rows + t goes to row b y_rows + t when
+  // t < y_rows; over a tile those rows rise by at most one per row, so they
+  // lie within BM + 1 rows of the tile's first one (crop0).
+  int crop0 = 0;
+  if (p.y_rows != p.rows) {
+    const int b0 = (int)fm_div((unsigned)m0, p.rows_div);
+    crop0 = b0 * p.y_rows + min((int)m0 - b0 * p.rows, p.y_rows);
+  }
+  const __amdgpu_buffer_rsrc_t rc = fm_buffer(p.y + (long)crop0 * p.N, (BM + 1) * p.N * 4);
+  static_assert(ROT == ROPE_NEVER || (32 * FN) % 64 == 0, "RoPE partners within the wave tile");
+  auto epilogue = [&](auto crop_c, auto rope_c) {
+    constexpr bool CROP = decltype(crop_c)::value, ROPE = decltype(rope_c)::value;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int c = wn0 + 32 * j + lcol;
+      const int n = n0 + c;
+      const bool n_ok = n < p.N;
+      const int ncl = n_ok ? n : 0;
+      const bool rope = ROPE && n < p.rope_cols;
+      const float bias = (p.bias && !part) ? p.bias[ncl % p.bias_len] : 0.0f;
+      const float scale = scaled ? p.scale[ncl] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int rb = wm0 + 32 * i;
+        // Lane offset of the accumulator's first row; row 8 (r / 4) + r % 4
+        // further down is a wave-uniform scalar offset.
+        const int voff = n_ok ? ((rb + 4 * (lane >> 5)) * p.N + n) * 4 : INT_MIN;
+        auto soff = [&](int r) { return (8 * (r >> 2) + (r & 3)) * p.N * 4; };
+        float res[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) res[r] = (!ROPE && has_res) ? fm_buf_load1(rr, voff, soff(r)) : 0.0f;
+        // RoPE factors in two halves of eight rows (all sixteen at once
+        // would spill).
+        float cs[8], sn[8];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          float v = acc[i][j][r];
+          if constexpr (ROPE) {
+            if (r % 8 == 0) {
+#pragma unroll
+              for (int q = 0; q < 8; ++q) {
+                const int m = (int)min(m0 + rb + fm_mfma32_row(r + q, lane), M - 1);
+                const int t = m - (int)fm_div((unsigned)m, p.seq_div) * p.rows_per_seq;
+                cs[q] = rope ? p.rope_cos[t * 64 + (c & 63)] : 1.0f;
+                sn[q] = rope ? p.rope_sin[t * 64 + (c & 63)] : 0.0f;
+              }
+            }
+            // x*cos - x[d+32]*sin for d < 32, x*cos + x[d-32]*sin after; each
+            // product and the sum rounded separately.
+            const float pv = acc[i][j ^ 1][r];
+            if (rope) v = __fadd_rn(__fmul_rn(v, cs[r % 8]), __fmul_rn((j & 1) ? pv : -pv, sn[r % 8]));
+          }
+          if (!part) v = epilogue_v(v, bias, res[r], scale, p.flags);
+          if constexpr (CROP) {
+            const int m = (int)m0 + rb + fm_mfma32_row(r, lane);
+            const int b = (int)fm_div((unsigned)m, p.rows_div);
+            const int t = m - b * p.rows;
+            const bool ok = m < M && n_ok && t < p.y_rows;
+            fm_buf_store1(v, rc, ok ? ((b * p.y_rows + t - crop0) * p.N + n) * 4 : INT_MIN, 0);
+          } else {
+            fm_buf_store1(v, ry, voff, soff(r));
+          }
+        }
+      }
+    }
+  };
+  using yes = std::true_type;
+  using no = std::false_type;
+  const bool crop = p.y_rows != p.rows && !part;
+  if (ROT == ROPE_ALWAYS || (ROT == ROPE_FLAG && (p.flags & FM_EPI_ROPE))) {
+    if constexpr (ROT != ROPE_NEVER) {
+      if (crop) epilogue(yes{}, yes{});
+      else epilogue(no{}, yes{});
+    }
+  } else if constexpr (ROT != ROPE_ALWAYS) {
+    if (crop) epilogue(yes{}, no{});
+    else epilogue(no{}, no{});
+  }
+}
+
+
+// ---------------------------------------------------------------------------
 // bf16x6 tile with the FP32 A operand loaded global -> LDS directly: each
 // lane's 16-byte chunk of the 16-deep A k-tile lands in an XOR-swizzled slot
 // (chunk c of row r at position c ^ ((r / 4) & 3), so the 16-lane groups of a
@@ -1326,101 +1432,273 @@ void gemm_x6d_kernel(GemmArgs p, const __bf16* __restrict__ w3) {
       if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
     }
   }
-  // Epilogue straight from the accumulators (no LDS pass, no barrier): lane
-  // l of a 32x32 accumulator holds column l % 32 of rows
-  // 8 (r / 4) + 4 (l / 32) + r % 4, so each store instruction writes two
-  // 128-byte row segments.  Stores and residual loads go through buffer
-  // resources over this tile's rows, so past-M rows and past-N columns
-  // (offset INT_MIN) are dropped / read as zero without a branch.  An
-  // accumulator's residuals are all loaded before its first store, its RoPE
-  // factors eight rows at a time: the compiler does not move a load above a
-  // store to y (which may alias the residual), so each would otherwise wait
-  // out a memory round trip.  RoPE's partner column c ^ 32 of a 64-column head is the same
-  // lane's accumulator of the neighbouring 32-column tile (wave tiles start
-  // on 64-column boundaries).
-  const int lcol = lane & 31;
-  float* part = p.partial ? p.partial + (long)blockIdx.y * M * p.N : nullptr;
-  const bool has_res = (p.flags & (FM_EPI_RES_ADD | FM_EPI_RES_SCALE)) && !part;
-  const bool scaled = (p.flags & FM_EPI_RES_SCALE) && !part;
-  const int tile_bytes = (int)min((long)BM, M - m0) * p.N * 4;
-  const __amdgpu_buffer_rsrc_t ry = fm_buffer((part ? part : p.y) + m0 * p.N, tile_bytes);
-  const __amdgpu_buffer_rsrc_t rr = fm_buffer(has_res ? p.res + m0 * p.N : p.y, has_res ? tile_bytes : 0);
-  // Cropped outputs: row m = b rows + t goes to row b y_rows + t when
-  // t < y_rows; over a tile those rows rise by at most one per row, so they
-  // lie within BM + 1 rows of the tile's first one (crop0).
-  int crop0 = 0;
-  if (p.y_rows != p.rows) {
-    const int b0 = (int)fm_div((unsigned)m0, p.rows_div);
-    crop0 = b0 * p.y_rows + min((int)m0 - b0 * p.rows, p.y_rows);
+  tile_epilogue<BM, FM, FN, ELU ? ROPE_NEVER : ROPE_FLAG>(p, acc, M, m0, n0, wm0, wn0, lane);
+}
+
+// ---------------------------------------------------------------------------
+// FP32 contraction on the fp16 matrix cores ("h3").  An FP32 operand scaled by
+// a power of two is h0 + h1 (each a round-to-nearest fp16, 11 bits) to within
+// 2^-23 of its magnitude, and a product is the three terms a1b0 + a0b1 + a0b0;
+// the dropped a1b1 is below 2^-22 |a b| and of either sign.  Half of the
+// bf16x6 form's MFMA work, two planes in LDS instead of three and 28 vector
+// instructions per eight A elements instead of 44; with half as many roundings
+// into the FP32 accumulator its error against float64 is smaller too (rms over
+// the decoder's shapes 1.4-3.6e-7 of the output scale, bf16x6 1.7-4.9e-7).
+// fp16's range is what the scales are for:
+//   * a weight row n (one output column) is scaled by 2^s_n so that its largest
+//     magnitude lies in [2^13, 2^14) (fm_split_weights_h3; s_n is stored);
+//   * an A row is scaled by its own power of two, taken from the first k-tile
+//     in which the row is not zero (largest magnitude in [2^9, 2^10)) and
+//     lowered, with the row's accumulators, when a later element would leave
+//     fp16's range (|a| 2^s > 2^15).  The test is one running maximum of the
+//     eight elements a lane holds; the rescale is a rarely taken branch.
+//     So h1 is exact to 2^-25 at a row maximum of at least 2^9: 2^-34 of it,
+//     whatever the data's scale, quiet and loud rows in one tile included.
+// A non-finite element makes its row NaN, as the bf16 split does.
+//
+// Planes per weight: [2][K/16][N][16] fp16 in the bf16x6 planes' k16-tile order,
+// then int s_n [N].
+FM_DEVICE int h3_exp_field(float v) { return (int)(__builtin_bit_cast(unsigned, v) >> 23) & 255; }
+// 2^s as a float and the largest magnitude it may meet, for a row maximum m > 0
+// (s puts m in [2^9, 2^10); the exponent fields are clamped to normal numbers).
+FM_DEVICE int h3_scale_exp(float m) { return min(max(263 - h3_exp_field(m), 1), 253) - 127; }
+FM_DEVICE float h3_limit(float m) {
+  const int f = h3_exp_field(m) + 6;
+  return __builtin_bit_cast(float, (unsigned)min(f, 255) << 23);  // 2^15 / 2^s, or inf
+}
+
+__global__ __launch_bounds__(256) void split_weights_h3_kernel(const float* __restrict__ w, int N, int K,
+                                                               _Float16* __restrict__ out) {
+  const int n = blockIdx.x, tid = threadIdx.x;
+  const float* row = w + (long)n * K;
+  float m = 0.0f;
+  for (int k = tid; k < K; k += 256) m = fmaxf(m, fabsf(row[k]));
+  __shared__ float part[256];
+  part[tid] = m;
+  __syncthreads();
+  for (int d = 128; d > 0; d >>= 1) {
+    if (tid < d) part[tid] = fmaxf(part[tid], part[tid + d]);
+    __syncthreads();
   }
-  const __amdgpu_buffer_rsrc_t rc = fm_buffer(p.y + (long)crop0 * p.N, (BM + 1) * p.N * 4);
-  static_assert(WTN % 64 == 0, "RoPE partners within the wave tile");
-  auto epilogue = [&](auto crop_c, auto rope_c) {
-    constexpr bool CROP = decltype(crop_c)::value, ROPE = decltype(rope_c)::value;
+  // The row maximum in [2^13, 2^14); a zero row keeps s = 0.
+  const float top = part[0];
+  const int s = top > 0.0f ? min(max(267 - h3_exp_field(top), 1), 253) - 127 : 0;
+  const float sc = __builtin_bit_cast(float, (unsigned)(s + 127) << 23);
+  const long NK = (long)N * K;
+  if (tid == 0) reinterpret_cast<int*>(out + 2 * NK)[n] = s;
+  for (int k = tid; k < K; k += 256) {
+    const float v = row[k] * sc;
+    const _Float16 h = (_Float16)v;
+    const long o = ((long)(k >> 4) * N + n) * 16 + (k & 15);
+    out[o] = h;
+    out[NK + o] = (_Float16)(v - (float)h);
+  }
+}
+
+// The tile: A k-tiles travel global -> LDS as FP32 and the two weight planes
+// beside them, in the layouts and with the two-stage ring of gemm_x6d_kernel;
+// each wave reads, scales and splits the A fragments of its rows and runs the
+// three products a1b0, a0b1, a0b0 per fragment pair.  WPE: waves per SIMD the
+// registers are held to.
+template <int BM, int BN, int WM, int WN, int KS, int WPE, bool ELU, bool ROPE = false>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WPE)))
+void gemm_h3_kernel(GemmArgs p, const _Float16* __restrict__ wh) {
+  constexpr int NW = WM * WN, BK = 16 * KS;
+  constexpr int WTM = BM / WM, WTN = BN / WN, FM = WTM / 32, FN = WTN / 32;
+  // A: 16-byte chunks per row, rows per load instruction, swizzle period (as
+  // gemm_x6d_kernel).
+  constexpr int CPR = 4 * KS, RPI = 64 / CPR, SWR = 16 / CPR;
+  constexpr int AI = BM / (NW * RPI);
+  static_assert(AI >= 1 && AI * NW * RPI == BM && FM >= 1 && FN >= 1 && BN % 32 == 0, "tiling");
+  constexpr int PLANE_B = BN * BK * 2, STAGE_A = BM * BK * 4, STAGE = STAGE_A + 2 * PLANE_B;
+  constexpr int NBI = 2 * KS * BN / 32;  // 1 KB B load instructions per stage
+  __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+  // Each wave's row exponents (rescale steps, then the final s of each row).
+  __shared__ __attribute__((aligned(16))) int row_exp[NW][WTM];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm0 = (wave / WN) * WTM, wn0 = (wave % WN) * WTN;
+  const long M = (long)p.batch * p.rows;
+  const int tiles_n = (p.N + BN - 1) / BN;
+  const int tile = tile_index();
+  const long m0 = (long)(tile / tiles_n) * BM;
+  const int n0 = (tile % tiles_n) * BN;
+  const int k_begin = blockIdx.y * p.k_split;
+  const int k_end = min(p.K, k_begin + p.k_split);
+
+  const int lr = lane / CPR, cp = lane % CPR;
+  const float* a_row[AI];
+  int a_p0[AI], a_voff[AI];
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int c = wn0 + 32 * j + lcol;
-      const int n = n0 + c;
-      const bool n_ok = n < p.N;
-      const int ncl = n_ok ? n : 0;
-      const bool rope = ROPE && n < p.rope_cols;
-      const float bias = (p.bias && !part) ? p.bias[ncl % p.bias_len] : 0.0f;
-      const float scale = scaled ? p.scale[ncl] : 0.0f;
+  for (int i = 0; i < AI; ++i) {
+    const int r = (wave * AI + i) * RPI + lr;
+    const long mm = m0 + r;
+    const int m = (int)min(mm, M - 1);
+    const int b = (int)fm_div((unsigned)m, p.rows_div);
+    const int t = m - b * p.rows;
+    a_p0[i] = mm < M ? t * p.rs - p.padL : INT_MIN / 2;
+    a_row[i] = p.x + (long)b * p.L_in * p.C_in + (long)a_p0[i] * p.C_in + 4 * (cp ^ ((r / SWR) & (CPR - 1)));
+    a_voff[i] = (int)((a_row[i] - p.x) * 4);
+  }
+  const long x_bytes = (long)p.batch * p.L_in * p.C_in * 4;
+  const bool a_buf = x_bytes < 0x7fffffffL;
+  const __amdgpu_buffer_rsrc_t ra = fm_buffer(p.x, a_buf ? (int)x_bytes : 0);
+  const long KN = (long)p.K * p.N;
+  constexpr int NBW = (NBI + NW - 1) / NW;
+  const __amdgpu_buffer_rsrc_t rb = fm_buffer(wh, (int)(2 * KN * 2));
+  int b_voff[NBW], b_lds[NBW];
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int rb = wm0 + 32 * i;
-        // Lane offset of the accumulator's first row; row 8 (r / 4) + r % 4
-        // further down is a wave-uniform scalar offset.
-        const int voff = n_ok ? ((rb + 4 * (lane >> 5)) * p.N + n) * 4 : INT_MIN;
-        auto soff = [&](int r) { return (8 * (r >> 2) + (r & 3)) * p.N * 4; };
-        float res[16];
+  for (int q = 0; q < NBW; ++q) {
+    const int i = min(wave + q * NW, NBI - 1);
+    const int pl = i / (KS * BN / 32), kt = i % (KS * BN / 32) / (BN / 32), rg = i % (BN / 32);
+    const int row = rg * 32 + (lane & 31);  // LDS as [k-half][row] (see gemm_x6d_kernel)
+    b_voff[q] = n0 + row < p.N ? (int)((pl * KN + (long)kt * p.N * 16 + (long)(n0 + row) * 16 + 8 * (lane >> 5)) * 2)
+                               : INT_MIN;
+    b_lds[q] = pl * PLANE_B + kt * BN * 32 + rg * 1024;
+  }
+  auto issue = [&](int stage, int k0) {
+    char* As = smem + stage * STAGE;
+    char* Bs = As + STAGE_A;
+    const int tap = k0 / p.C_in;  // uniform: a k-tile lies in one tap
+    if (a_buf) {
+      const int tap_off = tap * p.C_in * 4, soff = k0 * 4 - tap_off;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) res[r] = (!ROPE && has_res) ? fm_buf_load1(rr, voff, soff(r)) : 0.0f;
-        // RoPE factors in two halves of eight rows (all sixteen at once
-        // would spill).
-        float cs[8], sn[8];
+      for (int i = 0; i < AI; ++i) {
+        const bool ok = (unsigned)(a_p0[i] + tap) < (unsigned)p.L_in;
+        fm_buf_load_lds16(ra, As + (wave * AI + i) * RPI * BK * 4, ok ? a_voff[i] + tap_off : INT_MIN, soff);
+      }
+    } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float v = acc[i][j][r];
-          if constexpr (ROPE) {
-            if (r % 8 == 0) {
-#pragma unroll
-              for (int q = 0; q < 8; ++q) {
-                const int m = (int)min(m0 + rb + fm_mfma32_row(r + q, lane), M - 1);
-                const int t = m - (int)fm_div((unsigned)m, p.seq_div) * p.rows_per_seq;
-                cs[q] = rope ? p.rope_cos[t * 64 + (c & 63)] : 1.0f;
-                sn[q] = rope ? p.rope_sin[t * 64 + (c & 63)] : 0.0f;
-              }
-            }
-            // x*cos - x[d+32]*sin for d < 32, x*cos + x[d-32]*sin after; each
-            // product and the sum rounded separately.
-            const float pv = acc[i][j ^ 1][r];
-            if (rope) v = __fadd_rn(__fmul_rn(v, cs[r % 8]), __fmul_rn((j & 1) ? pv : -pv, sn[r % 8]));
-          }
-          if (!part) v = epilogue_v(v, bias, res[r], scale, p.flags);
-          if constexpr (CROP) {
-            const int m = (int)m0 + rb + fm_mfma32_row(r, lane);
-            const int b = (int)fm_div((unsigned)m, p.rows_div);
-            const int t = m - b * p.rows;
-            const bool ok = m < M && n_ok && t < p.y_rows;
-            fm_buf_store1(v, rc, ok ? ((b * p.y_rows + t - crop0) * p.N + n) * 4 : INT_MIN, 0);
-          } else {
-            fm_buf_store1(v, ry, voff, soff(r));
-          }
-        }
+      for (int i = 0; i < AI; ++i) {
+        const bool ok = (unsigned)(a_p0[i] + tap) < (unsigned)p.L_in;
+        const float* src = ok ? a_row[i] + k0 : g_zero16;
+        __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)(As + (wave * AI + i) * RPI * BK * 4),
+                                         16, 0, 0);
       }
     }
+    const int soff = (k0 >> 4) * p.N * 32;
+#pragma unroll
+    for (int q = 0; q < NBW; ++q)
+      if (wave + q * NW < NBI) fm_buf_load_lds16(rb, Bs + b_lds[q], b_voff[q], soff);
   };
-  using yes = std::true_type;
-  using no = std::false_type;
-  const bool crop = p.y_rows != p.rows && !part;
-  if (!ELU && (p.flags & FM_EPI_ROPE)) {
-    if (crop) epilogue(yes{}, yes{});
-    else epilogue(no{}, yes{});
-  } else {
-    if (crop) epilogue(yes{}, no{});
-    else epilogue(no{}, no{});
+
+  floatx16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  const int lrow = lane & 31, lk = lane >> 5;
+  // Per fragment row (lanes l and l + 32 hold one row): its scale 2^s, s, and
+  // the magnitude it covers (0: the row has been zero so far).
+  float sc[FM], lim[FM];
+  int se[FM];
+#pragma unroll
+  for (int i = 0; i < FM; ++i) sc[i] = 1.0f, lim[i] = 0.0f, se[i] = 0;
+  // acc[i][.][r] *= 2^row_exp[wave][row of r], rows of wave fragment i.
+  auto scale_rows = [&](int i, int col_exp, floatx16& a) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int4 e = *reinterpret_cast<const int4*>(&row_exp[wave][32 * i + 8 * q + 4 * lk]);
+      a[4 * q] = __builtin_amdgcn_ldexpf(a[4 * q], e.x + col_exp);
+      a[4 * q + 1] = __builtin_amdgcn_ldexpf(a[4 * q + 1], e.y + col_exp);
+      a[4 * q + 2] = __builtin_amdgcn_ldexpf(a[4 * q + 2], e.z + col_exp);
+      a[4 * q + 3] = __builtin_amdgcn_ldexpf(a[4 * q + 3], e.w + col_exp);
+    }
+  };
+
+  const int nkt = (k_end - k_begin) / BK;
+  if (nkt > 0) issue(0, k_begin);
+  for (int kt = 0; kt < nkt; ++kt) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (kt + 1 < nkt) issue((kt + 1) & 1, k_begin + (kt + 1) * BK);
+    const char* As = smem + (kt & 1) * STAGE;
+    const char* Bs = As + STAGE_A;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      floatx4 v[FM][2];
+      float top[FM];
+      bool out = false;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int row = wm0 + 32 * i + lrow;
+        const int sw = (row / SWR) & (CPR - 1);
+        v[i][0] = *reinterpret_cast<const floatx4*>(As + row * BK * 4 + 16 * ((4 * ks + 2 * lk) ^ sw));
+        v[i][1] = *reinterpret_cast<const floatx4*>(As + row * BK * 4 + 16 * ((4 * ks + 2 * lk + 1) ^ sw));
+        if constexpr (ELU) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[i][0][e] = fm_elu(v[i][0][e]), v[i][1][e] = fm_elu(v[i][1][e]);
+        }
+        float m = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = fmaxf(fmaxf(m, fabsf(v[i][0][e])), fabsf(v[i][1][e]));
+        top[i] = m;
+        out |= m > lim[i];
+      }
+      if (__builtin_expect(__any(out), 0)) {
+        // Some row outgrew its scale (or is the first non-zero one): new
+        // scales, and the accumulators follow.
+        wave_lds_fence();
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          const float m = fmaxf(top[i], __shfl_xor(top[i], 32));
+          int step = 0;
+          if (m > lim[i]) {
+            const int s = h3_scale_exp(m);
+            step = lim[i] > 0.0f ? s - se[i] : 0;
+            se[i] = s;
+            sc[i] = __builtin_bit_cast(float, (unsigned)(s + 127) << 23);
+            lim[i] = h3_limit(m);
+          }
+          if (lane < 32) row_exp[wave][32 * i + lane] = step;
+        }
+        wave_lds_fence();
+        // The accumulators are read 19 cycles or more after the last MFMA.
+        asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) scale_rows(i, 0, acc[i][j]);
+      }
+      halfx8 a0[FM], a1[FM], b0[FN], b1[FN];
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const char* bb = Bs + ks * BN * 32 + (wn0 + 32 * j) * 32 + lk * 512 + lrow * 16;
+        b0[j] = *reinterpret_cast<const halfx8*>(bb);
+        b1[j] = *reinterpret_cast<const halfx8*>(bb + PLANE_B);
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i) split2(v[i][0], v[i][1], sc[i], a0[i], a1[i]);
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          acc[i][j] = fm_mfma32_f16(a1[i], b0[j], acc[i][j]);
+          acc[i][j] = fm_mfma32_f16(a0[i], b1[j], acc[i][j]);
+          acc[i][j] = fm_mfma32_f16(a0[i], b0[j], acc[i][j]);
+        }
+    }
   }
+  // Back to the caller's scale: 2^-(s_row + s_column) in one exact step.
+  wave_lds_fence();
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+    if (lane < 32) row_exp[wave][32 * i + lane] = -se[i];
+  wave_lds_fence();
+  const int* col_exp = reinterpret_cast<const int*>(wh + 2 * KN);
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int n = n0 + wn0 + 32 * j + lrow;
+    const int e = n < p.N ? -col_exp[n] : 0;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) scale_rows(i, e, acc[i][j]);
+  }
+  tile_epilogue<BM, FM, FN, ROPE ? ROPE_ALWAYS : ROPE_NEVER>(p, acc, M, m0, n0, wm0, wn0, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1561,6 +1839,11 @@ constexpr TileCfg kX6Wide = {192, 128, 1, 32, 19, 0};  // direct-load A, twelve 
 constexpr TileCfg kX6K32 = {128, 128, 1, 32, 20, 0};
 constexpr TileCfg kX6WideK32 = {192, 128, 1, 32, 22, 0};
 constexpr TileCfg kDl192 = {192, 128, 1, 32, 14, 0};
+// h3 tiles (gemm_h3_kernel), waves of 64x64 / 32x64 / 32x64 / 32x32.
+constexpr TileCfg kH3 = {128, 128, 1, 32, 24, 0};       // 16-deep k-tiles, 33 KB: four blocks per CU
+constexpr TileCfg kH3K32 = {128, 128, 1, 32, 25, 0};    // 32-deep, 65 KB: two blocks per CU
+constexpr TileCfg kH3Small = {64, 128, 1, 32, 26, 0};   // 32-deep, 49 KB: three blocks per CU
+constexpr TileCfg kH3Tiny = {64, 64, 1, 64, 27, 0};     // 64-deep, 65 KB: two blocks per CU
 // 64x128 runs one block per CU: 64-deep k-tiles (96 KB ring) halve its barriers.
 constexpr TileCfg kDl64 = {64, 128, 1, 64, 15, 0};
 
@@ -1620,6 +1903,10 @@ const char* kernel_name(int id, bool elu) {
     case 19: return elu ? "gemm_x6d_kernel<192,128,6,2,2,true>" : "gemm_x6d_kernel<192,128,6,2,2,false>";
     case 20: return "gemm_x6d_kernel<128,128,4,2,2,false,2>";
     case 22: return "gemm_x6d_kernel<192,128,6,2,2,false,2>";
+    case 24: return elu ? "gemm_h3_kernel<128,128,2,2,1,4,true>" : "gemm_h3_kernel<128,128,2,2,1,4,false>";
+    case 25: return elu ? "gemm_h3_kernel<128,128,4,2,2,4,true>" : "gemm_h3_kernel<128,128,4,2,2,4,false>";
+    case 26: return elu ? "gemm_h3_kernel<64,128,2,2,2,3,true>" : "gemm_h3_kernel<64,128,2,2,2,3,false>";
+    case 27: return elu ? "gemm_h3_kernel<64,64,2,2,4,2,true>" : "gemm_h3_kernel<64,64,2,2,4,2,false>";
     case 7: return "gemm_mid_kernel<64,64,1>";
     case 8: return "gemm_mid_kernel<32,32,4>";
     default: return "gemm_generic_kernel";
@@ -1629,6 +1916,44 @@ const char* kernel_name(int id, bool elu) {
 void record_plan(int id, bool elu, long tiles, int splits) {
   snprintf(g_last_plan, sizeof g_last_plan, "%s tiles=%ld splits=%d%s", kernel_name(id, elu), tiles,
            splits, splits > 1 ? " +split-K reduce" : "");
+}
+
+// The h3 tile and K split of a contraction of M rows, N columns and depth K
+// (C_in channels per tap).  Above 512 128x128 tiles (more than two per CU) the
+// four-blocks-per-CU tile; below, fewer and deeper blocks, split along K once
+// they leave CUs idle.  Measured on the decoder's shapes (us, best bf16x6 or
+// FP32 tile -> h3): 7500-15000 tiles, K = 256-512: 778 -> 567, 604 -> 432;
+// 1500-3000, K = 1024: 457 -> 318; 470 tiles, K = 512: 45 -> 35; 4000-row
+// qkv 38 -> 32, fc1 47 -> 35, fc2 53 -> 43, o 25 -> 22; 6240 x 256 x 256:
+// 13.8 -> 10.6; 1248 x 640 x 512: 30 -> 13; 26 x 4096 x 2048: 19 -> 15;
+// 16 x 1536 x 1024: 15.7 -> 10.
+void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tiles, int& splits) {
+  const long t128 = tile_count(M, p.N, kH3);
+  const bool k32 = p.C_in % 32 == 0 && p.K % 32 == 0, k64 = p.C_in % 64 == 0 && p.K % 64 == 0;
+  // Smallest power-of-two split that reaches 320 blocks, >= min_k deep.
+  auto fewest = [&](long t, int most, int min_k) {
+    int sp = 1;
+    while (workspace && sp < most && t * sp < 320 && p.K / (2 * sp) >= min_k) sp *= 2;
+    return sp;
+  };
+  splits = 1;
+  if (!k32 || t128 > 512) {
+    cfg = kH3;
+  } else if (p.K >= 1024 ? t128 >= 64 : t128 >= 192) {
+    // Long K: 64 tiles x 8 splits 30 us against 77 us unsplit (250 rows of
+    // the stride-8 upsampling), 192 x 2 40 against 43, 256 x 2 109 against
+    // 129, 128 x 4 (fc2 at 4000 rows) 43 against 78.
+    cfg = kH3K32;
+    if (p.K >= 1024) splits = fewest(t128, 8, 256);
+  } else if (!k64 || (p.K < 1024 && M >= 2048 && p.N >= 512)) {
+    // The 512-column projections at 2500-4000 rows (20.6-21.6 us; 128x128
+    // tiles 21.3-22.2).
+    cfg = kH3Small;
+  } else {
+    cfg = kH3Tiny;
+    if (p.K >= 512) splits = fewest(tile_count(M, p.N, kH3Tiny), 16, 128);
+  }
+  tiles = tile_count(M, p.N, cfg);
 }
 
 int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s) {
@@ -1654,7 +1979,14 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
   const bool big_ok = p.N % 4 == 0 && !(p.bias && p.bias_len % 4);
   const TileCfg big = p.N >= 128 ? kBigSquare : kBigTile;
   const long big_tiles = tile_count(M, p.N, big);
-  if (!fast) {
+  // fp16 planes: the h3 tiles take every such contraction they can address
+  // (weight planes and a tile's rows behind 32-bit buffer offsets) with
+  // columns enough to fill a fragment.
+  const bool h3 = (p.flags & FM_WEIGHTS_H3) && !(p.flags & FM_REPLICATE) && p.C_in % 16 == 0 && p.K % 16 == 0 &&
+                  p.N >= 32 && 4L * p.K * p.N <= 0x7fffffffL && 257L * p.N * 4 <= 0x7fffffffL;
+  if (h3) {
+    pick_h3(M, p, workspace != nullptr, cfg, tiles, splits);
+  } else if (!fast) {
     cfg = TileCfg{64, 64, 1, 16, -1, 0};
     tiles = tile_count(M, p.N, cfg);
   } else if (p.K >= 1024 && big_tiles < 384 && M >= 1024 && big_ok && workspace) {
@@ -1729,7 +2061,7 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
   // The direct-load tiles need every k-tile (32 deep) inside one tap.
   const bool dl_ok = big_ok && !(p.flags & (FM_REPLICATE | FM_ELU_IN)) && p.C_in % 32 == 0 &&
                      p.K % 32 == 0;
-  if (dl_ok) {
+  if (dl_ok && !h3) {
     if (cfg.id == 9) cfg = kDl128;
     if (cfg.id == 10) cfg = kDl192;
     if (cfg.id == 11 && p.C_in % 64 == 0 && p.K % 64 == 0) cfg = kDl64;
@@ -1747,7 +2079,7 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
   const bool x6_ok = (p.flags & FM_WEIGHTS_X6) && big_ok && !(p.flags & FM_REPLICATE) &&
                      p.C_in % 16 == 0 && p.K % 16 == 0 && 6L * p.K * p.N <= 0x7fffffffL &&
                      257L * p.N * 4 <= 0x7fffffffL;
-  if (x6_ok && cfg.id >= 9 && cfg.id <= 15 && cfg.id != 12) {
+  if (x6_ok && !h3 && cfg.id >= 9 && cfg.id <= 15 && cfg.id != 12) {
     const long t128 = tile_count(M, p.N, kX6);
     if (p.K >= 1024 && M >= 1024 && t128 < 360 && workspace) {
       // Long K over a few hundred tiles (the 2048-deep fc2 projection at
@@ -1815,7 +2147,7 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
     if (cfg.id == kX6.id) cfg = kX6K32;
     else if (cfg.id == kX6Wide.id) cfg = kX6WideK32;
   }
-  const bool rope_after = (p.flags & FM_EPI_ROPE) && (!(cfg.id >= 16 && cfg.id <= 22) || splits != 1);
+  const bool rope_after = (p.flags & FM_EPI_ROPE) && (!(cfg.id >= 16 && cfg.id <= 26) || splits != 1);
   if (rope_after) p.flags &= ~FM_EPI_ROPE;
   if (splits > 1) {
     const size_t per = (size_t)M * p.N * sizeof(float);
@@ -1830,6 +2162,8 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
   p.partial = splits > 1 ? workspace : nullptr;
 
   dim3 grid((unsigned)tiles, splits);
+  // The fp16 planes follow the FP32 weight and its bf16 planes.
+  const _Float16* wh = reinterpret_cast<const _Float16*>(p.w + (long)p.N * p.K + 3L * p.N * p.K / 2);
   record_plan(cfg.id, (p.flags & FM_ELU_IN) != 0, tiles, splits);
   // Zero-page loader of the large tiles (their k-tile is 32).
   const bool zp = !(p.flags & FM_REPLICATE) && p.C_in % 32 == 0;
@@ -1891,6 +2225,21 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
       hipLaunchKernelGGL((gemm_x6d_kernel<192, 128, 6, 2, 2, false, 2>), grid, dim3(768), 0, s, p,
                          reinterpret_cast<const __bf16*>(p.w + (long)p.N * p.K));
       break;
+#define FM_H3(BM_, BN_, WM_, WN_, KS_, WPE_, ROPE_)                                                          \
+  if (p.flags & FM_ELU_IN)                                                                                   \
+    hipLaunchKernelGGL((gemm_h3_kernel<BM_, BN_, WM_, WN_, KS_, WPE_, true>), grid, dim3(64 * WM_ * WN_), 0, \
+                       s, p, wh);                                                                            \
+  else if (ROPE_ && (p.flags & FM_EPI_ROPE))                                                                 \
+    hipLaunchKernelGGL((gemm_h3_kernel<BM_, BN_, WM_, WN_, KS_, WPE_, false, ROPE_>), grid,                  \
+                       dim3(64 * WM_ * WN_), 0, s, p, wh);                                                   \
+  else                                                                                                       \
+    hipLaunchKernelGGL((gemm_h3_kernel<BM_, BN_, WM_, WN_, KS_, WPE_, false>), grid, dim3(64 * WM_ * WN_),   \
+                       0, s, p, wh)
+    case 24: FM_H3(128, 128, 2, 2, 1, 4, true); break;
+    case 25: FM_H3(128, 128, 4, 2, 2, 4, true); break;
+    case 26: FM_H3(64, 128, 2, 2, 2, 3, true); break;
+    case 27: FM_H3(64, 64, 2, 2, 4, 2, false); break;
+#undef FM_H3
     case 7: hipLaunchKernelGGL((gemm_mid_kernel<64, 64, 1>), grid, dim3(NTHREADS), 0, s, p); break;
     case 8: hipLaunchKernelGGL((gemm_mid_kernel<32, 32, 4>), grid, dim3(NTHREADS), 0, s, p); break;
     default: hipLaunchKernelGGL(gemm_generic_kernel, grid, dim3(256), 0, s, p); break;
@@ -1933,7 +2282,7 @@ int fm_conv1d(const float* x, int batch, int length, int in_channels, const floa
   p.y_rows = y_length; p.bias_len = out_channels;
   p.flags = (flags & ~FM_REPLICATE) | (pad_mode == 1 ? FM_REPLICATE : 0);
   if (p.flags & FM_EPI_RES_SCALE) return FM_BAD_ARGUMENT;
-  const int plain = p.flags & ~(FM_EPI_ELU | FM_ELU_IN | FM_WEIGHTS_X6);
+  const int plain = p.flags & ~(FM_EPI_ELU | FM_ELU_IN | FM_WEIGHTS_X6 | FM_WEIGHTS_H3);
   if (x && weight_packed && y && batch > 0 && length > 0 && stride == 1 && plain == 0 &&
       y_length >= 0 && y_length <= length) {
     // The packed layout W^T[c_out][(tap, c_in)] doubles as [C][k] / [k*C] here.
@@ -1990,6 +2339,15 @@ int fm_split_weights(const float* weight_packed, int rows, int cols, void* plane
   return (int)hipGetLastError();
 }
 
+// The fp16 planes and row exponents of a packed weight (see gemm_h3_kernel).
+int fm_split_weights_h3(const float* weight_packed, int rows, int cols, void* planes, hipStream_t stream) {
+  if (!weight_packed || !planes || rows <= 0 || cols <= 0) return FM_BAD_ARGUMENT;
+  if (cols % 16) return FM_UNSUPPORTED;
+  hipLaunchKernelGGL(split_weights_h3_kernel, dim3(rows), dim3(256), 0, stream, weight_packed, rows, cols,
+                     reinterpret_cast<_Float16*>(planes));
+  return (int)hipGetLastError();
+}
+
 int fm_conv_transpose1d(const float* x, int batch, int length, int in_channels,
                         const float* weight_packed, const float* bias, int out_channels, int kernel,
                         int stride, int flags, const float* residual, float* y, float* workspace,
@@ -2023,12 +2381,13 @@ int fm_linear_rope(const float* x, int rows, int in_features, const float* weigh
   if (!cos_table || !sin_table || rope_cols <= 0 || rope_cols % 64 || rope_cols > out_features ||
       out_features % 64 || rows_per_seq <= 0)
     return FM_BAD_ARGUMENT;
-  if (flags != FM_WEIGHTS_X6) return FM_UNSUPPORTED;  // bf16x6 tiles only, no other epilogue
+  // 16-bit tiles only, no other epilogue.
+  if ((flags & ~FM_WEIGHTS_H3) != FM_WEIGHTS_X6) return FM_UNSUPPORTED;
   GemmArgs p{};
   p.x = x; p.w = weight_packed; p.bias = nullptr; p.res = nullptr; p.scale = nullptr; p.y = y;
   p.batch = 1; p.L_in = rows; p.C_in = in_features; p.rows = rows; p.rs = 1; p.padL = 0;
   p.K = in_features; p.N = out_features; p.y_rows = rows; p.bias_len = 0;
-  p.flags = FM_WEIGHTS_X6 | FM_EPI_ROPE;
+  p.flags = flags | FM_EPI_ROPE;
   p.rope_cos = cos_table; p.rope_sin = sin_table; p.rope_cols = rope_cols; p.rows_per_seq = rows_per_seq;
   return run_gemm(p, workspace, workspace_bytes, stream);
 }

@@ -823,7 +823,7 @@ int fm_resblock(const float* x, int batch, int length, int channels, const float
   if (!fm_resblock_supported(channels)) return FM_UNSUPPORTED;
   if (x == y) return FM_BAD_ARGUMENT;  // the halo rows of other blocks must stay intact
   if (batch == 0 || length == 0) return FM_OK;
-  const int elu = (elu_out & ~(FM_WEIGHTS_X6 | FM_ACT_EXP)) != 0;
+  const int elu = (elu_out & ~(FM_WEIGHTS_X6 | FM_WEIGHTS_H3 | FM_ACT_EXP)) != 0;
   const bool x6 = elu_out & FM_WEIGHTS_X6, fa = elu_out & FM_ACT_EXP;
   if (x6) {
     // Split planes follow each packed weight (fm_split_weights).
@@ -866,7 +866,7 @@ int fm_conv_resblock64(const float* wav, int batch, int length, const float* w0_
       length < 0)
     return FM_BAD_ARGUMENT;
   if (batch == 0 || length == 0) return FM_OK;
-  const int elu = (elu_out & ~(FM_WEIGHTS_X6 | FM_ACT_EXP)) != 0;
+  const int elu = (elu_out & ~(FM_WEIGHTS_X6 | FM_WEIGHTS_H3 | FM_ACT_EXP)) != 0;
   if (elu_out & FM_WEIGHTS_X6) {
     if (elu_out & FM_ACT_EXP)
       hipLaunchKernelGGL((resblock_x6_kernel<64, 128, 4, 2, true, false, true>), dim3((length + 127) / 128, batch),
@@ -902,7 +902,7 @@ int fm_resblock64_conv(const float* x, int batch, int length, const float* w1_pa
   if (batch == 0 || y_len == 0) return FM_OK;
   if (!workspace || workspace_bytes < fm_resblock64_conv_workspace_bytes(batch, length))
     return FM_WORKSPACE_TOO_SMALL;
-  const int elu = (elu_mid & ~(FM_WEIGHTS_X6 | FM_ACT_EXP)) != 0;
+  const int elu = (elu_mid & ~(FM_WEIGHTS_X6 | FM_WEIGHTS_H3 | FM_ACT_EXP)) != 0;
   if (elu_mid & FM_WEIGHTS_X6) {
     if (elu_mid & FM_ACT_EXP)
       hipLaunchKernelGGL((resblock_x6_kernel<64, 128, 4, 2, false, true, true>), dim3((length + 127) / 128, batch),

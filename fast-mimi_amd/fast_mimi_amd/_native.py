@@ -27,6 +27,7 @@ EPI_RES_ADD = 16
 EPI_RES_SCALE = 32
 WEIGHTS_X6 = 64
 ACT_EXP = 128  # residual blocks: ELU as e^x - 1 (decoder-side calls)
+WEIGHTS_H3 = 512  # fp16 planes after the bf16 ones (decoder-side layers)
 
 _STATUS = {1000: "bad argument", 1001: "workspace too small", 1002: "unsupported shape",
            1003: "input larger than the fixed scratch of an allocation-free entry point"}
@@ -50,6 +51,7 @@ _SIGNATURES = {
     "fm_abi_version": ([], _I),
     "fm_gemm_last_plan": ([ctypes.c_char_p, _I], _I),
     "fm_split_weights": ([_P, _I, _I, _P, _P], _I),
+    "fm_split_weights_h3": ([_P, _I, _I, _P, _P], _I),
     "fm_conv1d": ([_P, _I, _I, _I, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P, _S, _P], _I),
     "fm_conv1d_rows_supported": ([_I, _I, _I, _I], _I),
     "fm_conv1d_rows": ([_P, _I, _I, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P], _I),

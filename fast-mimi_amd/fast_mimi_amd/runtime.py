@@ -24,6 +24,7 @@ Fusion plan (one kernel per line):
 
 from __future__ import annotations
 
+import copy
 import threading
 
 import torch
@@ -208,12 +209,20 @@ class MimiRuntime:
         # Convolution and large-row projection weights carry their bf16x6
         # planes: W^T followed by [3][N][K] bf16 in one buffer.
         self._x6: dict[int, torch.Tensor] = {}
-        for layer in self._conv_layers():
-            w = self._with_planes(layer.w)
+        # The decoder side, whose waveform is continuous, also carries the fp16
+        # planes of the three-product form; the encoder side must not (its
+        # codes sit at near-ties that another rounding would tip).
+        for name, layer in self._named_conv_layers():
+            h3 = name.startswith("dec.")
+            w = self._with_planes(layer.w, h3)
             if w is not layer.w:
-                layer.w, layer.flags = w, nat.WEIGHTS_X6
-        for w in [m for lay in self.enc_tf + self.dec_tf for m in (lay.wqkv, lay.wo, lay.w1, lay.w2)]:
-            self._x6[w.data_ptr()] = self._with_planes(w)
+                layer.w, layer.flags = w, nat.WEIGHTS_X6 | (nat.WEIGHTS_H3 if h3 else 0)
+        self._h3: set[int] = set()  # device addresses of the row-major weights that carry fp16 planes
+        for layers, h3 in ((self.enc_tf, False), (self.dec_tf, True)):
+            for w in [m for lay in layers for m in (lay.wqkv, lay.wo, lay.w1, lay.w2)]:
+                wx = self._x6[w.data_ptr()] = self._with_planes(w, h3)
+                if h3 and wx is not w:
+                    self._h3.add(w.data_ptr())
         # Which layers took planes, checked against the declared plan (a layer
         # without planes would silently run its FP32 kernels instead).
         self.x6_layers = {name: bool(layer.flags & nat.WEIGHTS_X6) for name, layer in self._named_conv_layers()}
@@ -261,17 +270,21 @@ class MimiRuntime:
     def _conv_layers(self):
         return [layer for _, layer in self._named_conv_layers()]
 
-    def _with_planes(self, w: torch.Tensor) -> torch.Tensor:
+    def _with_planes(self, w: torch.Tensor, h3: bool = False) -> torch.Tensor:
         """``w`` [N, K] (FP32 W^T) as the first N*K floats of a buffer that
-        continues with its three bf16 planes (``fm_split_weights``); ``w``
-        itself when K is not a multiple of 16."""
+        continues with its three bf16 planes (``fm_split_weights``) and, with
+        ``h3``, its fp16 planes (``fm_split_weights_h3``); ``w`` itself when K
+        is not a multiple of 16."""
         rows, cols = w.shape
         if cols % 16:
             return w
         n = w.numel()
-        buf = torch.empty(n + 3 * n // 2, device=self.device)
+        x6 = n + 3 * n // 2
+        buf = torch.empty(x6 + (n + rows if h3 else 0), device=self.device)
         buf[:n].copy_(w.reshape(-1))
-        ops.call("fm_split_weights", buf[:n], rows, cols, buf[n:])
+        ops.call("fm_split_weights", buf[:n], rows, cols, buf[n:x6])
+        if h3:
+            ops.call("fm_split_weights_h3", buf[:n], rows, cols, buf[x6:])
         return buf[:n].view(w.shape)
 
     # ------------------------------------------------------------------ ops
@@ -304,7 +317,7 @@ class MimiRuntime:
                 and not flags & ~(nat.ELU_IN | nat.EPI_ELU | nat.EPI_RES_ADD)):
             self._call("fm_conv1d_rows", x, B, L, layer.c_in, layer.wr, layer.b, layer.c_out,
                        layer.c_out, layer.k, layer.stride, layer.replicate,
-                       flags | (layer.flags if layer.wr is layer.w else 0), residual, y)
+                       flags | (layer.flags & nat.WEIGHTS_X6 if layer.wr is layer.w else 0), residual, y)
             return y, rows
         self._call("fm_conv1d", x, B, L, layer.c_in, layer.w, layer.b,
                  layer.c_out, layer.k, layer.stride, layer.replicate, flags | layer.flags, residual,
@@ -323,7 +336,8 @@ class MimiRuntime:
         y = torch.empty((rows, n), device=self.device) if out is None else out
         wx = self._x6.get(w.data_ptr())
         if wx is not None:
-            w, flags = wx, flags | nat.WEIGHTS_X6
+            flags |= nat.WEIGHTS_X6 | (nat.WEIGHTS_H3 if w.data_ptr() in self._h3 else 0)
+            w = wx
         self._call("fm_linear", x, rows, k, w, n, flags, residual,
                  scale, y, self.workspace, _WORKSPACE_BYTES)
         return y
@@ -333,7 +347,8 @@ class MimiRuntime:
         attention then reads rotated q / k)."""
         n, k = w.shape
         y = torch.empty((rows, n), device=self.device)
-        self._call("fm_linear_rope", x, rows, k, self._x6[w.data_ptr()], n, nat.WEIGHTS_X6, cos, sin,
+        flags = nat.WEIGHTS_X6 | (nat.WEIGHTS_H3 if w.data_ptr() in self._h3 else 0)
+        self._call("fm_linear_rope", x, rows, k, self._x6[w.data_ptr()], n, flags, cos, sin,
                    rope_cols, per_seq, y, self.workspace, _WORKSPACE_BYTES)
         return y
 
@@ -388,7 +403,7 @@ class MimiRuntime:
         if fused:
             self._tag = tag
             y = torch.empty_like(x)
-            flags = (1 if elu_after else 0) | (c1.flags & c2.flags & nat.WEIGHTS_X6)
+            flags = (1 if elu_after else 0) | (c1.flags & c2.flags)
             if act_exp and flags & nat.WEIGHTS_X6:
                 flags |= nat.ACT_EXP
             self._call("fm_resblock", x, B, L, c2.c_out, c1.w, c1.b, c2.w, c2.b, flags, y)
@@ -514,7 +529,7 @@ class MimiRuntime:
             h = torch.empty((B, S, 64), device=self.device)
             self._call("fm_conv_resblock64", x, B, S, first.w,
                        first.b, c1.w, c1.b, c2.w,
-                       c2.b, 1 | (c1.flags & c2.flags & nat.WEIGHTS_X6), h)
+                       c2.b, 1 | (c1.flags & c2.flags), h)
             L, start = S, 1
         else:
             self._tag = "enc.first"
@@ -694,7 +709,7 @@ class MimiRuntime:
                 y = torch.empty((B, out_length), device=self.device)
                 last = self.dec_last
                 self._call("fm_resblock64_conv", h, B, L, c1.w, c1.b,
-                           c2.w, c2.b, 1 | nat.ACT_EXP | (c1.flags & c2.flags & nat.WEIGHTS_X6), last.w, last.b,
+                           c2.w, c2.b, 1 | nat.ACT_EXP | (c1.flags & c2.flags), last.w, last.b,
                            out_length, y, d, d.numel() * 4)
                 return y.view(B, 1, out_length)
             h = self._resblock(h, B, L, block, elu_after=True, tag=f"dec.res{convt.c_out}", act_exp=True)
@@ -708,10 +723,13 @@ class MimiRuntime:
         return y.transpose(1, 2).contiguous()
 
     # ------------------------------------------------------- measurement
-    def layer_op(self, name: str, batch: int, samples: int):
+    def layer_op(self, name: str, batch: int, samples: int, planes: int = nat.WEIGHTS_X6):
         """A closure running one SEANet contraction at its real shape for a
         ``batch x samples`` round trip (names as in ``flops.layer_table``), on
-        fixed random inputs.  Used to time a single kernel."""
+        fixed random inputs.  Used to time a single kernel.  ``planes`` are the
+        16-bit weight planes the launch may use of those the layer carries:
+        the bf16 ones every layer has, or with ``WEIGHTS_X6 | WEIGHTS_H3`` what
+        the round trip itself launches."""
         cfg = self.config
         specs = {}
         L = samples
@@ -737,6 +755,8 @@ class MimiRuntime:
             specs[f"dec.res{ch}.c2"] = (c2, L, nat.EPI_RES_ADD | nat.EPI_ELU, True)
         specs["dec.last"] = (self.dec_last, L, 0, False)
         layer, length, flags, needs_res = specs[name]
+        layer = copy.copy(layer)
+        layer.flags &= planes
         g = torch.Generator(device=self.device).manual_seed(0)
         x = torch.randn((batch, length, layer.c_in), device=self.device, generator=g)
         if isinstance(layer, _ConvT):

@@ -46,7 +46,8 @@ enum {
   FM_EPI_RES_ADD = 16,  /* y = residual + (acc + bias)                         */
   FM_EPI_RES_SCALE = 32, /* y = residual + scale[n] * acc   (fm_linear only)    */
   FM_WEIGHTS_X6 = 64,    /* weight is followed by its bf16 planes (fm_split_weights) */
-  FM_ACT_EXP = 128       /* residual blocks: ELU as e^x - 1 (see fm_resblock)     */
+  FM_ACT_EXP = 128,      /* residual blocks: ELU as e^x - 1 (see fm_resblock)     */
+  FM_WEIGHTS_H3 = 512    /* the bf16 planes are followed by the fp16 ones (fm_split_weights_h3) */
 };
 
 /* ABI version of the library (bumped when a contract changes). */
@@ -76,6 +77,23 @@ int fm_gemm_last_plan(char* buf, int size);
  * entry points below replace.
  */
 int fm_split_weights(const float* weight_packed, int rows, int cols, void* planes, hipStream_t stream);
+
+/*
+ * fp16 weights ("h3"): each row n of W^T [rows][cols] (cols a multiple of 16,
+ * else FM_UNSUPPORTED), scaled by a power of two 2^s_n that brings its largest
+ * magnitude into [2^13, 2^14), as two round-to-nearest fp16 pieces in the
+ * k16-tile order [2][cols/16][rows][16], followed by int s_n [rows]: rows *
+ * cols * 4 + rows * 4 bytes at `planes`.  A caller that stores them directly
+ * after the fm_split_weights planes and adds FM_WEIGHTS_H3 (512) to `flags`
+ * lets fm_conv1d / fm_conv1d_valid / fm_conv_transpose1d / fm_linear /
+ * fm_linear_rope run the FP32 contraction as three fp16 MFMA products per
+ * operand pair, activations split on the fly with a power-of-two scale per
+ * row.  The error against float64 is that of FP32 sums (below the bf16x6
+ * form's); results differ from it in the last bits, so callers whose codes
+ * depend on exact sums keep FM_WEIGHTS_X6 alone.
+ * No reference counterpart (as fm_split_weights).
+ */
+int fm_split_weights_h3(const float* weight_packed, int rows, int cols, void* planes, hipStream_t stream);
 
 /*
  * Causal Conv1d, dilation 1: left zero (pad_mode 0) or edge (pad_mode 1)

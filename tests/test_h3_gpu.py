@@ -1,0 +1,201 @@
+"""The three-product fp16 form (FM_WEIGHTS_H3) against float64.
+
+Tolerance: a product drops a1 b1 (at most 2^-22 |a b|) and each operand is
+within 2^-23 of its value, so a sum of K products is within
+(2^-22 + 2 * 2^-23) sum |a b| of the exact one plus the FP32 rounding of its
+accumulation, which the FP32 and bf16x6 kernels are held to as 1e-5 sum |a b|;
+the same 1e-5 holds here.  Row scales make that a per-row property, whatever
+the magnitudes of the other rows.
+"""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from fast_mimi_amd import _native as nat
+from fast_mimi_amd.config import MimiConfig
+from fast_mimi_amd.runtime import _Conv, _ConvT, rope_tables
+from oracle.mimi_oracle import causal_conv1d, causal_conv_transpose1d
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+WS_BYTES = 64 << 20
+FLAGS = nat.WEIGHTS_X6 | nat.WEIGHTS_H3
+
+
+@pytest.fixture(scope="module")
+def ws():
+    return torch.empty(WS_BYTES // 4, device=DEV)
+
+
+def stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+def with_planes(w):
+    """W^T [N, K], then its bf16 planes, then its fp16 planes and row exponents."""
+    rows, cols = w.shape
+    n = w.numel()
+    x6 = n + 3 * n // 2
+    buf = torch.empty(x6 + n + rows, device=DEV)
+    buf[:n].copy_(w.reshape(-1))
+    nat.call("fm_split_weights", buf.data_ptr(), rows, cols, buf.data_ptr() + 4 * n, stream())
+    nat.call("fm_split_weights_h3", buf.data_ptr(), rows, cols, buf.data_ptr() + 4 * x6, stream())
+    torch.cuda.synchronize()
+    return buf[:n].view(w.shape), buf[x6:]
+
+
+def linear(x, w, ws, flags=FLAGS, res=None, scale=None):
+    rows, k = x.shape
+    n = w.shape[0]
+    y = torch.full((rows, n), float("nan"), device=DEV)
+    nat.call("fm_linear", x.data_ptr(), rows, k, w.data_ptr(), n, flags, None if res is None else res.data_ptr(),
+             None if scale is None else scale.data_ptr(), y.data_ptr(), ws.data_ptr(), WS_BYTES, stream())
+    torch.cuda.synchronize()
+    return y
+
+
+def close_dot(got, want, absref, rel=1e-5):
+    worst = ((got.double() - want).abs() / (rel * absref + 1e-300)).max().item()
+    assert worst <= 1.0, f"error {worst:.2f}x the per-element bound"
+
+
+def test_split_weights_h3_layout():
+    """Two fp16 pieces per weight, within 2^-22 of it, each row scaled so its
+    largest magnitude lies in [2^13, 2^14); zero and tiny rows included."""
+    g = torch.Generator().manual_seed(1)
+    w = torch.randn(48, 80, generator=g) * torch.logspace(-30, 30, 48)[:, None]
+    w[5] = 0
+    _, planes = with_planes(w.to(DEV))
+    n = w.numel()
+    half = planes[:n].view(torch.float16).view(2, 5, 48, 16).permute(0, 2, 1, 3).reshape(2, 48, 80).cpu().double()
+    s = planes[n:].view(torch.int32).cpu().double()
+    top = half[0].abs().amax(1)
+    assert torch.all((top >= 2 ** 13) & (top <= 2 ** 14) | (w.abs().amax(1) == 0))
+    back = half.sum(0) * torch.exp2(-s)[:, None]
+    assert torch.all((back - w.double()).abs() <= w.double().abs() * 2.0 ** -22 + w.abs().amax(1, keepdim=True) * 2.0 ** -38)
+    with pytest.raises(nat.NativeError, match="unsupported"):
+        nat.call("fm_split_weights_h3", planes.data_ptr(), 4, 24, planes.data_ptr(), stream())
+    with pytest.raises(nat.NativeError, match="bad argument"):
+        nat.call("fm_split_weights_h3", planes.data_ptr(), 0, 16, planes.data_ptr(), stream())
+
+
+@pytest.mark.parametrize("rows,k,n,plan", [
+    (1, 2048, 512, "<64,64,2,2,4,2"), (63, 64, 32, "<64,64,2,2,4,2"), (65, 1024, 1536, "<64,64,2,2,4,2"),
+    (250, 2048, 4096, "<128,128,4,2,2,4"), (2500, 512, 512, "<64,128,2,2,2,3"), (2500, 96, 100, "<64,128,2,2,2,3"),
+    (2500, 512, 1536, "<128,128,4,2,2,4"), (4000, 2048, 512, "<128,128,4,2,2,4"),
+    (127, 48, 36, "<128,128,2,2,1,4"), (66000, 256, 128, "<128,128,2,2,1,4"), (16001, 512, 640, "<128,128,2,2,1,4"),
+])
+def test_linear_tiles(rows, k, n, plan, ws):
+    """Each tile and K split, ragged rows and columns, against float64; no
+    further from it (2-norm) than the FP32 / bf16x6 plan of the same call."""
+    g = torch.Generator().manual_seed(rows + k + n)
+    x = torch.randn(rows, k, generator=g).to(DEV)
+    w, _ = with_planes((torch.randn(n, k, generator=g) / math.sqrt(k)).to(DEV))
+    want = x.double() @ w.double().t()
+    got = linear(x, w, ws)
+    assert f"gemm_h3_kernel{plan}" in nat.last_gemm_plan(), nat.last_gemm_plan()
+    close_dot(got, want, x.double().abs() @ w.double().abs().t())
+    other = linear(x, w, ws, nat.WEIGHTS_X6)
+    err, was = ((v.double() - want).norm() / want.norm() for v in (got, other))
+    assert err <= max(1.1 * was, 1.5e-7), f"{err:.2e} against {was:.2e}"
+    res, scale = torch.randn(rows, n, generator=g).to(DEV), torch.randn(n, generator=g).to(DEV)
+    close_dot(linear(x, w, ws, FLAGS | nat.EPI_RES_SCALE, res, scale), res.double() + scale.double() * want,
+              res.double().abs() + scale.double().abs() * (x.double().abs() @ w.double().abs().t()))
+
+
+@pytest.mark.parametrize("rows,k,n", [(200, 512, 256), (2500, 512, 1536), (2500, 512, 512), (70000, 128, 128)])
+def test_row_scales(rows, k, n, ws):
+    """Rows from 1e-30 to 1e30 side by side, rows that start with zeros, rows
+    that grow by 2^60 along k and rows of zeros all keep their own relative
+    accuracy; a row holding an inf or a NaN spoils only itself."""
+    g = torch.Generator().manual_seed(rows + n)
+    x = torch.randn(rows, k, generator=g)
+    x *= 10.0 ** (60 * torch.rand(rows, 1, generator=g) - 30)
+    x[3::7, :k // 2] = 0
+    x[4::7] *= torch.exp2(torch.linspace(-40, 20, k))
+    x[5::7] *= torch.exp2(torch.linspace(20, -40, k))
+    x[6::7] = 0
+    x[0, 5], x[64, k - 1], x[130, 0] = float("inf"), float("nan"), float("-inf")
+    x = x.to(DEV)
+    w, _ = with_planes((torch.randn(n, k, generator=g) / math.sqrt(k)).to(DEV))
+    got = linear(x, w, ws)
+    assert "gemm_h3_kernel" in nat.last_gemm_plan()
+    bad = torch.zeros(rows, dtype=torch.bool, device=DEV)
+    bad[[0, 64, 130]] = True
+    assert not torch.isfinite(got[bad]).any()
+    x, got = x[~bad], got[~bad]
+    close_dot(got, x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t())
+    assert torch.all(got[(x == 0).all(1)] == 0)
+
+
+@pytest.mark.parametrize("B,cin,cout,stride,L", [(1, 1024, 512, 8, 26), (1, 128, 64, 4, 6240), (3, 256, 128, 5, 1001),
+                                                 (2, 128, 64, 4, 40001), (1, 48, 16, 4, 777)])
+def test_conv_transpose1d(B, cin, cout, stride, L, ws):
+    """Stride phases, batch seams inside a tile and the zero row before each clip."""
+    g = torch.Generator().manual_seed(L)
+    x = torch.randn(B, cin, L, generator=g)
+    w, b = torch.randn(cin, cout, 2 * stride, generator=g) / math.sqrt(2 * cin), torch.randn(cout, generator=g)
+    layer = _ConvT(w.to(DEV), b.to(DEV), stride)
+    wp, _ = with_planes(layer.w)
+    xd = x.transpose(1, 2).contiguous().to(DEV)
+    y = torch.full((B, L * stride, cout), float("nan"), device=DEV)
+    nat.call("fm_conv_transpose1d", xd.data_ptr(), B, L, cin, wp.data_ptr(), layer.b.data_ptr(), cout, layer.k,
+             stride, FLAGS, None, y.data_ptr(), ws.data_ptr(), WS_BYTES, stream())
+    torch.cuda.synchronize()
+    assert "gemm_h3_kernel" in nat.last_gemm_plan()
+    want = causal_conv_transpose1d(x.double(), w.double(), b.double(), stride)
+    absref = causal_conv_transpose1d(x.double().abs(), w.double().abs(), b.double().abs(), stride)
+    close_dot(y.cpu().transpose(1, 2), want, absref)
+
+
+@pytest.mark.parametrize("B,cin,cout,k,L,y_len,flags", [
+    (1, 512, 256, 3, 208, None, nat.ELU_IN | nat.EPI_ELU), (16, 512, 256, 3, 2000, None, nat.ELU_IN | nat.EPI_ELU),
+    (3, 256, 512, 1, 700, None, nat.EPI_RES_ADD | nat.EPI_ELU), (2, 512, 1024, 7, 61, 50, nat.EPI_ELU),
+    (4, 64, 128, 3, 20001, 19000, 0)])
+def test_conv1d(B, cin, cout, k, L, y_len, flags, ws):
+    """ELU on load, residual and ELU epilogues, cropped outputs."""
+    g = torch.Generator().manual_seed(L + cin)
+    x = torch.randn(B, cin, L, generator=g)
+    w, b = torch.randn(cout, cin, k, generator=g) / math.sqrt(cin * k), torch.randn(cout, generator=g)
+    res = torch.randn(B, cout, L, generator=g)
+    y_len = L if y_len is None else y_len
+    layer = _Conv(w.to(DEV), b.to(DEV))
+    wp, _ = with_planes(layer.w)
+    xd, rd = (t.transpose(1, 2).contiguous().to(DEV) for t in (x, res))
+    y = torch.full((B, y_len, cout), float("nan"), device=DEV)
+    nat.call("fm_conv1d", xd.data_ptr(), B, L, cin, wp.data_ptr(), layer.b.data_ptr(), cout, k, 1, 0, flags | FLAGS,
+             rd.data_ptr(), y.data_ptr(), y_len, ws.data_ptr(), WS_BYTES, stream())
+    torch.cuda.synchronize()
+    assert "gemm_h3_kernel" in nat.last_gemm_plan()
+    xin = F.elu(x.double()) if flags & nat.ELU_IN else x.double()
+    want = causal_conv1d(xin, w.double(), b.double())
+    absref = causal_conv1d(xin.abs(), w.double().abs(), b.double().abs())
+    if flags & nat.EPI_RES_ADD:
+        want, absref = want + res, absref + res.abs()
+    if flags & nat.EPI_ELU:
+        want = F.elu(want)
+    close_dot(y.cpu().transpose(1, 2), want[..., :y_len], absref[..., :y_len])
+
+
+@pytest.mark.parametrize("rows,per_seq,n,rope_cols", [(2500, 2500, 1536, 1024), (30000, 250, 1536, 1024),
+                                                      (2500, 100, 512, 512), (100, 100, 1536, 1024)])
+def test_linear_rope_equals_linear_then_rope(rows, per_seq, n, rope_cols, ws):
+    """RoPE in the tile's epilogue, or after it where the tile cannot, equals
+    fm_linear followed by fm_apply_rope bit for bit."""
+    g = torch.Generator().manual_seed(rows + n)
+    x = torch.randn(rows, 512, generator=g).to(DEV)
+    w, _ = with_planes((torch.randn(n, 512, generator=g) / math.sqrt(512)).to(DEV))
+    cos, sin = (t.to(DEV) for t in rope_tables(MimiConfig(), per_seq))
+    want = linear(x, w, ws)
+    nat.call("fm_apply_rope", want.data_ptr(), rows, n, rope_cols, 64, cos.data_ptr(), sin.data_ptr(), per_seq,
+             stream())
+    got = torch.full((rows, n), float("nan"), device=DEV)
+    nat.call("fm_linear_rope", x.data_ptr(), rows, 512, w.data_ptr(), n, FLAGS, cos.data_ptr(), sin.data_ptr(),
+             rope_cols, per_seq, got.data_ptr(), ws.data_ptr(), WS_BYTES, stream())
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)

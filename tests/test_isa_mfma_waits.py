@@ -13,7 +13,7 @@ N + 1, any other instruction 1, branches followed both ways); each such read
 must come at least passes + 1 wait states after the MFMA.  (The compiler's
 own straight-line waits are passes + 2; the bad read had 1.)  Passes per
 instruction on gfx950, from the MFMA busy cycles the counters report (4 per
-pass): 32x32x2 f32 16, 32x32x16 bf16 8, 16x16x4 f32 8, 16x16x32 bf16 4.
+pass): 32x32x2 f32 16, 32x32x16 bf16 / f16 8, 16x16x4 f32 8, 16x16x32 bf16 / f16 4.
 """
 
 from __future__ import annotations
@@ -36,7 +36,8 @@ HIPCC = build_native.HIPCC
 CSRC = REPO / "fast-mimi_amd" / "csrc"
 OUT = REPO / "fast-mimi_amd" / "_build" / "isa"
 PASSES = {"v_mfma_f32_32x32x2_f32": 16, "v_mfma_f32_32x32x16_bf16": 8,
-          "v_mfma_f32_16x16x4_f32": 8, "v_mfma_f32_16x16x32_bf16": 4}
+          "v_mfma_f32_16x16x4_f32": 8, "v_mfma_f32_16x16x32_bf16": 4,
+          "v_mfma_f32_32x32x16_f16": 8, "v_mfma_f32_16x16x32_f16": 4}
 MARGIN = 1
 _REG = re.compile(r"\b([va])\[(\d+):(\d+)\]|\b([va])(\d+)\b")
 _STORES = ("ds_write", "buffer_store", "global_store", "flat_store", "scratch_store", "global_atomic",
