@@ -895,6 +895,392 @@ __global__ __launch_bounds__(256) void rvq_decode_kernel(const int64_t* codes, i
   out[m * 2 * dim + dim + k] = ac;
 }
 
+// ---------------------------------------------------------------------------
+// Whole split encode of many rows in one launch, exact codes from a screened
+// search.  A block owns 32 rows for the whole residual chain (no exchange
+// between blocks, no launch per codebook).  Per codebook step:
+//   screen: approximate distances of the rows to every entry from one fp16
+//     MFMA product per 16 dims (entries and rows scaled by powers of two),
+//     eight waves striding over 32-entry tiles whose fragments stream from L2
+//     one tile ahead, across steps too; each lane keeps the three smallest
+//     of the 128 distances it sees;
+//   candidates: the entries within `margin` of the row's smallest screened
+//     distance.  margin bounds twice the largest difference between a
+//     screened distance and the FP32 one the codes are defined by (fp16
+//     rounding of both operands by Cauchy-Schwarz, FP32 accumulation, the
+//     7-bit entry tag in the key, the rounding before the square root), so
+//     the FP32 argmin and everything that ties with it is among them;
+//   exact: a row with one candidate is done (about 85% of rows); otherwise
+//     the candidates' FP32 distances are evaluated and compared as
+//     rvq_step_mfma_kernel<256, 1> does, operation for operation: the
+//     32x32x2 FP32 MFMA rounds like fma(a1, b1, fma(a0, b0, c)), so one lane's
+//     FMA chain in its dim order gives the same bits.
+// A row that cannot be screened (non-finite values or margin, or a lane whose
+// third smallest distance is a candidate too) sends the block through the
+// FP32 MFMA scan of every entry for that step.  The codes are therefore
+// those of the step kernel bit for bit.
+// Bound by the fp16 codebook stream, 1 MB per step and CU through the L1 port
+// (about two thirds of a step; the rest is the chain residual -> screen ->
+// candidates -> exact): 8000 rows x 32 codebooks 3.17 ms in step launches ->
+// 0.71 ms, 2000 rows x 8 0.27 -> 0.14 ms.
+constexpr int SCREEN_WAVES = 8;
+constexpr int SCREEN_ENTRIES = 2048;     // 8 waves x 8 tiles x 32 entries: 7-bit tags
+constexpr int SCREEN_PAIRS = 512;        // exact candidates per block and step
+
+// Per codebook: the power of two its fp16 copy is scaled by, and a bound on
+// its entries' norms (inf when an entry is not finite).
+struct ScreenInfo {
+  int exp;
+  float top;
+};
+
+struct ScreenArgs {
+  const float* x;  // [M][ld_x]: semantic input in columns [0, 256), acoustic in [256, 512)
+  int ld_x, M, rows_per_batch, entries, batch_stride;
+  int n_semantic, count;    // codebooks: the semantic branch's, then the acoustic one's
+  const float* embeds;      // [count][entries][256]
+  const float* norms;       // [count][entries]
+  const _Float16* planes;   // [count][16][entries][16]
+  const ScreenInfo* info;   // [count]
+  int64_t* codes;           // codebook 0; codebook c at + c * rows_per_batch
+};
+
+__global__ __launch_bounds__(256) void rvq_screen_prepare_kernel(const float* __restrict__ embed,
+                                                                 const float* __restrict__ norms, int entries,
+                                                                 _Float16* __restrict__ planes,
+                                                                 ScreenInfo* __restrict__ info) {
+  // One block per codebook: largest magnitude and norm, then the scaled copy.
+  const long cb = blockIdx.x;
+  embed += cb * entries * 256;
+  planes += cb * entries * 256;
+  norms += cb * entries;
+  float m = 0.0f, nm = 0.0f;
+  bool bad = false;
+  for (long i = threadIdx.x; i < (long)entries * 256; i += 256) {
+    const float v = fabsf(embed[i]);
+    bad |= !(v < INFINITY);
+    m = fmaxf(m, v);
+  }
+  for (int i = threadIdx.x; i < entries; i += 256) {
+    bad |= !(norms[i] < INFINITY);
+    nm = fmaxf(nm, norms[i]);
+  }
+  __shared__ float red[2][256];
+  red[0][threadIdx.x] = m;
+  red[1][threadIdx.x] = nm;
+  bad = __syncthreads_or(bad);
+  for (int d = 128; d > 0; d >>= 1) {
+    if (threadIdx.x < d)
+      for (int q = 0; q < 2; ++q) red[q][threadIdx.x] = fmaxf(red[q][threadIdx.x], red[q][threadIdx.x + d]);
+    __syncthreads();
+  }
+  m = red[0][0];
+  // m in [2^9, 2^10) after scaling.
+  const int s = m > 0.0f && !bad ? min(max(263 - (int)(__builtin_bit_cast(unsigned, m) >> 23), 1), 253) - 127 : 0;
+  const float sc = __builtin_bit_cast(float, (unsigned)(s + 127) << 23);
+  if (threadIdx.x == 0) info[cb] = ScreenInfo{s, bad ? INFINITY : sqrtf(red[1][0]) * 1.0001f};
+  for (long i = threadIdx.x; i < (long)entries * 256; i += 256) {
+    const long n = i / 256;
+    const int k = (int)(i % 256);
+    planes[((long)(k >> 4) * entries + n) * 16 + (k & 15)] = (_Float16)(embed[i] * sc);
+  }
+}
+
+__global__ __launch_bounds__(64 * SCREEN_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void rvq_screen_kernel(ScreenArgs a) {
+  constexpr int DIM = 256, PX = DIM + 4, CH = DIM / 32, KF = DIM / 16;
+  __shared__ __attribute__((aligned(16))) float Xs[RB * PX];       // residual rows, FP32
+  __shared__ __attribute__((aligned(16))) char Xh[RB * DIM * 2];   // their fp16 fragments [k16][half][row][8]
+  __shared__ __attribute__((aligned(16))) float normS[SCREEN_ENTRIES];
+  __shared__ float low[3][2 * SCREEN_WAVES][RB + 1];  // each lane list's smallest three keys per row
+  __shared__ float xnS[RB], coefS[RB], marginS[RB];
+  __shared__ int codeS[RB];
+  __shared__ unsigned long long exactS[RB];  // (ordered distance, entry) minimum over a row's candidates
+  __shared__ int pairS[SCREEN_PAIRS];        // row << 16 | entry
+  __shared__ int npairS, fullS;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, col = lane & 31;
+  const long m0 = (long)blockIdx.x * RB;
+  const int tiles = a.entries / 32;
+  const int mine = (tiles - wave + SCREEN_WAVES - 1) / SCREEN_WAVES;  // tiles wave, wave + 8, ...
+
+  // Fragments of one 32-entry tile: lane (entry col, k half h), 16 k16 steps.
+  halfx8 cur[KF];
+  const long cb = (long)a.entries * DIM;
+  const __amdgpu_buffer_rsrc_t rp = fm_buffer(a.planes, (int)(a.count * cb * 2));
+  const int voff = 32 * col + 16 * h;
+  auto frag = [&](int c, int tile, int k) {
+    return __builtin_bit_cast(halfx8, fm_buf_load4(rp, voff, ((c * KF + k) * a.entries + 32 * tile) * 32));
+  };
+  if (wave < tiles) {
+#pragma unroll
+    for (int k = 0; k < KF; ++k) cur[k] = frag(0, wave, k);
+  }
+
+  // Waves 4-7 form the residual rows, eight lanes per row as the step kernel's
+  // prologue; waves 0-3 decide ambiguous rows meanwhile.
+  const bool former = wave >= SCREEN_WAVES / 2;
+  // The final code of codebook c for row r: its only candidate, or the best of
+  // the exact stage; written out by one lane.
+  auto decide = [&](int c, int r, bool write) {
+    int code = codeS[r];
+    if (code < 0) code = code_index((int)(unsigned)exactS[r], a.entries);
+    if (write && m0 + r < a.M) {
+      const int m = (int)m0 + r, b = m / a.rows_per_batch;
+      a.codes[(long)b * a.batch_stride + (long)c * a.rows_per_batch + (m - b * a.rows_per_batch)] = code;
+    }
+    return code;
+  };
+  floatx4 ev[CH];     // the chosen entry's dims, fetched early when `have`
+  bool have = false;
+  auto forget = [&]() {  // (assigned, so that nothing stays live across the screen)
+    have = false;
+#pragma unroll
+    for (int u = 0; u < CH; ++u) ev[u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  forget();
+  floatx4 nv = {0.0f, 0.0f, 0.0f, 0.0f};  // this thread's four norms of the step's codebook
+  if (tid < a.entries / 4) nv = *reinterpret_cast<const floatx4*>(a.norms + 4 * tid);
+  ScreenInfo info = a.info[0];
+
+  for (int c = 0; c < a.count; ++c) {
+    const bool first = c == 0 || c == a.n_semantic;  // of its branch: fresh rows
+    const float* embed = a.embeds + c * cb;
+    const int next = min(c + 1, a.count - 1);
+    // The phases' addresses are formed where they are used: hoisted out of
+    // the loop they would spill, and a reload ahead of the screen's loop puts
+    // a full wait on its prefetches into every iteration.
+    int lt = tid;
+    asm volatile("" : "+v"(lt));
+    const int wr = (lt - 256) >> 3, pt = lt & 7;  // row and lane part (waves 4-7)
+    // ---- residual rows.
+    if (former) {
+      const long m = m0 + wr;
+      int code = 0;
+      if (c > 0) code = decide(c - 1, wr, pt == 0);
+      floatx4 xv[CH];
+      if (first) {
+        const float* src = a.x + min(m, (long)a.M - 1) * a.ld_x + (c >= a.n_semantic ? DIM : 0);
+#pragma unroll
+        for (int u = 0; u < CH; ++u) xv[u] = *reinterpret_cast<const floatx4*>(src + 4 * (pt + 8 * u));
+      } else {
+        if (!have) {
+          const float* er = embed - cb + (long)code * DIM;
+#pragma unroll
+          for (int u = 0; u < CH; ++u) ev[u] = *reinterpret_cast<const floatx4*>(er + 4 * (pt + 8 * u));
+        }
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+          xv[u] = *reinterpret_cast<const floatx4*>(Xs + wr * PX + 4 * (pt + 8 * u));
+#pragma unroll
+          for (int q = 0; q < 4; ++q) xv[u][q] = __fsub_rn(xv[u][q], ev[u][q]);
+        }
+      }
+      float xn = 0.0f, top = 0.0f;
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        if (m >= a.M) xv[u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          xn = fmaf(xv[u][q], xv[u][q], xn);
+          top = fmaxf(top, fabsf(xv[u][q]));
+        }
+        *reinterpret_cast<floatx4*>(Xs + wr * PX + 4 * (pt + 8 * u)) = xv[u];
+      }
+#pragma unroll
+      for (int o = 1; o < 8; o <<= 1) {
+        xn += __shfl_xor(xn, o, 64);
+        top = fmaxf(top, __shfl_xor(top, o, 64));
+      }
+      const int s = top > 0.0f ? min(max(263 - (int)(__builtin_bit_cast(unsigned, top) >> 23), 1), 253) - 127 : 0;
+      const float sc = __builtin_bit_cast(float, (unsigned)(s + 127) << 23);
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int k = 4 * (pt + 8 * u);
+        halfx4 v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = (_Float16)(xv[u][q] * sc);
+        *reinterpret_cast<halfx4*>(Xh + (k >> 4) * 1024 + ((k >> 3) & 1) * 512 + wr * 16 + (k & 7) * 2) = v;
+      }
+      if (pt == 0) {
+        xnS[wr] = xn;
+        coefS[wr] = -2.0f * ldexpf(1.0f, -(s + info.exp));
+        // Twice the bound on |screened - FP32| (see above), X = |x|, T = top norm.
+        const float X = sqrtf(xn) * 1.0001f, T = info.top;
+        marginS[wr] =
+            2.0f * (X * T * (0x1p-9f + 0x1p-11f) + T * T * 0x1p-15f + (xn + T * T) * 0x1p-19f) + 0x1p-96f;
+        exactS[wr] = ~0ull;
+      }
+    }
+    if (tid < a.entries / 4) *reinterpret_cast<floatx4*>(normS + 4 * tid) = nv;
+    if (tid == 0) npairS = 0, fullS = 0;
+    lds_barrier();
+
+    // ---- screen.
+    halfx8 q[KF];
+#pragma unroll
+    for (int k = 0; k < KF; ++k) q[k] = *reinterpret_cast<const halfx8*>(Xh + k * 1024 + h * 512 + col * 16);
+    const float coef = coefS[col];
+    float l1 = INFINITY, l2 = INFINITY, l3 = INFINITY;
+    for (int t = 0; t < mine; ++t) {
+      const int tile = wave + SCREEN_WAVES * t;
+      // The next tile of this wave: of the next codebook after the last.
+      const int nc = t + 1 < mine ? c : next;
+      const int nt = t + 1 < mine ? tile + SCREEN_WAVES : wave;
+      floatx16 acc;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+      for (int k = 0; k < KF; ++k) {
+        acc = fm_mfma32_f16(cur[k], q[k], acc);
+        cur[k] = frag(nc, nt, k);
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const floatx4 en = *reinterpret_cast<const floatx4*>(normS + 32 * tile + 8 * g + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float d = fmaf(acc[4 * g + e], coef, en[e]);
+          // The key's low 7 bits name the entry within this lane.
+          const float key = __builtin_bit_cast(
+              float, (__builtin_bit_cast(unsigned, d) & ~127u) | (unsigned)(16 * t + 4 * g + e));
+          l3 = __builtin_amdgcn_fmed3f(l2, l3, key);
+          l2 = __builtin_amdgcn_fmed3f(l1, l2, key);
+          l1 = fminf(l1, key);
+        }
+      }
+    }
+    low[0][2 * wave + h][col] = l1;
+    low[1][2 * wave + h][col] = l2;
+    low[2][2 * wave + h][col] = l3;
+    // The next step's norms and scale.
+    if (tid < a.entries / 4) nv = *reinterpret_cast<const floatx4*>(a.norms + (long)next * a.entries + 4 * tid);
+    info = a.info[next];
+    lds_barrier();
+
+    // ---- candidates: sixteen lanes per row, one per list.
+    asm volatile("" : "+v"(lt));
+    {
+      const int r = lt >> 4, s = lt & 15;
+      const float k1 = low[0][s][r], k2 = low[1][s][r], k3 = low[2][s][r];
+      float best = k1;
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) best = fminf(best, __shfl_xor(best, o, 64));
+      const float lim = best + marginS[r];
+      const bool finite = fabsf(lim) < INFINITY;  // false for a NaN too
+      const bool c1 = k1 <= lim, c2 = k2 <= lim;
+      const unsigned long long m1 = __ballot(c1) >> (lane & 48) & 0xffff, m2 = __ballot(c2) >> (lane & 48) & 0xffff;
+      const int n = __popcll(m1) + __popcll(m2);
+      auto entry_of = [&](float key) {
+        const int tag = (int)(__builtin_bit_cast(unsigned, key) & 127u);
+        return 32 * ((s >> 1) + SCREEN_WAVES * (tag >> 4)) + 8 * ((tag & 15) >> 2) + 4 * (s & 1) + (tag & 3);
+      };
+      if (m0 + r < a.M && (!finite || k3 <= lim)) fullS = 1;
+      if (finite && n == 1) {
+        if (c1) codeS[r] = entry_of(k1);
+      } else if (finite && m0 + r < a.M) {
+        if (c1) {
+          const int p = atomicAdd(&npairS, 1);
+          if (p < SCREEN_PAIRS) pairS[p] = r << 16 | entry_of(k1);
+          else fullS = 1;
+        }
+        if (c2) {
+          const int p = atomicAdd(&npairS, 1);
+          if (p < SCREEN_PAIRS) pairS[p] = r << 16 | entry_of(k2);
+          else fullS = 1;
+        }
+        if (s == 0) codeS[r] = -1;
+      } else if (s == 0) {
+        codeS[r] = 0;
+      }
+    }
+    lds_barrier();
+    asm volatile("" : "+v"(lt));
+    // An FP32 distance as an ordered key: dist_key's -inf below every
+    // non-negative distance; equal distances go to the lowest entry.
+    auto order = [&](float acc, int r, int entry) {
+      const float d = dist_key(__fadd_rn(__fadd_rn(__fmul_rn(-2.0f, acc), xnS[r]), normS[entry]));
+      const unsigned u = d >= 0.0f ? (__builtin_bit_cast(unsigned, d) & 0x7fffffffu) + 1u : 0u;
+      return (unsigned long long)u << 32 | (unsigned)entry;
+    };
+    if (fullS) {
+      // ---- every entry in FP32 (rvq_step_mfma_kernel<256, 1>'s main loop).
+      const int fl = lt & 63, fh = fl >> 5, fc = fl & 31;
+      for (int t = 0; t < mine; ++t) {
+        const int tile = wave + SCREEN_WAVES * t;
+        floatx16 acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+        for (int pc = 0; pc < DIM / 64; ++pc) {
+          const float* src = embed + (long)(32 * tile + fc) * DIM + 64 * pc + 32 * fh;
+          const float* xr = Xs + fc * PX + 64 * pc + 32 * fh;
+#pragma unroll 2
+          for (int u = 0; u < 8; ++u) {
+            const floatx4 e4 = *reinterpret_cast<const floatx4*>(src + 4 * u);
+            const floatx4 x4 = *reinterpret_cast<const floatx4*>(xr + 4 * u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = fm_mfma32(e4[e], x4[e], acc);
+          }
+        }
+        unsigned long long best = ~0ull;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const unsigned long long o = order(acc[r], fc, 32 * tile + fm_mfma32_row(r, fl));
+          best = o < best ? o : best;
+        }
+        atomicMin(&exactS[fc], best);
+      }
+      if (tid < RB) codeS[tid] = -1;
+      forget();
+    } else {
+      if (former) {
+        // Most rows are decided: fetch their entries while the others wait.
+        const int code = codeS[(lt - 256) >> 3];
+        have = code >= 0;
+        const float* er = embed + (long)max(code, 0) * DIM + 4 * (lt & 7);
+#pragma unroll
+        for (int u = 0; u < CH; ++u) ev[u] = *reinterpret_cast<const floatx4*>(er + 32 * u);
+      } else {
+        // Eight lanes per candidate, 32 dims each in the step kernel's order
+        // (dims k, k + 32 of a 64-dim piece by turns): the FMA chain passes
+        // from lane to lane.
+        forget();
+        const int n = npairS;
+        for (int i0 = 0; i0 < n; i0 += 32) {
+          const int i = i0 + (lt >> 3);
+          const int pr = i < n ? pairS[i] : 0;
+          const int r = pr >> 16, entry = pr & 0xffff;
+          const int part = lt & 7, k0 = 64 * (part >> 1) + 16 * (part & 1);
+          floatx4 e0[4], e1[4], x0[4], x1[4];
+          const float* er = embed + (long)entry * DIM + k0;
+          const float* xr = Xs + r * PX + k0;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            e0[u] = *reinterpret_cast<const floatx4*>(er + 4 * u);
+            e1[u] = *reinterpret_cast<const floatx4*>(er + 32 + 4 * u);
+            x0[u] = *reinterpret_cast<const floatx4*>(xr + 4 * u);
+            x1[u] = *reinterpret_cast<const floatx4*>(xr + 32 + 4 * u);
+          }
+          float acc = 0.0f;
+          for (int step = 0; step < 8; ++step) {
+            float v = acc;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v = fmaf(e1[u][e], x1[u][e], fmaf(e0[u][e], x0[u][e], v));
+            // Lane `step` of the eight holds the chain's true value.
+            acc = __shfl(v, (lt & 56) + step, 64);
+          }
+          if (part == 0 && i < n) atomicMin(&exactS[r], order(acc, r, entry));
+        }
+      }
+    }
+    lds_barrier();
+  }
+  if (former) decide(a.count - 1, (tid - 256) >> 3, (tid & 7) == 0);
+}
+
 size_t step_lds_bytes(int dim) {
   return (size_t)dim * (RB + 1) * 4 + (size_t)KSL * PB * 4 + RB * 4 + 4 * RB * 4 + 4 * RB * 4 +
          RB * 4;
@@ -1212,6 +1598,45 @@ int fm_rvq_decode(const int64_t* codes, int batch, int num_codebooks, int frames
   hipLaunchKernelGGL(rvq_decode_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
                      stream, codes, num_codebooks, num_semantic, frames, M, embeds, entries, dim,
                      out);
+  return (int)hipGetLastError();
+}
+
+}  // extern "C"
+
+// ---------------------------------------------------------------------------
+// Screened split encode (rvq_screen_kernel).
+extern "C" {
+
+int fm_rvq_prepare_screen(const float* embeds, const float* norms, int entries, int dim, int count,
+                          void* planes, void* info, hipStream_t stream) {
+  if (!embeds || !norms || !planes || !info || entries <= 0 || count <= 0) return FM_BAD_ARGUMENT;
+  if (dim != 256) return FM_UNSUPPORTED;
+  hipLaunchKernelGGL(rvq_screen_prepare_kernel, dim3(count), dim3(256), 0, stream, embeds, norms, entries,
+                     static_cast<_Float16*>(planes), static_cast<ScreenInfo*>(info));
+  return (int)hipGetLastError();
+}
+
+// Above 1024 rows, where the step launches sum a dot product as one chain (as
+// the exact stage does) and take 34 us a step at 2000 rows, 100 us at 8000;
+// below, they split the codebook over more CUs than there are 32-row blocks.
+int fm_rvq_screen_supported(int rows, int dim, int entries) {
+  return rows > 1024 && dim == 256 && entries > 0 && entries % 32 == 0 && entries <= SCREEN_ENTRIES;
+}
+
+int fm_rvq_encode_split_screened(const float* x, int ld_x, int rows, int rows_per_batch, int dim, int entries,
+                                 int n_semantic, int n_acoustic, const float* embeds, const float* norms,
+                                 const void* planes, const void* info, int64_t* codes, int batch_stride,
+                                 hipStream_t stream) {
+  const long count = (long)n_semantic + n_acoustic;
+  if (!rvq_args_ok(x, ld_x, rows, rows_per_batch, dim, entries, embeds, embeds, norms, codes) || !planes ||
+      !info || n_semantic < 0 || n_acoustic < 0 || count <= 0 || ld_x < 2 * dim)
+    return FM_BAD_ARGUMENT;
+  // (The fp16 codebooks are addressed through one buffer resource.)
+  if (!fm_rvq_screen_supported(rows, dim, entries) || count * entries * dim * 2 > INT_MAX) return FM_UNSUPPORTED;
+  const ScreenArgs a{x, ld_x, rows, rows_per_batch, entries, batch_stride, n_semantic, (int)count, embeds, norms,
+                     static_cast<const _Float16*>(planes), static_cast<const ScreenInfo*>(info), codes};
+  hipLaunchKernelGGL(rvq_screen_kernel, dim3((unsigned)((rows + RB - 1) / RB)), dim3(64 * SCREEN_WAVES), 0, stream,
+                     a);
   return (int)hipGetLastError();
 }
 

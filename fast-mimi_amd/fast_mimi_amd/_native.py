@@ -73,6 +73,9 @@ _SIGNATURES = {
     "fm_rvq_encode": ([_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _S, _P], _I),
     "fm_rvq_split_workspace_bytes": ([_I, _I, _I], _S),
     "fm_rvq_encode_split": ([_P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _S, _P], _I),
+    "fm_rvq_prepare_screen": ([_P, _P, _I, _I, _I, _P, _P, _P], _I),
+    "fm_rvq_screen_supported": ([_I, _I, _I], _I),
+    "fm_rvq_encode_split_screened": ([_P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P], _I),
     "fm_rvq_noalloc_scratch_bytes": ([], _S),
     "fm_rvq_encode_split_noalloc": ([_P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P], _I),
     "fm_rvq_decode": ([_P, _I, _I, _I, _I, _P, _I, _I, _P, _P], _I),

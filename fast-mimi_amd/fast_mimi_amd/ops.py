@@ -47,6 +47,8 @@ SPECS = {
     "fm_rvq_prepare_codebook": "in:embed_sum in:cluster_usage i:entries i:dim f:eps out:embed out:embed_t out:norms",
     "fm_rvq_encode": "in:x i:ld_x i:rows i:rows_per_batch i:dim i:entries i:count in:embeds in:embeds_t in:norms out:codes i:batch_stride out:workspace i:workspace_bytes",
     "fm_rvq_encode_split": "in:x i:ld_x i:rows i:rows_per_batch i:dim i:entries i:n_semantic i:n_acoustic in:embeds in:embeds_t in:norms out:codes i:batch_stride out:workspace i:workspace_bytes",
+    "fm_rvq_prepare_screen": "in:embeds in:norms i:entries i:dim i:count out:planes out:info",
+    "fm_rvq_encode_split_screened": "in:x i:ld_x i:rows i:rows_per_batch i:dim i:entries i:n_semantic i:n_acoustic in:embeds in:norms in:planes in:info out:codes i:batch_stride",
     "fm_rvq_encode_split_noalloc": "in:x i:ld_x i:rows i:rows_per_batch i:dim i:entries i:n_semantic i:n_acoustic in:embeds in:embeds_t in:norms out:codes i:batch_stride",
     "fm_rvq_decode": "in:codes i:batch i:num_codebooks i:frames i:num_semantic in:embeds i:entries i:dim out:out",
     "fm_upsample_depthwise": "in:x i:batch i:length i:channels in:weight i:kernel i:stride out:y",

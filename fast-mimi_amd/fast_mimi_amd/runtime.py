@@ -195,6 +195,13 @@ class MimiRuntime:
                      st[f"{p}.cluster_usage"].contiguous(), e, d, 1e-5,
                      self.embeds[j], self.embeds_t[j],
                      self.norms[j])
+        # Scaled fp16 copies for the screened search of many rows.
+        self.screen = self.screen_info = None
+        if d == 256:
+            self.screen = torch.empty((len(prefixes), e * d), dtype=torch.float16, device=device)
+            self.screen_info = torch.empty((len(prefixes), 2), dtype=torch.int32, device=device)
+            ops.call("fm_rvq_prepare_screen", self.embeds, self.norms, e, d, len(prefixes), self.screen,
+                     self.screen_info)
         # Fragment-packed copies of the projection weights for the few-row kernels,
         # keyed by the row-major weight's device address.
         self._packed: dict[int, torch.Tensor] = {}
@@ -648,8 +655,14 @@ class MimiRuntime:
         proj = self.quantizer_inputs(h, B, T)
         self._tag = "rvq.encode"
         codes = torch.empty((B, nq, T), dtype=torch.int64, device=self.device)
-        ws_bytes = nat.library().fm_rvq_split_workspace_bytes(M, vq, cfg.codebook_size)
         n_sem = min(cfg.num_semantic_quantizers, nq)
+        lib = nat.library()
+        if self.screen is not None and lib.fm_rvq_screen_supported(M, vq, cfg.codebook_size):
+            self._call("fm_rvq_encode_split_screened", proj, 2 * vq, M, T, vq, cfg.codebook_size,
+                       n_sem, nq - n_sem, self.embeds, self.norms, self.screen, self.screen_info, codes,
+                       nq * T)
+            return codes
+        ws_bytes = lib.fm_rvq_split_workspace_bytes(M, vq, cfg.codebook_size)
         # Both chains in shared launches (step s of each branch in one grid).
         ws = torch.empty((ws_bytes + 3) // 4, device=self.device)
         self._call("fm_rvq_encode_split", proj, 2 * vq, M, T, vq, cfg.codebook_size,

@@ -418,6 +418,25 @@ int fm_rvq_encode_split_noalloc(const float* x, int ld_x, int rows, int rows_per
                                 int batch_stride, hipStream_t stream);
 
 /*
+ * fm_rvq_encode_split as a screened search for many rows: approximate fp16
+ * distances pick the entries that can be nearest, and their FP32 distances
+ * decide, so the codes are fm_rvq_encode_split's bit for bit.  Supported where
+ * fm_rvq_screen_supported(rows, dim, entries) != 0 (above 1024 rows, 256-dim
+ * codebooks of at most 2048 entries, a multiple of 32), else FM_UNSUPPORTED.
+ * planes / info come from fm_rvq_prepare_screen over the same `count` =
+ * n_semantic + n_acoustic codebooks: [count][16][entries][16] fp16 (count *
+ * entries * 512 bytes, at most 2 GiB) and 8 bytes per codebook.
+ * Replaces MimiSplitResidualVectorQuantizer.encode (model.py:2485-2501).
+ */
+int fm_rvq_screen_supported(int rows, int dim, int entries);
+int fm_rvq_prepare_screen(const float* embeds, const float* norms, int entries, int dim, int count,
+                          void* planes, void* info, hipStream_t stream);
+int fm_rvq_encode_split_screened(const float* x, int ld_x, int rows, int rows_per_batch, int dim,
+                                 int entries, int n_semantic, int n_acoustic, const float* embeds,
+                                 const float* norms, const void* planes, const void* info,
+                                 int64_t* codes, int batch_stride, hipStream_t stream);
+
+/*
  * Split-RVQ decode gather-sum: out[(b*frames + t)][0:dim] = 0 + E_0[c_0]
  * (the num_semantic first codebooks summed left to right),
  * out[...][dim:2*dim] = 0 + E_s[c_s] + E_{s+1}[c_{s+1}] + ... left to right.
