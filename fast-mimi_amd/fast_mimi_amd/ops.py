@@ -52,6 +52,8 @@ SPECS = {
     "fm_rvq_encode_split_noalloc": "in:x i:ld_x i:rows i:rows_per_batch i:dim i:entries i:n_semantic i:n_acoustic in:embeds in:embeds_t in:norms out:codes i:batch_stride",
     "fm_rvq_decode": "in:codes i:batch i:num_codebooks i:frames i:num_semantic in:embeds i:entries i:dim out:out",
     "fm_upsample_depthwise": "in:x i:batch i:length i:channels in:weight i:kernel i:stride out:y",
+    "fm_stream_append": "in:context in:x i:batch i:pad i:length i:channels i:replicate out:buf out:next",
+    "fm_kv_append": "in:qkv i:q_cols i:kv_cols i:batch i:length in:keys in:values i:cached i:keep out:comb out:next_keys out:next_values",
     "fm_copy_buffers": "in:src0 out:dst0 i:bytes0 in:src1 out:dst1 i:bytes1",
 }
 

@@ -33,6 +33,7 @@ from . import _native as nat
 from . import ops
 from .config import MimiConfig
 from .flops import layer_table
+from .streaming import MimiConv1dPaddingCache, MimiKVCache
 from .weights import decoder_layer_indices, encoder_layer_indices
 
 _WORKSPACE_BYTES = 64 << 20
@@ -115,6 +116,11 @@ def x6_plan(config: MimiConfig) -> dict[str, bool]:
         if kind in ("conv", "convt") or (kind == "gemm" and name.rsplit(".", 1)[-1] in _PROJECTIONS):
             plan[name] = k % 16 == 0
     return plan
+
+
+def _plain(t: torch.Tensor, like: torch.Tensor, shape: tuple) -> bool:
+    """A contiguous float32 tensor of ``shape`` on ``like``'s device."""
+    return t.shape == shape and t.dtype == torch.float32 and t.device == like.device and t.is_contiguous()
 
 
 def rope_tables(config: MimiConfig, length: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -567,9 +573,8 @@ class MimiRuntime:
     def _stream_conv(self, x, layer: _Conv, cache, idx: int, flags: int = 0, residual=None):
         """One cached causal conv: the layer runs on (context ++ chunk) with no
         padding; the cache keeps the newest ``k - stride`` input rows."""
-        B, L, _ = x.shape
-        ctx = cache.update(x, idx)
-        buf = torch.cat((ctx, x), dim=1) if ctx.shape[1] else x
+        B, L, C = x.shape
+        buf = self._stream_input(x, cache, idx)
         total = buf.shape[1]
         if total < layer.k:
             raise RuntimeError(f"streaming chunk too short: {total} rows for a kernel of {layer.k}")
@@ -579,6 +584,51 @@ class MimiRuntime:
                    layer.b, layer.c_out, layer.k, layer.stride, flags | layer.flags, residual,
                    y, self.workspace, _WORKSPACE_BYTES)
         return y, rows
+
+    def _stream_input(self, x, cache, idx: int):
+        """``x`` behind the layer's cached left context, the cache advanced:
+        ``cache.update`` and the concatenation in one launch where the cache
+        holds what that launch can read, else as two steps."""
+        B, L, C = x.shape
+        pad = cache.per_layer_padding[idx]
+        ctx = cache.padding_cache[idx]
+        if type(cache) is MimiConv1dPaddingCache and pad > 0 and L > 0 and (ctx is None or _plain(ctx, x, (B, pad, C))):
+            x = x.contiguous()
+            buf = torch.empty((B, pad + L, C), device=self.device)
+            new = torch.empty((B, pad, C), device=self.device)
+            self._call("fm_stream_append", ctx, x, B, pad, L, C,
+                       1 if cache.per_layer_padding_mode[idx] == "replicate" else 0, buf, new)
+            cache.padding_cache[idx] = new
+            return buf
+        ctx = cache.update(x, idx)
+        return torch.cat((ctx, x), dim=1) if ctx.shape[1] else x
+
+    def _attention_rows(self, q3, kv, li: int, qd: int, kd: int):
+        """(operand, cached rows) of layer ``li``'s attention over the chunk
+        ``q3`` [B, T, qd + 2 kd] and what ``kv`` retains, the cache advanced."""
+        B, T, ld = q3.shape
+        key = kv.key_cache[li] if li < len(kv.key_cache) else None
+        value = kv.value_cache[li] if key is not None else None
+        n = 0 if key is None else key.shape[1]
+        if (type(kv) is MimiKVCache and T > 0 and kv.sliding_window is not None and
+                (key is None or (_plain(key, q3, (B, n, kd)) and _plain(value, q3, (B, n, kd))))):
+            kv._ensure_layer(li)
+            keep = min(n + T, kv.sliding_window - 1)
+            comb = torch.empty((B, n + T, ld), device=self.device)
+            new_k = torch.empty((B, keep, kd), device=self.device)
+            new_v = torch.empty((B, keep, kd), device=self.device)
+            self._call("fm_kv_append", q3, qd, kd, B, T, key if n else None, value if n else None, n, keep, comb,
+                       new_k if keep else None, new_v if keep else None)
+            kv._cumulative_lengths[li] += T
+            kv.key_cache[li], kv.value_cache[li] = new_k, new_v
+            return comb, n
+        keys, values = kv.update(q3[:, :, qd:qd + kd], q3[:, :, qd + kd:], li)
+        n = keys.shape[1] - T
+        comb = torch.empty((B, n + T, ld), device=self.device)
+        comb[:, :, qd:qd + kd] = keys
+        comb[:, :, qd + kd:] = values
+        comb[:, n:, :qd] = q3[:, :, :qd]
+        return comb, n
 
     def _encoder_seanet_stream(self, x, B, cache):
         i = 0
@@ -627,13 +677,7 @@ class MimiRuntime:
                 self._call("fm_apply_rope", qkv, M, qkv.shape[1], qd + kd, hd,
                            cos, sin, T)
             ld = qkv.shape[1]
-            q3 = qkv.view(B, T, ld)
-            keys, values = kv.update(q3[:, :, qd:qd + kd], q3[:, :, qd + kd:], li)
-            n = keys.shape[1] - T
-            comb = torch.empty((B, n + T, ld), device=self.device)
-            comb[:, :, qd:qd + kd] = keys
-            comb[:, :, qd + kd:] = values
-            comb[:, n:, :qd] = q3[:, :, :qd]
+            comb, n = self._attention_rows(qkv.view(B, T, ld), kv, li, qd, kd)
             self._call("fm_window_attention_rows", comb, ld, 0, qd, qd + kd, None, None,
                        B, n + T, n, nh, nkv, hd, cfg.sliding_window, 1.0 / (hd ** 0.5),
                        att, qd)

@@ -459,6 +459,31 @@ int fm_upsample_depthwise(const float* x, int batch, int length, int channels,
                           hipStream_t stream);
 
 /*
+ * Streaming convolution input: buf [batch][pad + length][channels] = context
+ * [batch][pad][channels] followed by x [batch][length][channels], and next =
+ * buf's last pad rows (the layer's next context; context != next).  context
+ * NULL starts a stream: zeros, or with replicate the first row of x.
+ * Replaces MimiConv1dPaddingCache.update and the concatenation in
+ * MimiConv1d.forward (model.py:536-620, :764-797).
+ */
+int fm_stream_append(const float* context, const float* x, int batch, int pad, int length, int channels,
+                     int replicate, float* buf, float* next, hipStream_t stream);
+
+/*
+ * Streaming attention operand: comb [batch][cached + length][q_cols + 2 *
+ * kv_cols] whose key / value columns are the cached rows keys / values
+ * [batch][cached][kv_cols] followed by the chunk's rows of qkv
+ * [batch][length][q_cols + 2 * kv_cols], whose query columns are written for
+ * the chunk's rows only; next_keys / next_values [batch][keep][kv_cols] are the
+ * last keep of those key / value rows (other memory than keys / values).
+ * Replaces MimiKVCache.update (model.py:363-518) and the operand assembly of
+ * the cached attention (model.py:1870-1961).
+ */
+int fm_kv_append(const float* qkv, int q_cols, int kv_cols, int batch, int length, const float* keys,
+                 const float* values, int cached, int keep, float* comb, float* next_keys,
+                 float* next_values, hipStream_t stream);
+
+/*
  * Copies bytes0 bytes from src0 to dst0 and bytes1 from src1 to dst1 (device
  * memory, buffers not overlapping; a zero size skips its pair) in one launch
  * on `stream`.  No reference counterpart: the hipGraph runner uses it to move
