@@ -129,7 +129,10 @@ def check(status: int, name: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(library(), name)(*args), name)
+    lib = _lib if _lib is not None else library()
+    status = getattr(lib, name)(*args)
+    if status != 0:
+        check(status, name)
 
 
 def last_gemm_plan() -> str:

@@ -108,6 +108,41 @@ def op(entry: str):
     return getattr(torch.ops.fast_mimi_amd, entry[3:])
 
 
+_POINTERS = {entry: tuple(i for i, item in enumerate(spec.split()) if item[:3] in ("in:", "out", "res"))
+             for entry, spec in SPECS.items()}
+
+
+def _observed() -> bool:
+    """Whether something watches or transforms operator calls: a dispatch
+    mode (tracing, fake tensors), torch.compile, torch.jit.trace, a functorch
+    transform or the profiler."""
+    return bool(torch._C._len_torch_dispatch_stack() or torch.compiler.is_compiling()
+                or torch._C._get_tracing_state() is not None
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch._C._autograd._profiler_enabled())
+
+
 def call(entry: str, *args) -> None:
-    """Run C-ABI entry point ``entry`` through its operator."""
+    """Run C-ABI entry point ``entry``: through its operator when something
+    observes operator calls or a tensor is not a plain one (a subclass, or
+    one that requires a gradient), else the C function itself on the current
+    stream, which is all the operator's implementation does.  A streamed 80 ms
+    chunk is some 85 calls; the dispatcher's way took about 11 us of host time
+    each, this one about 4."""
+    if not _observed():
+        values = list(args)
+        device = None
+        for i in _POINTERS[entry]:
+            t = values[i]
+            if t is None:
+                continue
+            if type(t) is not torch.Tensor or t.requires_grad:
+                break
+            if device is None:
+                device = t.device
+            values[i] = t.data_ptr()
+        else:
+            if device is not None and device.type == "cuda":
+                nat.call(entry, *values, torch._C._cuda_getCurrentRawStream(device.index))
+                return
     getattr(torch.ops.fast_mimi_amd, entry[3:])(*args)

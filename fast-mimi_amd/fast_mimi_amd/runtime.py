@@ -258,6 +258,7 @@ class MimiRuntime:
                 ops.call("fm_pack_row_weights", layer.w, layer.c_out, layer.k * layer.c_in, layer.wr)
         self.workspace = torch.empty(_WORKSPACE_BYTES // 4, device=device)
         self._rope: dict[int, tuple[torch.Tensor, torch.Tensor]] = {}
+        self._stream_tabs: list[tuple[torch.Tensor, torch.Tensor]] = []
         # Optional per-op timing: a list of (tag, start_event, end_event).
         self.profile: list | None = None
         self._tag = ""
@@ -437,6 +438,26 @@ class MimiRuntime:
             tabs = (c.to(self.device), s.to(self.device))
             self._rope[length] = tabs
         return tabs
+
+    def _stream_rope(self, past: int, length: int) -> tuple[torch.Tensor, torch.Tensor]:
+        """RoPE rows ``past .. past + length - 1`` of one table that doubles as
+        streams get longer (a table per position would be built on the host
+        and uploaded at every chunk, and kept)."""
+        end = past + length
+        tabs = self._stream_tabs[-1] if self._stream_tabs else None
+        if tabs is None or tabs[0].shape[0] < end:
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError("RoPE tables must be prepared before graph capture")
+            size = 512
+            while size < end:
+                size *= 2
+            c, s = rope_tables(self.config, size)
+            tabs = (c.to(self.device), s.to(self.device))
+            # Shorter tables stay: a kernel in flight on another stream, or a
+            # graph a caller captured, may still read them (together they are
+            # no longer than the newest).
+            self._stream_tabs.append(tabs)
+        return tabs[0][past:end], tabs[1][past:end]
 
     def prepare(self, length: int) -> None:
         """Upload the RoPE tables a sequence of ``length`` frames needs."""
@@ -661,8 +682,7 @@ class MimiRuntime:
                  and lib.fm_row_linear_supported(nh * hd, C))
         kv.configure_sliding_window(cfg.sliding_window)
         past = kv.get_seq_length()
-        cos, sin = self._rope_tables(past + T)
-        cos, sin = cos[past:], sin[past:]
+        cos, sin = self._stream_rope(past, T)
         h = h.reshape(M, C)
         att = torch.empty((M, nh * hd), device=self.device)
         qd, kd = nh * hd, nkv * hd

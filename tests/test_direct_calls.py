@@ -1,0 +1,48 @@
+"""ops.call takes the C function directly only when nothing observes operator
+calls, and a streamed RoPE table is a slice of a longer one (CPU only)."""
+
+from __future__ import annotations
+
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from fast_mimi_amd import MimiConfig, ops
+from fast_mimi_amd.runtime import rope_tables
+
+
+def test_observers_keep_the_operator_path():
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    def look(x):
+        seen.append(ops._observed())
+        return x * 2
+
+    x = torch.ones(3)
+    assert not ops._observed()
+    with Mode():
+        look(x)
+    torch.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    torch.func.grad(lambda v: look(v).sum())(x)
+    torch.jit.trace(look, (x,), check_trace=False)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        look(x)
+    assert len(seen) >= 6 and all(seen)
+    assert not ops._observed()
+
+
+def test_pointer_arguments_follow_the_schema():
+    for entry, spec in ops.SPECS.items():
+        kinds = [item.split(":")[0] for item in spec.split()]
+        assert ops._POINTERS[entry] == tuple(i for i, k in enumerate(kinds) if k in ("in", "out", "res"))
+
+
+def test_rope_table_prefixes():
+    whole = rope_tables(MimiConfig(), 2048)
+    for n in (1, 2, 3, 7, 100, 251, 777, 2047):
+        for a, b in zip(whole, rope_tables(MimiConfig(), n)):
+            assert torch.equal(a[:n], b)
