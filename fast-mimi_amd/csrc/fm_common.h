@@ -132,12 +132,12 @@ FM_DEVICE floatx16 fm_mfma32_f16(halfx8 a, halfx8 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-FM_DEVICE void split2(floatx4 lo, floatx4 hi, float sc, halfx8& h0, halfx8& h1) {
+FM_DEVICE void split2(floatx4 v, float sc, halfx4& h0, halfx4& h1) {
   typedef _Float16 halfx2_t __attribute__((ext_vector_type(2)));
   typedef float floatx2_t __attribute__((ext_vector_type(2)));
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float a = q < 2 ? lo[2 * q] : hi[2 * q - 4], b = q < 2 ? lo[2 * q + 1] : hi[2 * q - 3];
+  for (int q = 0; q < 2; ++q) {
+    const float a = v[2 * q], b = v[2 * q + 1];
     const halfx2_t p = __builtin_convertvector((floatx2_t{a * sc, b * sc}), halfx2_t);
     // The residual a sc - h0 is exact in FP32.
     const halfx2_t r = __builtin_convertvector(
@@ -145,6 +145,19 @@ FM_DEVICE void split2(floatx4 lo, floatx4 hi, float sc, halfx8& h0, halfx8& h1) 
     h0[2 * q] = p[0], h0[2 * q + 1] = p[1];
     h1[2 * q] = r[0], h1[2 * q + 1] = r[1];
   }
+}
+FM_DEVICE void split2(floatx4 lo, floatx4 hi, float sc, halfx8& h0, halfx8& h1) {
+  halfx4 l0, l1, u0, u1;
+  split2(lo, sc, l0, l1);
+  split2(hi, sc, u0, u1);
+  h0 = __builtin_shufflevector(l0, u0, 0, 1, 2, 3, 4, 5, 6, 7);
+  h1 = __builtin_shufflevector(l1, u1, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+// The exponent s that brings a magnitude m > 0 into [2^to, 2^(to + 1)), kept
+// where 2^s and 2^-s are normal numbers; 0 for m = 0.
+FM_DEVICE int h3_exp_for(float m, int to) {
+  const int f = (int)(__builtin_bit_cast(unsigned, m) >> 23) & 255;
+  return m > 0.0f ? min(max(127 + to + 127 - f, 1), 253) - 127 : 0;
 }
 
 static inline int fm_ceil_div(long a, long b) { return (int)((a + b - 1) / b); }

@@ -1461,7 +1461,7 @@ void gemm_x6d_kernel(GemmArgs p, const __bf16* __restrict__ w3) {
 FM_DEVICE int h3_exp_field(float v) { return (int)(__builtin_bit_cast(unsigned, v) >> 23) & 255; }
 // 2^s as a float and the largest magnitude it may meet, for a row maximum m > 0
 // (s puts m in [2^9, 2^10); the exponent fields are clamped to normal numbers).
-FM_DEVICE int h3_scale_exp(float m) { return min(max(263 - h3_exp_field(m), 1), 253) - 127; }
+FM_DEVICE int h3_scale_exp(float m) { return h3_exp_for(m, 9); }
 FM_DEVICE float h3_limit(float m) {
   const int f = h3_exp_field(m) + 6;
   return __builtin_bit_cast(float, (unsigned)min(f, 255) << 23);  // 2^15 / 2^s, or inf
@@ -1480,9 +1480,10 @@ __global__ __launch_bounds__(256) void split_weights_h3_kernel(const float* __re
     if (tid < d) part[tid] = fmaxf(part[tid], part[tid + d]);
     __syncthreads();
   }
-  // The row maximum in [2^13, 2^14); a zero row keeps s = 0.
+  // The row maximum in [2^13, 2^14); a zero row takes the largest exponent, so
+  // that 2^(14 - min s) bounds every weight tightly (the residual blocks).
   const float top = part[0];
-  const int s = top > 0.0f ? min(max(267 - h3_exp_field(top), 1), 253) - 127 : 0;
+  const int s = top > 0.0f ? h3_exp_for(top, 13) : 126;
   const float sc = __builtin_bit_cast(float, (unsigned)(s + 127) << 23);
   const long NK = (long)N * K;
   if (tid == 0) reinterpret_cast<int*>(out + 2 * NK)[n] = s;

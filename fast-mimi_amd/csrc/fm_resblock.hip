@@ -14,6 +14,8 @@
 // e).  Weights are the packed conv layout: W1^T [C/2][3C] (k = tap*C + c_in)
 // and W2^T [C][C/2].
 
+#include <type_traits>
+
 #include "fm_common.h"
 
 namespace {
@@ -496,22 +498,37 @@ __global__ __launch_bounds__(NT, 3) void resblock_direct_kernel(
 // .. +7, so a wave's weight fragment (32 rows x 16 k) is one contiguous 1 KB
 // run (a [3][N][K] row-major layout spreads it over 32 cache lines, which the
 // per-CU address path, not the MFMAs, then limits: 1.55x slower).
-template <int C, int BM, int WM, int PD, bool WAVE_IN, bool WAVE_OUT, bool FAST_ACT = false>
-__global__ __launch_bounds__(NT, 3) void resblock_x6_kernel(
+//
+// H3: the same block on fp16 weights (fm_split_weights_h3) with three products
+// per operand pair and two planes per operand.  ELU(x) is scaled by one power
+// of two per block, from the block's largest magnitude (into [2^13, 2^14):
+// a value's error is 2^-23 of it or 2^-39 of that largest one); the hidden
+// tile by one from a bound on it, max |ELU(x)| * K1 * max |w1| + max |b1|
+// (some 2^6 above what it reaches, of fp16's 2^39 range), so neither can
+// overflow and no exchange between the waves is needed.  Accumulators return
+// to the caller's scale in one exact step.
+template <int C, int BM, int WM, int PD, bool WAVE_IN, bool WAVE_OUT, bool FAST_ACT = false, bool H3 = false>
+__global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     const float* __restrict__ x, int L, const __bf16* __restrict__ w1x, const float* __restrict__ b1,
     const __bf16* __restrict__ w2x, const float* __restrict__ b2, int elu_out, float* __restrict__ y,
     const float* __restrict__ w0, const float* __restrict__ b0) {
   constexpr int WN = 4 / WM, HC = C / 2, K1 = 3 * C;
+  // Planes per operand and their element type.
+  constexpr int NP = H3 ? 2 : 3;
+  using frag8 = std::conditional_t<H3, halfx8, bf16x8>;
   constexpr int XR = BM + 2, XPLANE = XR * C * 2, HPLANE = BM * HC * 2;
   constexpr int T1 = K1 / 32, T2 = HC / 32, FN2 = 2;
   constexpr int T = T1 + T2 * FN2;
   static_assert(BM == 32 * WM && HC / WN == 32 && C / WN == 32 * FN2, "wave tiling");
-  static_assert(3 * HPLANE <= 3 * XPLANE, "hidden planes fit over the ELU(x) planes");
+  static_assert(HPLANE <= XPLANE, "hidden planes fit over the ELU(x) planes");
   static_assert(!(WAVE_IN || WAVE_OUT) || (C == 64 && WM == 4), "waveform ends: one wave per 32 rows x 64 channels");
-  static_assert(!WAVE_OUT || 4 * 32 * 68 * 4 <= 3 * XPLANE, "output tiles fit");
+  constexpr int EBYTES = WAVE_OUT ? 4 * 32 * 68 * 4 : 0;  // WAVE_OUT's output tiles, over the consumed planes
+  static_assert(!(H3 && WAVE_IN), "the encoder's first block keeps its bf16 arithmetic");
   auto act = [](float v) { return FAST_ACT ? fm_elu_exp(v) : fm_elu(v); };
-  __shared__ __attribute__((aligned(16))) char smem[3 * XPLANE];
+  __shared__ __attribute__((aligned(16))) char smem[NP * XPLANE > EBYTES ? NP * XPLANE : EBYTES];
   __shared__ float wins[WAVE_IN ? BM + 8 : 1];  // WAVE_IN: waveform samples t0-8 .. t0+BM-1
+
+  __shared__ float topS[4];  // H3: each wave's largest |ELU(x)|
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, lcol = lane & 31;
@@ -598,11 +615,11 @@ __global__ __launch_bounds__(NT, 3) void resblock_x6_kernel(
   // Weight fragments through buffer resources: the lane's offset is fixed,
   // each unit's place in the planes is a scalar offset, so the streamed
   // loads take no vector address arithmetic.
-  const __amdgpu_buffer_rsrc_t rw1 = fm_buffer(w1x, 3 * HC * K1 * 2);
-  const __amdgpu_buffer_rsrc_t rw2 = fm_buffer(w2x, 3 * C * HC * 2);
+  const __amdgpu_buffer_rsrc_t rw1 = fm_buffer(w1x, NP * HC * K1 * 2);
+  const __amdgpu_buffer_rsrc_t rw2 = fm_buffer(w2x, NP * C * HC * 2);
   const int w1v = ((wc * 32 + lcol) * 16 + 8 * h) * 2, w2v = ((wc * 64 + lcol) * 16 + 8 * h) * 2;
-  bf16x8 ring[PD][3][2];
-  auto load_unit = [&](int u, bf16x8 (&d)[3][2]) {
+  frag8 ring[PD][NP][2];
+  auto load_unit = [&](int u, frag8 (&d)[NP][2]) {
     int base, plane;  // elements
     if (u < T1) {
       base = u * 2 * HC * 16;
@@ -614,60 +631,110 @@ __global__ __launch_bounds__(NT, 3) void resblock_x6_kernel(
     }
     const int tile = u < T1 ? HC * 16 : C * 16;  // elements per k16 tile of a plane
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl)
+    for (int pl = 0; pl < NP; ++pl)
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const int soff = (base + pl * plane + s * tile) * 2;
-        d[pl][s] = __builtin_bit_cast(bf16x8, u < T1 ? fm_buf_load4(rw1, w1v, soff) : fm_buf_load4(rw2, w2v, soff));
+        d[pl][s] = __builtin_bit_cast(frag8, u < T1 ? fm_buf_load4(rw1, w1v, soff) : fm_buf_load4(rw2, w2v, soff));
       }
   };
 #pragma unroll
   for (int d = 0; d < PD; ++d) load_unit(d, ring[d]);
+  // H3: row exponents of the two weights (after their planes), the block's
+  // scale 2^sx and the hidden tile's 2^sh.
+  const int* e1 = reinterpret_cast<const int*>(w1x + 2 * HC * K1);
+  const int* e2 = reinterpret_cast<const int*>(w2x + 2 * C * HC);
+  int sx = 0, sh = 0;
+  if constexpr (H3) {
+    float top = 0.0f, bmax = 0.0f;
+    int emin = 127;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xv[u][e] = act(xv[u][e]);
+        const float m = fabsf(xv[u][e]);
+        top = fmaxf(top, m < INFINITY ? m : 0.0f);  // a non-finite value spoils its own outputs only
+      }
+#pragma unroll
+    for (int n = 0; n < (HC + 63) / 64; ++n) {
+      const int i = min(lane + 64 * n, HC - 1);
+      emin = min(emin, e1[i]);
+      bmax = fmaxf(bmax, fabsf(b1[i]));
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      top = fmaxf(top, __shfl_xor(top, o, 64));
+      emin = min(emin, __shfl_xor(emin, o, 64));
+      bmax = fmaxf(bmax, __shfl_xor(bmax, o, 64));
+    }
+    if (lane == 0) topS[wave] = top;
+    __syncthreads();
+    top = fmaxf(fmaxf(topS[0], topS[1]), fmaxf(topS[2], topS[3]));
+    sx = h3_exp_for(top, 13);
+    // |w1| < 2^(14 - emin): the bound in [2^14, 2^15).
+    sh = h3_exp_for(__builtin_amdgcn_ldexpf(top * K1, 14 - emin) + bmax, 14);
+  }
+  const float scx = __builtin_amdgcn_ldexpf(1.0f, sx), sch = __builtin_amdgcn_ldexpf(1.0f, sh);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int c = tid + u * NT;
     if (c >= CH) continue;
     const int r = c / (C / 4), k = (c % (C / 4)) * 4;
-    bf16x4 p0, p1, p2;
-    split3(floatx4{act(xv[u].x), act(xv[u].y), act(xv[u].z), act(xv[u].w)}, p0, p1, p2);
-    char* dst = smem + chunk(r, k >> 3, C * 2) + (k & 4) * 2;
-    *reinterpret_cast<bf16x4*>(dst) = p0;
-    *reinterpret_cast<bf16x4*>(dst + XPLANE) = p1;
-    *reinterpret_cast<bf16x4*>(dst + 2 * XPLANE) = p2;
+    if constexpr (H3) {
+      halfx4 p0, p1;
+      split2(xv[u], scx, p0, p1);
+      char* dst = smem + chunk(r, k >> 3, C * 2) + (k & 4) * 2;
+      *reinterpret_cast<halfx4*>(dst) = p0;
+      *reinterpret_cast<halfx4*>(dst + XPLANE) = p1;
+    } else {
+      bf16x4 p0, p1, p2;
+      split3(floatx4{act(xv[u].x), act(xv[u].y), act(xv[u].z), act(xv[u].w)}, p0, p1, p2);
+      char* dst = smem + chunk(r, k >> 3, C * 2) + (k & 4) * 2;
+      *reinterpret_cast<bf16x4*>(dst) = p0;
+      *reinterpret_cast<bf16x4*>(dst + XPLANE) = p1;
+      *reinterpret_cast<bf16x4*>(dst + 2 * XPLANE) = p2;
+    }
   }
   __syncthreads();
 
   // k3 conv, transposed: acc[hidden][position].  The B fragments (ELU(x)
   // planes) of the next unit are read while the current unit's MFMAs run.
   const int prow = wr * 32 + lcol;
-  auto load_x = [&](int u, bf16x8 (&a)[3][2]) {
+  auto load_x = [&](int u, frag8 (&a)[NP][2]) {
     const int kk0 = u * 32, tap = kk0 / C, c0 = (kk0 % C) / 8 + h;
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl)
+    for (int pl = 0; pl < NP; ++pl)
 #pragma unroll
       for (int s = 0; s < 2; ++s)
-        a[pl][s] = *reinterpret_cast<const bf16x8*>(smem + pl * XPLANE + chunk(prow + tap, c0 + 2 * s, C * 2));
+        a[pl][s] = *reinterpret_cast<const frag8*>(smem + pl * XPLANE + chunk(prow + tap, c0 + 2 * s, C * 2));
   };
   floatx16 acc1[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc1[i][r] = 0.0f;
-  bf16x8 xf[2][3][2];
+  frag8 xf[2][NP][2];
   load_x(0, xf[0]);
 #pragma unroll
   for (int u = 0; u < T1; ++u) {
     if (u + 1 < T1) load_x(u + 1, xf[(u + 1) & 1]);
-    const bf16x8(&w)[3][2] = ring[u % PD];
-    const bf16x8(&a)[3][2] = xf[u & 1];
+    const frag8(&w)[NP][2] = ring[u % PD];
+    const frag8(&a)[NP][2] = xf[u & 1];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      acc1[0] = fm_mfma32_bf16(w[1][s], a[1][s], acc1[0]);
-      acc1[1] = fm_mfma32_bf16(w[2][s], a[0][s], acc1[1]);
-      acc1[0] = fm_mfma32_bf16(w[1][s], a[0][s], acc1[0]);
-      acc1[1] = fm_mfma32_bf16(w[0][s], a[2][s], acc1[1]);
-      acc1[0] = fm_mfma32_bf16(w[0][s], a[1][s], acc1[0]);
-      acc1[1] = fm_mfma32_bf16(w[0][s], a[0][s], acc1[1]);
+      if constexpr (H3) {
+        acc1[0] = fm_mfma32_f16(w[1][s], a[0][s], acc1[0]);
+        acc1[1] = fm_mfma32_f16(w[0][s], a[0][s], acc1[1]);
+        acc1[0] = fm_mfma32_f16(w[0][s], a[1][s], acc1[0]);
+      } else {
+        acc1[0] = fm_mfma32_bf16(w[1][s], a[1][s], acc1[0]);
+        acc1[1] = fm_mfma32_bf16(w[2][s], a[0][s], acc1[1]);
+        acc1[0] = fm_mfma32_bf16(w[1][s], a[0][s], acc1[0]);
+        acc1[1] = fm_mfma32_bf16(w[0][s], a[2][s], acc1[1]);
+        acc1[0] = fm_mfma32_bf16(w[0][s], a[1][s], acc1[0]);
+        acc1[1] = fm_mfma32_bf16(w[0][s], a[0][s], acc1[1]);
+      }
     }
     if (u + PD < T) load_unit(u + PD, ring[u % PD]);
     __builtin_amdgcn_sched_barrier(0);
@@ -679,14 +746,27 @@ __global__ __launch_bounds__(NT, 3) void resblock_x6_kernel(
     for (int g = 0; g < 4; ++g) {
       const floatx4 bb = *reinterpret_cast<const floatx4*>(b1 + wc * 32 + 8 * g + 4 * h);
       floatx4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = act(__fadd_rn(__fadd_rn(acc1[0][4 * g + e], acc1[1][4 * g + e]), bb[e]));
-      bf16x4 p0, p1, p2;
-      split3(v, p0, p1, p2);
       char* dst = smem + chunk(prow, wc * 4 + g, HC * 2) + 8 * h;
-      *reinterpret_cast<bf16x4*>(dst) = p0;
-      *reinterpret_cast<bf16x4*>(dst + HPLANE) = p1;
-      *reinterpret_cast<bf16x4*>(dst + 2 * HPLANE) = p2;
+      if constexpr (H3) {
+        const int4 en = *reinterpret_cast<const int4*>(e1 + wc * 32 + 8 * g + 4 * h);
+        const int es[4] = {en.x, en.y, en.z, en.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[e] = act(__fadd_rn(__builtin_amdgcn_ldexpf(__fadd_rn(acc1[0][4 * g + e], acc1[1][4 * g + e]),
+                                                       -(es[e] + sx)), bb[e]));
+        halfx4 p0, p1;
+        split2(v, sch, p0, p1);
+        *reinterpret_cast<halfx4*>(dst) = p0;
+        *reinterpret_cast<halfx4*>(dst + HPLANE) = p1;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = act(__fadd_rn(__fadd_rn(acc1[0][4 * g + e], acc1[1][4 * g + e]), bb[e]));
+        bf16x4 p0, p1, p2;
+        split3(v, p0, p1, p2);
+        *reinterpret_cast<bf16x4*>(dst) = p0;
+        *reinterpret_cast<bf16x4*>(dst + HPLANE) = p1;
+        *reinterpret_cast<bf16x4*>(dst + 2 * HPLANE) = p2;
+      }
     }
   }
   __syncthreads();
@@ -721,27 +801,41 @@ __global__ __launch_bounds__(NT, 3) void resblock_x6_kernel(
     for (int r = 0; r < 16; ++r) acc2[j][r] = 0.0f;
 #pragma unroll
   for (int kt = 0; kt < T2; ++kt) {
-    bf16x8 a[3][2];
+    frag8 a[NP][2];
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl)
+    for (int pl = 0; pl < NP; ++pl)
 #pragma unroll
       for (int s = 0; s < 2; ++s)
-        a[pl][s] = *reinterpret_cast<const bf16x8*>(smem + pl * HPLANE + chunk(prow, kt * 4 + 2 * s + h, HC * 2));
+        a[pl][s] = *reinterpret_cast<const frag8*>(smem + pl * HPLANE + chunk(prow, kt * 4 + 2 * s + h, HC * 2));
 #pragma unroll
     for (int j = 0; j < FN2; ++j) {
       const int u = T1 + kt * FN2 + j;
-      const bf16x8(&w)[3][2] = ring[u % PD];
+      const frag8(&w)[NP][2] = ring[u % PD];
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        acc2[j] = fm_mfma32_bf16(a[1][s], w[1][s], acc2[j]);
-        acc2[j] = fm_mfma32_bf16(a[2][s], w[0][s], acc2[j]);
-        acc2[j] = fm_mfma32_bf16(a[1][s], w[0][s], acc2[j]);
-        acc2[j] = fm_mfma32_bf16(a[0][s], w[2][s], acc2[j]);
-        acc2[j] = fm_mfma32_bf16(a[0][s], w[1][s], acc2[j]);
-        acc2[j] = fm_mfma32_bf16(a[0][s], w[0][s], acc2[j]);
+        if constexpr (H3) {
+          acc2[j] = fm_mfma32_f16(a[1][s], w[0][s], acc2[j]);
+          acc2[j] = fm_mfma32_f16(a[0][s], w[1][s], acc2[j]);
+          acc2[j] = fm_mfma32_f16(a[0][s], w[0][s], acc2[j]);
+        } else {
+          acc2[j] = fm_mfma32_bf16(a[1][s], w[1][s], acc2[j]);
+          acc2[j] = fm_mfma32_bf16(a[2][s], w[0][s], acc2[j]);
+          acc2[j] = fm_mfma32_bf16(a[1][s], w[0][s], acc2[j]);
+          acc2[j] = fm_mfma32_bf16(a[0][s], w[2][s], acc2[j]);
+          acc2[j] = fm_mfma32_bf16(a[0][s], w[1][s], acc2[j]);
+          acc2[j] = fm_mfma32_bf16(a[0][s], w[0][s], acc2[j]);
+        }
       }
       if (u + PD < T) load_unit(u + PD, ring[u % PD]);
       __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if constexpr (H3) {
+#pragma unroll
+    for (int j = 0; j < FN2; ++j) {
+      const int e = -(e2[wc * 64 + j * 32 + lcol] + sh);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc2[j][r] = __builtin_amdgcn_ldexpf(acc2[j][r], e);
     }
   }
   if constexpr (WAVE_OUT) {
@@ -808,6 +902,11 @@ static const __bf16* planes_after(const float* w, int rows, int cols) {
   return reinterpret_cast<const __bf16*>(w + (long)rows * cols);
 }
 
+// The fp16 planes and row exponents after the bf16 planes (fm_split_weights_h3).
+static const __bf16* h3_planes_after(const float* w, int rows, int cols) {
+  return reinterpret_cast<const __bf16*>(w + (long)rows * cols) + 3L * rows * cols;
+}
+
 extern "C" {
 
 // Channel widths with a fused kernel; others run as two fm_conv1d calls.
@@ -825,7 +924,18 @@ int fm_resblock(const float* x, int batch, int length, int channels, const float
   if (batch == 0 || length == 0) return FM_OK;
   const int elu = (elu_out & ~(FM_WEIGHTS_X6 | FM_WEIGHTS_H3 | FM_ACT_EXP)) != 0;
   const bool x6 = elu_out & FM_WEIGHTS_X6, fa = elu_out & FM_ACT_EXP;
-  if (x6) {
+  if ((elu_out & FM_WEIGHTS_H3) && fa) {
+    const __bf16* w1h = h3_planes_after(w1_packed, channels / 2, 3 * channels);
+    const __bf16* w2h = h3_planes_after(w2_packed, channels, channels / 2);
+#define FM_RBH(C_, BM_, WM_)                                                                                         \
+  hipLaunchKernelGGL((resblock_x6_kernel<C_, BM_, WM_, 2, false, false, true, true>),                                \
+                     dim3((length + BM_ - 1) / BM_, batch), dim3(NT), 0, stream, x, length, w1h, b1, w2h, b2, elu, y, \
+                     nullptr, nullptr)
+    if (channels == 64) FM_RBH(64, 128, 4);
+    else if (channels == 128) FM_RBH(128, 64, 2);
+    else FM_RBH(256, 32, 1);
+#undef FM_RBH
+  } else if (x6) {
     // Split planes follow each packed weight (fm_split_weights).
     const __bf16* w1x = planes_after(w1_packed, channels / 2, 3 * channels);
     const __bf16* w2x = planes_after(w2_packed, channels, channels / 2);
@@ -903,7 +1013,11 @@ int fm_resblock64_conv(const float* x, int batch, int length, const float* w1_pa
   if (!workspace || workspace_bytes < fm_resblock64_conv_workspace_bytes(batch, length))
     return FM_WORKSPACE_TOO_SMALL;
   const int elu = (elu_mid & ~(FM_WEIGHTS_X6 | FM_WEIGHTS_H3 | FM_ACT_EXP)) != 0;
-  if (elu_mid & FM_WEIGHTS_X6) {
+  if ((elu_mid & FM_WEIGHTS_H3) && (elu_mid & FM_ACT_EXP)) {
+    hipLaunchKernelGGL((resblock_x6_kernel<64, 128, 4, 2, false, true, true, true>), dim3((length + 127) / 128, batch),
+                       dim3(NT), 0, stream, x, length, h3_planes_after(w1_packed, 32, 192), b1,
+                       h3_planes_after(w2_packed, 64, 32), b2, elu, workspace, w3_packed, nullptr);
+  } else if (elu_mid & FM_WEIGHTS_X6) {
     if (elu_mid & FM_ACT_EXP)
       hipLaunchKernelGGL((resblock_x6_kernel<64, 128, 4, 2, false, true, true>), dim3((length + 127) / 128, batch),
                          dim3(NT), 0, stream, x, length, planes_after(w1_packed, 32, 192), b1,

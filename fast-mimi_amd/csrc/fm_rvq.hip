@@ -976,7 +976,7 @@ __global__ __launch_bounds__(256) void rvq_screen_prepare_kernel(const float* __
   }
   m = red[0][0];
   // m in [2^9, 2^10) after scaling.
-  const int s = m > 0.0f && !bad ? min(max(263 - (int)(__builtin_bit_cast(unsigned, m) >> 23), 1), 253) - 127 : 0;
+  const int s = bad ? 0 : h3_exp_for(m, 9);
   const float sc = __builtin_bit_cast(float, (unsigned)(s + 127) << 23);
   if (threadIdx.x == 0) info[cb] = ScreenInfo{s, bad ? INFINITY : sqrtf(red[1][0]) * 1.0001f};
   for (long i = threadIdx.x; i < (long)entries * 256; i += 256) {
@@ -1093,7 +1093,7 @@ void rvq_screen_kernel(ScreenArgs a) {
         xn += __shfl_xor(xn, o, 64);
         top = fmaxf(top, __shfl_xor(top, o, 64));
       }
-      const int s = top > 0.0f ? min(max(263 - (int)(__builtin_bit_cast(unsigned, top) >> 23), 1), 253) - 127 : 0;
+      const int s = h3_exp_for(top, 9);
       const float sc = __builtin_bit_cast(float, (unsigned)(s + 127) << 23);
 #pragma unroll
       for (int u = 0; u < CH; ++u) {

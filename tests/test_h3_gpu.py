@@ -199,3 +199,74 @@ def test_linear_rope_equals_linear_then_rope(rows, per_seq, n, rope_cols, ws):
              rope_cols, per_seq, got.data_ptr(), ws.data_ptr(), WS_BYTES, stream())
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+def block_reference(x, w1, b1, w2, b2):
+    """float64 block output [B, C, L] and the scale its error is held to: the
+    same sums on absolute values."""
+    a = F.elu(x)
+    hid = F.elu(causal_conv1d(a, w1, b1))
+    ref = causal_conv1d(a.abs(), w1.abs(), b1.abs())
+    return x + causal_conv1d(hid, w2, b2), x.abs() + causal_conv1d(ref, w2.abs(), b2.abs())
+
+
+@pytest.mark.parametrize("C,B,L", [(64, 1, 1000), (64, 2, 129), (128, 1, 777), (128, 3, 1), (128, 2, 66), (256, 1, 2000),
+                                   (256, 2, 33), (256, 1, 31)])
+@pytest.mark.parametrize("kind", ["plain", "loud_quiet", "zero_channels", "tiny"])
+def test_resblock(C, B, L, kind):
+    """The fp16 residual block against float64, no further from it than the
+    bf16 one; rows far below their neighbours, hidden channels of zero weight
+    and whole inputs near 1e-25 (the block's scales are dynamic).  ELU as
+    e^x - 1 adds an absolute error of a few 2^-24 to either form."""
+    g = torch.Generator().manual_seed(C + L)
+    x = torch.randn(B, C, L, generator=g)
+    w1, b1 = torch.randn(C // 2, C, 3, generator=g) / math.sqrt(3 * C), 0.1 * torch.randn(C // 2, generator=g)
+    w2, b2 = torch.randn(C, C // 2, 1, generator=g) / math.sqrt(C // 2), 0.1 * torch.randn(C, generator=g)
+    if kind == "loud_quiet":
+        x *= 10.0 ** (torch.arange(L) % 5 - 2)
+    elif kind == "zero_channels":
+        w1[::3] = 0
+    elif kind == "tiny":
+        x, b1, b2 = x * 1e-25, b1 * 0, b2 * 0
+    c1, c2 = _Conv(w1.to(DEV), b1.to(DEV)), _Conv(w2.to(DEV), b2.to(DEV))
+    (w1p, _), (w2p, _) = with_planes(c1.w), with_planes(c2.w)
+    xd = x.transpose(1, 2).contiguous().to(DEV)
+    want, absref = block_reference(*(t.double() for t in (x, w1, b1, w2, b2)))
+    out = {}
+    for flags in (FLAGS, nat.WEIGHTS_X6):
+        y = torch.full_like(xd, float("nan"))
+        nat.call("fm_resblock", xd.data_ptr(), B, L, C, w1p.data_ptr(), c1.b.data_ptr(), w2p.data_ptr(),
+                 c2.b.data_ptr(), flags | nat.ACT_EXP, y.data_ptr(), stream())
+        torch.cuda.synchronize()
+        out[flags] = y.cpu().double().transpose(1, 2)
+    # (FLAGS without bit 1 has no trailing ELU; the e^x - 1 error passes through both convs.)
+    if kind != "tiny":
+        close_dot(out[FLAGS], want, absref + 1.0)
+    err, was = ((v - want).norm() for v in out.values())
+    assert err <= 1.1 * was + 1e-7 * want.norm()
+
+
+@pytest.mark.parametrize("B,L,y_len", [(1, 1000, 1000), (2, 129, 100), (3, 33, 33), (1, 1, 1)])
+def test_resblock64_conv(B, L, y_len):
+    """The decoder's last block and waveform conv on fp16 weights."""
+    g = torch.Generator().manual_seed(L)
+    x = torch.randn(B, 64, L, generator=g)
+    w1, b1 = torch.randn(32, 64, 3, generator=g) / math.sqrt(192), 0.1 * torch.randn(32, generator=g)
+    w2, b2 = torch.randn(64, 32, 1, generator=g) / math.sqrt(32), 0.1 * torch.randn(64, generator=g)
+    w3, b3 = torch.randn(1, 64, 3, generator=g) / math.sqrt(192), torch.randn(1, generator=g)
+    c1, c2, c3 = (_Conv(w.to(DEV), b.to(DEV)) for w, b in ((w1, b1), (w2, b2), (w3, b3)))
+    (w1p, _), (w2p, _) = with_planes(c1.w), with_planes(c2.w)
+    xd = x.transpose(1, 2).contiguous().to(DEV)
+    d = torch.empty(nat.library().fm_resblock64_conv_workspace_bytes(B, L) // 4, device=DEV)
+    blk, _ = block_reference(*(t.double() for t in (x, w1, b1, w2, b2)))
+    want = causal_conv1d(F.elu(blk), w3.double(), b3.double())[..., :y_len]
+    errs = []
+    for flags in (FLAGS, nat.WEIGHTS_X6):
+        y = torch.full((B, y_len), float("nan"), device=DEV)
+        nat.call("fm_resblock64_conv", xd.data_ptr(), B, L, w1p.data_ptr(), c1.b.data_ptr(), w2p.data_ptr(),
+                 c2.b.data_ptr(), 1 | flags | nat.ACT_EXP, c3.w.data_ptr(), c3.b.data_ptr(), y_len, y.data_ptr(),
+                 d.data_ptr(), d.numel() * 4, stream())
+        torch.cuda.synchronize()
+        errs.append((y.cpu().double()[:, None] - want).norm())
+        assert (y.cpu().double()[:, None] - want).abs().max() <= 2e-5 * want.abs().max()
+    assert errs[0] <= 1.1 * errs[1] + 1e-7 * want.norm()
