@@ -902,7 +902,7 @@ __global__ __launch_bounds__(256) void rvq_decode_kernel(const int64_t* codes, i
 //   screen: approximate distances of the rows to every entry from one fp16
 //     MFMA product per 16 dims (entries and rows scaled by powers of two),
 //     eight waves striding over 32-entry tiles whose fragments stream from L2
-//     one tile ahead, across steps too; each lane keeps the three smallest
+//     one tile ahead, across steps too; each lane keeps the four smallest
 //     of the 128 distances it sees;
 //   candidates: the entries within `margin` of the row's smallest screened
 //     distance.  margin bounds twice the largest difference between a
@@ -916,7 +916,7 @@ __global__ __launch_bounds__(256) void rvq_decode_kernel(const int64_t* codes, i
 //     32x32x2 FP32 MFMA rounds like fma(a1, b1, fma(a0, b0, c)), so one lane's
 //     FMA chain in its dim order gives the same bits.
 // A row that cannot be screened (non-finite values or margin, or a lane whose
-// third smallest distance is a candidate too) sends the block through the
+// fourth smallest distance is a candidate too) sends the block through the
 // FP32 MFMA scan of every entry for that step.  The codes are therefore
 // those of the step kernel bit for bit.
 // Bound by the fp16 codebook stream, 1 MB per step and CU through the L1 port
@@ -992,7 +992,7 @@ void rvq_screen_kernel(ScreenArgs a) {
   __shared__ __attribute__((aligned(16))) float Xs[RB * PX];       // residual rows, FP32
   __shared__ __attribute__((aligned(16))) char Xh[RB * DIM * 2];   // their fp16 fragments [k16][half][row][8]
   __shared__ __attribute__((aligned(16))) float normS[SCREEN_ENTRIES];
-  __shared__ float low[3][2 * SCREEN_WAVES][RB + 1];  // each lane list's smallest three keys per row
+  __shared__ float low[4][2 * SCREEN_WAVES][RB + 1];  // each lane list's smallest four keys per row
   __shared__ float xnS[RB], coefS[RB], marginS[RB];
   __shared__ int codeS[RB];
   __shared__ unsigned long long exactS[RB];  // (ordered distance, entry) minimum over a row's candidates
@@ -1109,7 +1109,7 @@ void rvq_screen_kernel(ScreenArgs a) {
         // Twice the bound on |screened - FP32| (see above), X = |x|, T = top norm.
         const float X = sqrtf(xn) * 1.0001f, T = info.top;
         marginS[wr] =
-            2.0f * (X * T * (0x1p-9f + 0x1p-11f) + T * T * 0x1p-15f + (xn + T * T) * 0x1p-19f) + 0x1p-96f;
+            2.0f * (X * T * (0x1p-9f + 0x1p-13f) + T * T * 0x1p-15f + (xn + T * T) * 0x1p-20f) + 0x1p-96f;
         exactS[wr] = ~0ull;
       }
     }
@@ -1122,7 +1122,7 @@ void rvq_screen_kernel(ScreenArgs a) {
 #pragma unroll
     for (int k = 0; k < KF; ++k) q[k] = *reinterpret_cast<const halfx8*>(Xh + k * 1024 + h * 512 + col * 16);
     const float coef = coefS[col];
-    float l1 = INFINITY, l2 = INFINITY, l3 = INFINITY;
+    float l1 = INFINITY, l2 = INFINITY, l3 = INFINITY, l4 = INFINITY;
     for (int t = 0; t < mine; ++t) {
       const int tile = wave + SCREEN_WAVES * t;
       // The next tile of this wave: of the next codebook after the last.
@@ -1145,6 +1145,7 @@ void rvq_screen_kernel(ScreenArgs a) {
           // The key's low 7 bits name the entry within this lane.
           const float key = __builtin_bit_cast(
               float, (__builtin_bit_cast(unsigned, d) & ~127u) | (unsigned)(16 * t + 4 * g + e));
+          l4 = __builtin_amdgcn_fmed3f(l3, l4, key);
           l3 = __builtin_amdgcn_fmed3f(l2, l3, key);
           l2 = __builtin_amdgcn_fmed3f(l1, l2, key);
           l1 = fminf(l1, key);
@@ -1154,6 +1155,7 @@ void rvq_screen_kernel(ScreenArgs a) {
     low[0][2 * wave + h][col] = l1;
     low[1][2 * wave + h][col] = l2;
     low[2][2 * wave + h][col] = l3;
+    low[3][2 * wave + h][col] = l4;
     // The next step's norms and scale.
     if (tid < a.entries / 4) nv = *reinterpret_cast<const floatx4*>(a.norms + (long)next * a.entries + 4 * tid);
     info = a.info[next];
@@ -1163,33 +1165,31 @@ void rvq_screen_kernel(ScreenArgs a) {
     asm volatile("" : "+v"(lt));
     {
       const int r = lt >> 4, s = lt & 15;
-      const float k1 = low[0][s][r], k2 = low[1][s][r], k3 = low[2][s][r];
+      const float k1 = low[0][s][r], k2 = low[1][s][r], k3 = low[2][s][r], k4 = low[3][s][r];
       float best = k1;
 #pragma unroll
       for (int o = 1; o < 16; o <<= 1) best = fminf(best, __shfl_xor(best, o, 64));
       const float lim = best + marginS[r];
       const bool finite = fabsf(lim) < INFINITY;  // false for a NaN too
-      const bool c1 = k1 <= lim, c2 = k2 <= lim;
-      const unsigned long long m1 = __ballot(c1) >> (lane & 48) & 0xffff, m2 = __ballot(c2) >> (lane & 48) & 0xffff;
-      const int n = __popcll(m1) + __popcll(m2);
+      const bool c1 = k1 <= lim, c2 = k2 <= lim, c3 = k3 <= lim;
+      // (c2 implies c1, c3 both: one candidate is one c1 and no c2.)
+      const int n = __popcll(__ballot(c1) >> (lane & 48) & 0xffff) + __popcll(__ballot(c2) >> (lane & 48) & 0xffff);
       auto entry_of = [&](float key) {
         const int tag = (int)(__builtin_bit_cast(unsigned, key) & 127u);
         return 32 * ((s >> 1) + SCREEN_WAVES * (tag >> 4)) + 8 * ((tag & 15) >> 2) + 4 * (s & 1) + (tag & 3);
       };
-      if (m0 + r < a.M && (!finite || k3 <= lim)) fullS = 1;
+      auto candidate = [&](float key) {
+        const int p = atomicAdd(&npairS, 1);
+        if (p < SCREEN_PAIRS) pairS[p] = r << 16 | entry_of(key);
+        else fullS = 1;
+      };
+      if (m0 + r < a.M && (!finite || k4 <= lim)) fullS = 1;
       if (finite && n == 1) {
         if (c1) codeS[r] = entry_of(k1);
       } else if (finite && m0 + r < a.M) {
-        if (c1) {
-          const int p = atomicAdd(&npairS, 1);
-          if (p < SCREEN_PAIRS) pairS[p] = r << 16 | entry_of(k1);
-          else fullS = 1;
-        }
-        if (c2) {
-          const int p = atomicAdd(&npairS, 1);
-          if (p < SCREEN_PAIRS) pairS[p] = r << 16 | entry_of(k2);
-          else fullS = 1;
-        }
+        if (c1) candidate(k1);
+        if (c2) candidate(k2);
+        if (c3) candidate(k3);
         if (s == 0) codeS[r] = -1;
       } else if (s == 0) {
         codeS[r] = 0;
