@@ -1281,6 +1281,15 @@ void rvq_screen_kernel(ScreenArgs a) {
   if (former) decide(a.count - 1, (tid - 256) >> 3, (tid & 7) == 0);
 }
 
+__global__ __launch_bounds__(256) void codes_check_kernel(const int64_t* __restrict__ codes, long n, int entries,
+                                                          int* flag) {
+  bool bad = false;
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256)
+    bad |= (uint64_t)codes[i] >= (uint64_t)entries;
+  // (Every writer stores the same value.)
+  if (__any(bad) && (threadIdx.x & 63) == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 size_t step_lds_bytes(int dim) {
   return (size_t)dim * (RB + 1) * 4 + (size_t)KSL * PB * 4 + RB * 4 + 4 * RB * 4 + 4 * RB * 4 +
          RB * 4;
@@ -1584,6 +1593,18 @@ int fm_rvq_encode_split(const float* x, int ld_x, int rows, int rows_per_batch, 
     if (e != hipSuccess) return e;
   }
   return FM_OK;
+}
+
+// Out-of-range check of a code tensor: *flag becomes 1 if any code lies outside
+// [0, entries), else stays as it is.  One pass where a min / max reduction, its
+// packing and its copy took three launches.
+int fm_codes_check(const int64_t* codes, size_t count, int entries, int* flag, hipStream_t stream) {
+  if (!codes || !flag || entries <= 0 || (long)count < 0) return FM_BAD_ARGUMENT;
+  if (count == 0) return FM_OK;
+  const long blocks = ((long)count + 255) / 256;
+  hipLaunchKernelGGL(codes_check_kernel, dim3((unsigned)std::min(blocks, 1024L)), dim3(256), 0, stream, codes,
+                     (long)count, entries, flag);
+  return (int)hipGetLastError();
 }
 
 int fm_rvq_decode(const int64_t* codes, int batch, int num_codebooks, int frames,

@@ -78,6 +78,7 @@ _SIGNATURES = {
     "fm_rvq_encode_split_screened": ([_P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P], _I),
     "fm_rvq_noalloc_scratch_bytes": ([], _S),
     "fm_rvq_encode_split_noalloc": ([_P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P], _I),
+    "fm_codes_check": ([_P, _S, _I, _P, _P], _I),
     "fm_rvq_decode": ([_P, _I, _I, _I, _I, _P, _I, _I, _P, _P], _I),
     "fm_upsample_depthwise": ([_P, _I, _I, _I, _P, _I, _I, _P, _P], _I),
     "fm_stream_append": ([_P, _P, _I, _I, _I, _I, _I, _P, _P, _P], _I),

@@ -159,6 +159,38 @@ def _copy_pairs(pairs, device) -> None:
                  0 if s1 is None else s1.numel() * s1.element_size(), stream)
 
 
+class _CodesCheck:
+    """One decode call's out-of-range check, in flight on the current stream:
+    the kernel sets a flag in pinned memory, an event marks it done.  Flags
+    are pooled on the model (as many as its calls overlap)."""
+
+    def __init__(self, model: "MimiModel", codes: torch.Tensor) -> None:
+        self.slot = None
+        if not codes.numel():
+            return
+        self.pool = model._check_flags
+        try:
+            self.slot = self.pool.pop()
+        except IndexError:
+            flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            self.slot = (flag, flag.numpy(), torch.cuda.Event())
+        flag, value, event = self.slot
+        value[0] = 0
+        nat.call("fm_codes_check", codes.data_ptr(), codes.numel(), model.config.codebook_size,
+                 flag.data_ptr(), torch.cuda.current_stream(codes.device).cuda_stream)
+        event.record()
+
+    def bad(self) -> bool:
+        """Wait for the check; whether some code was out of range."""
+        if self.slot is None:
+            return False
+        slot, self.slot = self.slot, None
+        slot[2].synchronize()
+        bad = bool(slot[1][0])
+        self.pool.append(slot)
+        return bad
+
+
 class MimiModel:
     """Mimi neural audio codec on one MI355X GPU."""
 
@@ -178,6 +210,7 @@ class MimiModel:
         self.use_graphs = use_graphs
         self._runtime = None
         self._graphs: dict[tuple, _GraphRunner] = {}
+        self._check_flags: list = []  # free (pinned flag, event) pairs of _CodesCheck
         self.training = False
         if device is not None:
             self.to(device)
@@ -215,6 +248,7 @@ class MimiModel:
     def _invalidate(self) -> None:
         self._runtime = None
         self._graphs.clear()
+        self._check_flags = []
 
     def to(self, device=None, dtype=None) -> "MimiModel":
         if dtype is not None and dtype != torch.float32:
@@ -395,24 +429,35 @@ class MimiModel:
             raise ValueError(f"audio_codes must hold 1..{self.config.num_quantizers} codebooks")
         rt = self.runtime()
         codes = self._on_device(audio_codes, torch.int64)
-        if codes.numel():
-            lo, hi = torch.aminmax(codes)
-            lo, hi = torch.stack((lo, hi)).tolist()  # one device->host sync
-            if lo < 0 or hi >= self.config.codebook_size:
-                raise IndexError("audio code out of range of the codebook")
         out_len = None if padding_mask is None else padding_mask.shape[-1]
         frames = codes.shape[-1]
         kv = decoder_past_key_values
         with torch.cuda.device(self.device), torch.inference_mode():
-            if kv is not None:
-                audio = rt.decode(codes, out_len, kv)
-            elif self.use_graphs:
-                rt.prepare(frames * (2 if rt.bottleneck else 1))
-                audio = self._graph(("dec", tuple(codes.shape), out_len),
-                                    lambda c: rt.decode(c, out_len), (codes,))
-            else:
-                rt.prepare(frames * (2 if rt.bottleneck else 1))
-                audio = rt.decode(codes, out_len)
+            # The work is queued behind the range check and the check's answer
+            # awaited before the call returns (the decode kernel reads no entry
+            # for a code out of range), so the GPU does not idle over a round
+            # trip to the host.  A caller's own cache type may not be undone,
+            # so it waits first.
+            check = _CodesCheck(self, codes)
+            ours = type(kv) is MimiKVCache
+            if kv is not None and not ours and check.bad():
+                raise IndexError("audio code out of range of the codebook")
+            saved = {k: list(v) if isinstance(v, list) else v for k, v in vars(kv).items()} if ours else None
+            try:
+                if kv is not None:
+                    audio = rt.decode(codes, out_len, kv)
+                elif self.use_graphs:
+                    rt.prepare(frames * (2 if rt.bottleneck else 1))
+                    audio = self._graph(("dec", tuple(codes.shape), out_len),
+                                        lambda c: rt.decode(c, out_len), (codes,))
+                else:
+                    rt.prepare(frames * (2 if rt.bottleneck else 1))
+                    audio = rt.decode(codes, out_len)
+            finally:
+                if check.bad():
+                    if saved is not None:
+                        vars(kv).update(saved)
+                    raise IndexError("audio code out of range of the codebook")
         if not return_dict:
             return audio, kv
         return MimiDecoderOutput(audio, kv)

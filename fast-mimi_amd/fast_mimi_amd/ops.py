@@ -50,6 +50,7 @@ SPECS = {
     "fm_rvq_prepare_screen": "in:embeds in:norms i:entries i:dim i:count out:planes out:info",
     "fm_rvq_encode_split_screened": "in:x i:ld_x i:rows i:rows_per_batch i:dim i:entries i:n_semantic i:n_acoustic in:embeds in:norms in:planes in:info out:codes i:batch_stride",
     "fm_rvq_encode_split_noalloc": "in:x i:ld_x i:rows i:rows_per_batch i:dim i:entries i:n_semantic i:n_acoustic in:embeds in:embeds_t in:norms out:codes i:batch_stride",
+    "fm_codes_check": "in:codes i:count i:entries out:flag",
     "fm_rvq_decode": "in:codes i:batch i:num_codebooks i:frames i:num_semantic in:embeds i:entries i:dim out:out",
     "fm_upsample_depthwise": "in:x i:batch i:length i:channels in:weight i:kernel i:stride out:y",
     "fm_stream_append": "in:context in:x i:batch i:pad i:length i:channels i:replicate out:buf out:next",

@@ -437,6 +437,15 @@ int fm_rvq_encode_split_screened(const float* x, int ld_x, int rows, int rows_pe
                                  int64_t* codes, int batch_stride, hipStream_t stream);
 
 /*
+ * Range check of decode input: *flag = 1 if any of `count` codes lies outside
+ * [0, entries), else left as it is.  flag may be pinned host memory (the store
+ * has system scope; read it after an event recorded behind the call).
+ * Replaces the bounds check of the reference's embedding gather
+ * (model.py:2570-2627), which raises IndexError.
+ */
+int fm_codes_check(const int64_t* codes, size_t count, int entries, int* flag, hipStream_t stream);
+
+/*
  * Split-RVQ decode gather-sum: out[(b*frames + t)][0:dim] = 0 + E_0[c_0]
  * (the num_semantic first codebooks summed left to right),
  * out[...][dim:2*dim] = 0 + E_s[c_s] + E_{s+1}[c_{s+1}] + ... left to right.
