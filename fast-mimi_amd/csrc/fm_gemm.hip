@@ -1126,7 +1126,11 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restr
 // lane's accumulator of the neighbouring 32-column tile (wave tiles start
 // on 64-column boundaries).
 enum TileRope { ROPE_NEVER, ROPE_FLAG, ROPE_ALWAYS };  // whether the tile rotates: p.flags says, or the kernel
-template <int BM, int FM, int FN, TileRope ROT>
+// NT: streaming stores, for an output larger than the last-level cache (256
+// MB): nothing of it is read back from there, and the input stays cached
+// (16 clips' stride-4 upsampling, 983 MB written: 571 -> 553 us; stride-5,
+// 491 MB: 442 -> 421 us).
+template <int BM, int FM, int FN, TileRope ROT, bool NT = false>
 FM_DEVICE void tile_epilogue(const GemmArgs& p, floatx16 (&acc)[FM][FN], long M, long m0, int n0, int wm0,
                              int wn0, int lane) {
   const int lcol = lane & 31;
@@ -1196,7 +1200,10 @@ FM_DEVICE void tile_epilogue(const GemmArgs& p, floatx16 (&acc)[FM][FN], long M,
             const bool ok = m < M && n_ok && t < p.y_rows;
             fm_buf_store1(v, rc, ok ? ((b * p.y_rows + t - crop0) * p.N + n) * 4 : INT_MIN, 0);
           } else {
-            fm_buf_store1(v, ry, voff, soff(r));
+            if constexpr (NT)
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), ry, voff, soff(r), 2);
+            else
+              fm_buf_store1(v, ry, voff, soff(r));
           }
         }
       }
@@ -1501,7 +1508,7 @@ __global__ __launch_bounds__(256) void split_weights_h3_kernel(const float* __re
 // each wave reads, scales and splits the A fragments of its rows and runs the
 // three products a1b0, a0b1, a0b0 per fragment pair.  WPE: waves per SIMD the
 // registers are held to.
-template <int BM, int BN, int WM, int WN, int KS, int WPE, bool ELU, bool ROPE = false>
+template <int BM, int BN, int WM, int WN, int KS, int WPE, bool ELU, bool ROPE = false, bool NT = false>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WPE)))
 void gemm_h3_kernel(GemmArgs p, const _Float16* __restrict__ wh) {
   constexpr int NW = WM * WN, BK = 16 * KS;
@@ -1699,7 +1706,7 @@ void gemm_h3_kernel(GemmArgs p, const _Float16* __restrict__ wh) {
 #pragma unroll
     for (int i = 0; i < FM; ++i) scale_rows(i, e, acc[i][j]);
   }
-  tile_epilogue<BM, FM, FN, ROPE ? ROPE_ALWAYS : ROPE_NEVER>(p, acc, M, m0, n0, wm0, wn0, lane);
+  tile_epilogue<BM, FM, FN, ROPE ? ROPE_ALWAYS : ROPE_NEVER, NT>(p, acc, M, m0, n0, wm0, wn0, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1845,6 +1852,7 @@ constexpr TileCfg kH3 = {128, 128, 1, 32, 24, 0};       // 16-deep k-tiles, 33 K
 constexpr TileCfg kH3K32 = {128, 128, 1, 32, 25, 0};    // 32-deep, 65 KB: two blocks per CU
 constexpr TileCfg kH3Small = {64, 128, 1, 32, 26, 0};   // 32-deep, 49 KB: three blocks per CU
 constexpr TileCfg kH3Tiny = {64, 64, 1, 64, 27, 0};     // 64-deep, 65 KB: two blocks per CU
+constexpr TileCfg kH3Tiny32 = {64, 64, 1, 32, 28, 0};   // 32-deep, 33 KB: four blocks per CU
 // 64x128 runs one block per CU: 64-deep k-tiles (96 KB ring) halve its barriers.
 constexpr TileCfg kDl64 = {64, 128, 1, 64, 15, 0};
 
@@ -1908,6 +1916,7 @@ const char* kernel_name(int id, bool elu) {
     case 25: return elu ? "gemm_h3_kernel<128,128,4,2,2,4,true>" : "gemm_h3_kernel<128,128,4,2,2,4,false>";
     case 26: return elu ? "gemm_h3_kernel<64,128,2,2,2,3,true>" : "gemm_h3_kernel<64,128,2,2,2,3,false>";
     case 27: return elu ? "gemm_h3_kernel<64,64,2,2,4,2,true>" : "gemm_h3_kernel<64,64,2,2,4,2,false>";
+    case 28: return elu ? "gemm_h3_kernel<64,64,2,2,2,4,true>" : "gemm_h3_kernel<64,64,2,2,2,4,false>";
     case 7: return "gemm_mid_kernel<64,64,1>";
     case 8: return "gemm_mid_kernel<32,32,4>";
     default: return "gemm_generic_kernel";
@@ -1925,7 +1934,7 @@ void record_plan(int id, bool elu, long tiles, int splits) {
 // they leave CUs idle.  Measured on the decoder's shapes (us, best bf16x6 or
 // FP32 tile -> h3): 7500-15000 tiles, K = 256-512: 778 -> 567, 604 -> 432;
 // 1500-3000, K = 1024: 457 -> 318; 470 tiles, K = 512: 45 -> 35; 4000-row
-// qkv 38 -> 32, fc1 47 -> 35, fc2 53 -> 43, o 25 -> 22; 6240 x 256 x 256:
+// qkv 38 -> 32, fc1 47 -> 35, fc2 53 -> 43, o 25 -> 16; 6240 x 256 x 256:
 // 13.8 -> 10.6; 1248 x 640 x 512: 30 -> 13; 26 x 4096 x 2048: 19 -> 15;
 // 16 x 1536 x 1024: 15.7 -> 10.
 void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tiles, int& splits) {
@@ -1946,13 +1955,16 @@ void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tile
     // 129, 128 x 4 (fc2 at 4000 rows) 43 against 78.
     cfg = kH3K32;
     if (p.K >= 1024) splits = fewest(t128, 8, 256);
-  } else if (!k64 || (p.K < 1024 && M >= 2048 && p.N >= 512)) {
-    // The 512-column projections at 2500-4000 rows (20.6-21.6 us; 128x128
-    // tiles 21.3-22.2).
+  } else if (!k64) {
     cfg = kH3Small;
   } else {
-    cfg = kH3Tiny;
-    if (p.K >= 512) splits = fewest(tile_count(M, p.N, kH3Tiny), 16, 128);
+    // 64x64 tiles: the 512-column projections at 2500 / 4000 rows 15.5 / 16.1
+    // us (64x128 18.4 / 19.1, 128x128 21.3 / 22.2), 64-deep while they fit
+    // two per CU (1100-row qkv 15.9 us, 32-deep 17.0), else 32-deep (1100-row
+    // fc1, 576 tiles: 20.7 us, 64x128 23.4).
+    const long t64 = tile_count(M, p.N, kH3Tiny);
+    cfg = t64 > 512 ? kH3Tiny32 : kH3Tiny;
+    if (p.K >= 512) splits = fewest(t64, 16, 128);
   }
   tiles = tile_count(M, p.N, cfg);
 }
@@ -2236,10 +2248,15 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
   else                                                                                                       \
     hipLaunchKernelGGL((gemm_h3_kernel<BM_, BN_, WM_, WN_, KS_, WPE_, false>), grid, dim3(64 * WM_ * WN_),   \
                        0, s, p, wh)
-    case 24: FM_H3(128, 128, 2, 2, 1, 4, true); break;
+    case 24:
+      if (M * p.N * 4 > (256L << 20) && !p.partial && !(p.flags & (FM_ELU_IN | FM_EPI_ROPE)))
+        hipLaunchKernelGGL((gemm_h3_kernel<128, 128, 2, 2, 1, 4, false, false, true>), grid, dim3(256), 0, s, p, wh);
+      else FM_H3(128, 128, 2, 2, 1, 4, true);
+      break;
     case 25: FM_H3(128, 128, 4, 2, 2, 4, true); break;
     case 26: FM_H3(64, 128, 2, 2, 2, 3, true); break;
     case 27: FM_H3(64, 64, 2, 2, 4, 2, false); break;
+    case 28: FM_H3(64, 64, 2, 2, 2, 4, false); break;
 #undef FM_H3
     case 7: hipLaunchKernelGGL((gemm_mid_kernel<64, 64, 1>), grid, dim3(NTHREADS), 0, s, p); break;
     case 8: hipLaunchKernelGGL((gemm_mid_kernel<32, 32, 4>), grid, dim3(NTHREADS), 0, s, p); break;
