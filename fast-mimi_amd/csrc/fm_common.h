@@ -132,6 +132,12 @@ FM_DEVICE floatx16 fm_mfma32_f16(halfx8 a, halfx8 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
+// One v_mfma_f32_16x16x32_f16: lane l supplies row / column l % 16, k = 8 (l /
+// 16) .. + 7; its four results are rows 4 (l / 16) .. + 3 of column l % 16.
+FM_DEVICE floatx4 fm_mfma16_f16(halfx8 a, halfx8 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
 FM_DEVICE void split2(floatx4 v, float sc, halfx4& h0, halfx4& h1) {
   typedef _Float16 halfx2_t __attribute__((ext_vector_type(2)));
   typedef float floatx2_t __attribute__((ext_vector_type(2)));
@@ -158,6 +164,25 @@ FM_DEVICE void split2(floatx4 lo, floatx4 hi, float sc, halfx8& h0, halfx8& h1) 
 FM_DEVICE int h3_exp_for(float m, int to) {
   const int f = (int)(__builtin_bit_cast(unsigned, m) >> 23) & 255;
   return m > 0.0f ? min(max(127 + to + 127 - f, 1), 253) - 127 : 0;
+}
+
+// A 16-row wave fragment of the few-row h3 kernels: S 32-deep k steps, lane (row
+// l % 16, k = 8 (l / 16) .. + 7 of each step).  Returns the exponent that puts
+// the row's largest magnitude over those steps into [2^13, 2^14) (every lane of
+// a row agrees; non-finite values do not count).
+template <int S>
+FM_DEVICE int h3_row_exp16(const floatx4 (&a)[S][2]) {
+  float m = 0.0f;
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float u = fabsf(a[s][0][e]), v = fabsf(a[s][1][e]);
+      m = fmaxf(m, fmaxf(u < INFINITY ? u : 0.0f, v < INFINITY ? v : 0.0f));
+    }
+  m = fmaxf(m, __shfl_xor(m, 16, 64));
+  m = fmaxf(m, __shfl_xor(m, 32, 64));
+  return h3_exp_for(m, 13);
 }
 
 static inline int fm_ceil_div(long a, long b) { return (int)((a + b - 1) / b); }

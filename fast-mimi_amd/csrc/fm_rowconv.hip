@@ -34,7 +34,12 @@ struct RowConvArgs {
   int L, c_in, stride, pad_l, replicate, rows_per_batch, rows, N, bias_len, flags;
 };
 
-template <int K, int BN, bool X6, int MT>
+// H3: the layer's fp16 planes and three v_mfma_f32_16x16x32_f16 products per
+// fragment pair.  A wave takes its k-range in chunks of at most seven steps,
+// reads a chunk's A fragments of its rows first (ELU applied), scales each row
+// by a power of two from them, and adds the chunk's products back at the
+// caller's scale.
+template <int K, int BN, bool X6, int MT, bool H3 = false>
 __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
   // MT 16-row MFMA tiles per block (bf16x6 only): each weight fragment a wave
   // loads serves all of them, so the weights cross L2 once per 16 * MT rows.
@@ -77,7 +82,83 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[mt][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  if constexpr (X6) {
+  if constexpr (H3) {
+    constexpr int KS = KW / 32, CS = KS <= 7 ? KS : KS / 2, NCH = KS / CS, NU = 2 * KS;
+    static_assert(KW % 32 == 0 && CS * NCH == KS && CS <= 7, "whole chunks");
+    constexpr int R = NU < 6 ? NU : 6;  // weight units (step, plane) in flight
+    const _Float16* wh = reinterpret_cast<const _Float16*>(p.w + (long)p.N * K + 3L * p.N * K / 2);
+    const long PL = (long)p.N * K;
+    const _Float16* wbh = wh + ((long)((kw0 >> 4) + (g >> 1)) * p.N + n0 + li) * 16 + 8 * (g & 1);
+    halfx8 bu[R][NT];
+    auto load_unit = [&](int buf, int u) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        bu[buf][j] =
+            *reinterpret_cast<const halfx8*>(wbh + (u & 1) * PL + (long)(u >> 1) * 2 * p.N * 16 + j * 256);
+    };
+#pragma unroll
+    for (int u = 0; u < R; ++u) load_unit(u, u);
+#pragma unroll
+    for (int ch = 0; ch < NCH; ++ch) {
+      floatx4 ah[MT][CS][2];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int st = 0; st < CS; ++st) {
+          const float* src = a_src(mt, kw0 + 32 * (ch * CS + st), 8 * g);
+          ah[mt][st][0] = *reinterpret_cast<const floatx4*>(src);
+          ah[mt][st][1] = *reinterpret_cast<const floatx4*>(src + 4);
+        }
+      if (elu_in) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int st = 0; st < CS; ++st)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              ah[mt][st][0][e] = fm_elu(ah[mt][st][0][e]), ah[mt][st][1][e] = fm_elu(ah[mt][st][1][e]);
+      }
+      int se[MT];
+      float sc[MT];
+      floatx4 part[MT][NT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        se[mt] = h3_row_exp16(ah[mt]);
+        sc[mt] = __builtin_amdgcn_ldexpf(1.0f, se[mt]);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) part[mt][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int st = 0; st < CS; ++st) {
+        const int u = 2 * (ch * CS + st);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          halfx8 p0v, p1v;
+          split2(ah[mt][st][0], ah[mt][st][1], sc[mt], p0v, p1v);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) part[mt][j] = fm_mfma16_f16(p1v, bu[u % R][j], part[mt][j]);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) part[mt][j] = fm_mfma16_f16(p0v, bu[u % R][j], part[mt][j]);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) part[mt][j] = fm_mfma16_f16(p0v, bu[(u + 1) % R][j], part[mt][j]);
+        }
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl)
+          if (u + pl + R < NU) load_unit((u + pl) % R, u + pl + R);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int e = -__shfl(se[mt], 4 * g + r, 64);
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            acc[mt][j][r] = __fadd_rn(acc[mt][j][r], __builtin_amdgcn_ldexpf(part[mt][j][r], e));
+        }
+    }
+  } else if constexpr (X6) {
     // bf16x6: W^T's planes [3][K/16][N][16] after the FP32 weight; 32-deep k
     // steps on v_mfma_f32_16x16x32_bf16, lane group g covering k = 8g .. 8g+7
     // of A and B.  Units (step, plane) stream through a ring of R weight
@@ -216,6 +297,9 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
     float v = red[er * PR + ec + c];
 #pragma unroll
     for (int q = 1; q < NWV; ++q) v = __fadd_rn(v, red[(q * BM + er) * PR + ec + c]);
+    if constexpr (H3)
+      v = __builtin_amdgcn_ldexpf(
+          v, -reinterpret_cast<const int*>(p.w + (long)p.N * K + 5L * p.N * K / 2)[n0 + ec + c]);
     if (p.bias) v = __fadd_rn(v, p.bias[(n0 + ec + c) % p.bias_len]);
     if (p.flags & FM_EPI_RES_ADD) v = __fadd_rn(p.res[m * p.N + n0 + ec + c], v);
     if (p.flags & FM_EPI_ELU) v = fm_elu(v);
@@ -245,7 +329,8 @@ int fm_conv1d_rows(const float* x, int batch, int length, int in_channels, const
       kernel < stride || (pad_mode != 0 && pad_mode != 1) || (bias && bias_len <= 0) ||
       (flags & FM_EPI_RES_ADD && !residual))
     return FM_BAD_ARGUMENT;
-  if (flags & ~(FM_ELU_IN | FM_EPI_ELU | FM_EPI_RES_ADD | FM_WEIGHTS_X6)) return FM_UNSUPPORTED;
+  if (flags & ~(FM_ELU_IN | FM_EPI_ELU | FM_EPI_RES_ADD | FM_WEIGHTS_X6 | FM_WEIGHTS_H3)) return FM_UNSUPPORTED;
+  if ((flags & FM_WEIGHTS_H3) && !(flags & FM_WEIGHTS_X6)) return FM_UNSUPPORTED;
   if (!fm_conv1d_rows_supported(in_channels, out_channels, kernel, flags)) return FM_UNSUPPORTED;
   const int rows_per_batch = (length + stride - 1) / stride;
   const long rows = (long)batch * rows_per_batch;
@@ -274,6 +359,20 @@ int fm_conv1d_rows(const float* x, int batch, int length, int in_channels, const
   // 21.1 us at C2; with fewer blocks the CUs left idle cost more than the
   // halved weight reads save).
   const bool two = !wide && (long)(out_channels / 32) * row_blocks >= 512;
+  // The decoder's depths on fp16 planes, in the same blocks.
+  if ((flags & FM_WEIGHTS_H3) && (K == 256 || K == 1536 || K == 3584)) {
+#define FM_ROWCONVH3(KK, BN, MT, G) hipLaunchKernelGGL((row16_conv_kernel<KK, BN, true, MT, true>), G, dim3(512), 0, stream, p)
+#define FM_ROWCONVH3K(KK)                      \
+  if (two) FM_ROWCONVH3(KK, 32, 2, grid32r);   \
+  else if (wide) FM_ROWCONVH3(KK, 64, 2, grid64); \
+  else FM_ROWCONVH3(KK, 32, 1, grid)
+    if (K == 256) { FM_ROWCONVH3K(256); }
+    else if (K == 1536) { FM_ROWCONVH3K(1536); }
+    else { FM_ROWCONVH3K(3584); }
+#undef FM_ROWCONVH3K
+#undef FM_ROWCONVH3
+    return (int)hipGetLastError();
+  }
   if ((flags & FM_WEIGHTS_X6) && two) {
     if (K == 256) FM_ROWCONV32R(256);
     else if (K == 1536) FM_ROWCONV32R(1536);

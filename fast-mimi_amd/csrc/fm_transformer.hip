@@ -1249,7 +1249,13 @@ __global__ __launch_bounds__(512) void row_stream_linear_kernel(
 // per channel (h[t-1] = 0 at a sequence start), computed in the epilogue: a
 // block's 16 rows are t0 - 1 .. t0 + 14 (the first one only feeds row t0's
 // taps), and y is the upsampled [rows * 2][N]; up_w is [N][4].
-template <int K, int BN, bool X6 = false, bool UPS = false>
+//
+// H3 (with X6's layouts): the weight's fp16 planes ([2][K/16][N][16] and N row
+// exponents, fm_split_weights_h3) and three v_mfma_f32_16x16x32_f16 products
+// per fragment pair.  A wave reads its whole k-range of the 16 rows first, takes
+// a power of two per row from it, and its partial tile returns to the caller's
+// scale as it goes to LDS; the column exponents follow after the sum.
+template <int K, int BN, bool X6 = false, bool UPS = false, bool H3 = false>
 __global__ __launch_bounds__(512) void row16_linear_kernel(
     const float* __restrict__ x, int rows, const float* __restrict__ gamma,
     const float* __restrict__ beta, float eps, const float* __restrict__ wp, int N, int flags,
@@ -1329,10 +1335,12 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
   const bool rope = BN == 64 && cos_t && n0 < rope_cols;
   const bool res_scale = flags & FM_EPI_RES_SCALE;
   float e_res[OPT], e_scale[OPT], e_cos[OPT], e_sin[OPT];
+  int e_col[OPT];  // H3: the columns' weight exponents
   auto fetch_epilogue = [&]() {
 #pragma unroll
     for (int c = 0; c < OPT; ++c) {
       const int n = n0 + ec + c;
+      if constexpr (H3) e_col[c] = reinterpret_cast<const int*>(wp + (long)N * K)[n];
       e_res[c] = res_scale ? res[mc * N + n] : 0.0f;
       e_scale[c] = res_scale ? scale[n] : 0.0f;
       e_cos[c] = rope ? cos_t[(long)tpos * 64 + ec + c] : 0.0f;
@@ -1356,6 +1364,7 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
       float v = red[er * PR + ec + c];
 #pragma unroll
       for (int q = 1; q < NWV; ++q) v = __fadd_rn(v, red[(q * BM + er) * PR + ec + c]);
+      if constexpr (H3) v = __builtin_amdgcn_ldexpf(v, -e_col[c]);
       out[c] = v;
     }
     if (rope || UPS) {
@@ -1407,7 +1416,68 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
 #pragma unroll
   for (int j = 0; j < NT; ++j) acc[j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  if constexpr (X6) {
+  if constexpr (H3) {
+    constexpr int KS = KW / 32, NU = 2 * KS;  // units: (k step, weight plane)
+    constexpr int R = NU < 8 ? NU : 8;        // weight units in flight
+    const _Float16* wh = reinterpret_cast<const _Float16*>(wp);
+    const long PL = (long)N * K;
+    const _Float16* wbh = wh + ((long)((kw0 >> 4) + (g >> 1)) * N + n0 + li) * 16 + 8 * (g & 1);
+    halfx8 bu[R][NT];
+    floatx4 ah[KS][2];
+    auto load_unit = [&](int buf, int u) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        bu[buf][j] =
+            *reinterpret_cast<const halfx8*>(wbh + (u & 1) * PL + (long)(u >> 1) * 2 * N * 16 + j * 256);
+    };
+    if (!STAGE) {
+      const float* xh = x + min(m0 + li, (long)rows - 1) * K + kw0 + 8 * g;
+#pragma unroll
+      for (int st = 0; st < KS; ++st)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) ah[st][h] = *reinterpret_cast<const floatx4*>(xh + 32 * st + 4 * h);
+    } else {
+      stage_rows();
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u) load_unit(u, u);
+    if (STAGE) {
+      __syncthreads();
+#pragma unroll
+      for (int st = 0; st < KS; ++st)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          ah[st][h] = *reinterpret_cast<const floatx4*>(As + li * PA + kw0 + 32 * st + 8 * g + 4 * h);
+    }
+    fetch_epilogue();
+    const int se = h3_row_exp16(ah);
+    const float sc = __builtin_amdgcn_ldexpf(1.0f, se);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int st = 0; st < KS; ++st) {
+      halfx8 p0, p1;
+      split2(ah[st][0], ah[st][1], sc, p0, p1);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = fm_mfma16_f16(p1, bu[2 * st % R][j], acc[j]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = fm_mfma16_f16(p0, bu[2 * st % R][j], acc[j]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = fm_mfma16_f16(p0, bu[(2 * st + 1) % R][j], acc[j]);
+#pragma unroll
+      for (int pl = 0; pl < 2; ++pl)
+        if (2 * st + pl + R < NU) load_unit((2 * st + pl) % R, 2 * st + pl + R);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int e = -__shfl(se, 4 * g + r, 64);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j][r] = __builtin_amdgcn_ldexpf(acc[j][r], e);
+    }
+    reduce_and_store(acc);
+    return;
+  }
+  if constexpr (X6 && !H3) {
     constexpr int KS = KW / 32, NU = 3 * KS;  // units: (k step, weight plane)
     // Weight units in flight: a ring of R (all of K = 512 at 32-column tiles,
     // four units of the 64-column tiles, six of the streamed K = 2048).
@@ -1599,6 +1669,18 @@ int fm_row_linear(const float* x, int rows, int in_features, const float* ln_gam
     const float* planes = weight + (long)out_features * in_features;
     const dim3 g64(out_features / 64, (rows + 15) / 16), g32(out_features / 32, (rows + 15) / 16);
     const bool wide = rope_cos || (long)(out_features / 32) * ((rows + 15) / 16) > 512;
+    if (flags & FM_WEIGHTS_H3) {
+      const float* h3 = planes + 3L * out_features * in_features / 2;
+#define FM_R16H3(KK, BN, G)                                                                                       \
+  hipLaunchKernelGGL((row16_linear_kernel<KK, BN, true, false, true>), G, dim3(512), 0, stream, x, rows, ln_gamma, \
+                     ln_beta, ln_eps, h3, out_features, flags, residual, scale, rope_cos, rope_sin, rope_cols,    \
+                     rows_per_seq, y)
+      if (in_features == 2048) FM_R16H3(2048, 32, g32);
+      else if (wide) FM_R16H3(512, 64, g64);
+      else FM_R16H3(512, 32, g32);
+#undef FM_R16H3
+      return (int)hipGetLastError();
+    }
 #define FM_R16X6(KK, BN, G)                                                                           \
   hipLaunchKernelGGL((row16_linear_kernel<KK, BN, true>), G, dim3(512), 0, stream, x, rows, ln_gamma, \
                      ln_beta, ln_eps, planes, out_features, flags, residual, scale, rope_cos,        \

@@ -331,7 +331,7 @@ class MimiRuntime:
                 and not flags & ~(nat.ELU_IN | nat.EPI_ELU | nat.EPI_RES_ADD)):
             self._call("fm_conv1d_rows", x, B, L, layer.c_in, layer.wr, layer.b, layer.c_out,
                        layer.c_out, layer.k, layer.stride, layer.replicate,
-                       flags | (layer.flags & nat.WEIGHTS_X6 if layer.wr is layer.w else 0), residual, y)
+                       flags | (layer.flags if layer.wr is layer.w else 0), residual, y)
             return y, rows
         self._call("fm_conv1d", x, B, L, layer.c_in, layer.w, layer.b,
                  layer.c_out, layer.k, layer.stride, layer.replicate, flags | layer.flags, residual,
@@ -381,14 +381,16 @@ class MimiRuntime:
         g, b = (ln[0], ln[1]) if ln is not None else (None, None)
         cos, sin, rope_cols, per_seq = rope if rope is not None else (None, None, 0, 1)
         few = rows <= _ROW16_MAX_ROWS
-        # bf16x6 where it measured faster at 250 rows: the wide 512-deep
-        # projections (qkv 7.5 vs 9.4 us, fc1 7.7 vs 9.6 us); the output
-        # projection (3.5 vs 3.4 us) and the streamed fc2 (8.1 vs 8.1 us)
-        # keep the FP32 fragment-packed kernel.
-        wx = self._x6.get(w.data_ptr()) if few and k == 512 and n >= 1024 else None
+        # 16-bit matrix cores where they measured faster at 250 rows: the fp16
+        # planes of the decoder's projections always; bf16x6 for the wide
+        # 512-deep ones (qkv 7.5 vs 9.4 us, fc1 7.7 vs 9.6 us), while the
+        # output projection (3.5 vs 3.4 us) and the streamed fc2 (8.1 vs 8.1
+        # us) keep the FP32 fragment-packed kernel.
+        h3 = w.data_ptr() in self._h3
+        wx = self._x6.get(w.data_ptr()) if few and (h3 or (k == 512 and n >= 1024)) else None
         packed = self._packed.get(w.data_ptr()) if few else None
-        if wx is not None:  # 16-row blocks on the bf16 matrix cores (bf16x6)
-            name, wp, flags = "fm_row_linear", wx, flags | nat.WEIGHTS_X6
+        if wx is not None:  # 16-row blocks on the 16-bit matrix cores
+            name, wp, flags = "fm_row_linear", wx, flags | nat.WEIGHTS_X6 | (nat.WEIGHTS_H3 if h3 else 0)
         elif packed is not None:
             name, wp = "fm_row_linear_packed", packed
         else:

@@ -271,3 +271,80 @@ def test_resblock64_conv(B, L, y_len):
         errs.append((y.cpu().double()[:, None] - want).norm())
         assert (y.cpu().double()[:, None] - want).abs().max() <= 2e-5 * want.abs().max()
     assert errs[0] <= 1.1 * errs[1] + 1e-7 * want.norm()
+
+
+@pytest.mark.parametrize("rows,k,n,ln,epi", [(250, 512, 1536, True, "rope"), (1, 512, 2048, True, "gelu"), (33, 512, 512, False, "res"),
+                                             (512, 512, 2048, True, "gelu"), (17, 2048, 512, False, "res"), (250, 2048, 512, False, "res"),
+                                             (16, 512, 64, False, "plain")])
+@pytest.mark.parametrize("kind", ["plain", "scales"])
+def test_row_linear(rows, k, n, ln, epi, kind):
+    """The few-row projections on fp16 planes, each epilogue; rows of any
+    magnitude side by side and k-ranges (one per wave) of any magnitude within a
+    row, zero rows and rows with an inf."""
+    g = torch.Generator().manual_seed(rows + k + n)
+    x = torch.randn(rows, k, generator=g)
+    if kind == "scales" and not ln:
+        x *= 10.0 ** (40 * torch.rand(rows, 1, generator=g) - 20)
+        x *= torch.exp2(torch.randint(-30, 30, (1, 8), generator=g).repeat_interleave(k // 8, 1).float())
+        x[2::5] = 0
+    x = x.to(DEV)
+    w, _ = with_planes((torch.randn(n, k, generator=g) / math.sqrt(k)).to(DEV))
+    gamma, beta = (1 + 0.1 * torch.randn(k, generator=g)).to(DEV), (0.1 * torch.randn(k, generator=g)).to(DEV)
+    res, scale = torch.randn(rows, n, generator=g).to(DEV), torch.randn(n, generator=g).to(DEV)
+    cos, sin = (t.to(DEV) for t in rope_tables(MimiConfig(), max(rows // 2, 1)))
+    flags = FLAGS | {"gelu": nat.EPI_GELU, "res": nat.EPI_RES_SCALE}.get(epi, 0)
+    rope_cols, per_seq = (1024, max(rows // 2, 1)) if epi == "rope" else (0, 1)
+    y = torch.full((rows, n), float("nan"), device=DEV)
+    nat.call("fm_row_linear", x.data_ptr(), rows, k, gamma.data_ptr() if ln else None, beta.data_ptr() if ln else None,
+             1e-5, w.data_ptr(), n, flags, res.data_ptr() if epi == "res" else None,
+             scale.data_ptr() if epi == "res" else None, cos.data_ptr() if rope_cols else None,
+             sin.data_ptr() if rope_cols else None, rope_cols, per_seq, y.data_ptr(), stream())
+    torch.cuda.synchronize()
+    a = x.double()
+    if ln:
+        a = F.layer_norm(a, (k,), gamma.double(), beta.double(), 1e-5)
+    want, absref = a @ w.double().t(), a.abs() @ w.double().abs().t()
+    if epi == "gelu":
+        want = F.gelu(want)
+    elif epi == "res":
+        want, absref = res.double() + scale.double() * want, res.double().abs() + scale.double().abs() * absref
+    elif epi == "rope":
+        pos = torch.arange(rows, device=DEV) % per_seq
+        c, s = (t.double()[pos].repeat(1, rope_cols // 64) for t in (cos, sin))
+        q = want[:, :rope_cols].view(rows, -1, 64)
+        half = torch.cat((-q[..., 32:], q[..., :32]), -1).reshape(rows, -1)
+        h2 = absref[:, :rope_cols].view(rows, -1, 64)
+        want[:, :rope_cols] = want[:, :rope_cols] * c + half * s
+        absref[:, :rope_cols] += torch.cat((h2[..., 32:], h2[..., :32]), -1).reshape(rows, -1)
+    close_dot(y, want, absref)
+
+
+@pytest.mark.parametrize("B,cin,cout,k,L,flags", [
+    (1, 512, 1024, 7, 2, nat.EPI_ELU), (1, 512, 1024, 7, 250, nat.EPI_ELU), (2, 512, 1024, 7, 131, 0), (1, 512, 1024, 7, 265, 0),
+    (1, 512, 256, 3, 208, nat.ELU_IN | nat.EPI_ELU), (1, 512, 256, 3, 2000, nat.ELU_IN | nat.EPI_ELU),
+    (1, 256, 512, 1, 16, nat.EPI_RES_ADD | nat.EPI_ELU), (3, 256, 512, 1, 701, nat.EPI_RES_ADD)])
+def test_conv1d_rows(B, cin, cout, k, L, flags):
+    """The few-row convolutions on fp16 planes: one- and two-tile blocks, batch
+    seams, ELU on load, residuals; quiet rows between loud ones."""
+    g = torch.Generator().manual_seed(L + cin)
+    x = torch.randn(B, cin, L, generator=g) * 10.0 ** (torch.arange(L) % 4 * 3 - 6)
+    w, b = torch.randn(cout, cin, k, generator=g) / math.sqrt(cin * k), torch.randn(cout, generator=g)
+    res = torch.randn(B, cout, L, generator=g)
+    layer = _Conv(w.to(DEV), b.to(DEV))
+    wp, _ = with_planes(layer.w)
+    xd, rd = (t.transpose(1, 2).contiguous().to(DEV) for t in (x, res))
+    y = torch.full((B, L, cout), float("nan"), device=DEV)
+    nat.call("fm_conv1d_rows", xd.data_ptr(), B, L, cin, wp.data_ptr(), layer.b.data_ptr(), cout, cout, k, 1, 0,
+             flags | FLAGS, rd.data_ptr(), y.data_ptr(), stream())
+    torch.cuda.synchronize()
+    xin = F.elu(x.double()) if flags & nat.ELU_IN else x.double()
+    want = causal_conv1d(xin, w.double(), b.double())
+    absref = causal_conv1d(xin.abs(), w.double().abs(), b.double().abs())
+    if flags & nat.EPI_RES_ADD:
+        want, absref = want + res, absref + res.abs()
+    if flags & nat.EPI_ELU:
+        want = F.elu(want)
+    close_dot(y.cpu().transpose(1, 2), want, absref)
+    with pytest.raises(nat.NativeError, match="unsupported"):
+        nat.call("fm_conv1d_rows", xd.data_ptr(), B, L, cin, wp.data_ptr(), layer.b.data_ptr(), cout, cout, k, 1, 0,
+                 nat.WEIGHTS_H3, rd.data_ptr(), y.data_ptr(), stream())
