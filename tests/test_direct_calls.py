@@ -4,6 +4,7 @@ calls, and a streamed RoPE table is a slice of a longer one (CPU only)."""
 from __future__ import annotations
 
 import torch
+from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from fast_mimi_amd import MimiConfig, ops
@@ -17,6 +18,10 @@ def test_observers_keep_the_operator_path():
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
             return func(*args, **(kwargs or {}))
 
+    class FunctionMode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
     def look(x):
         seen.append(ops._observed())
         return x * 2
@@ -25,13 +30,15 @@ def test_observers_keep_the_operator_path():
     assert not ops._observed()
     with Mode():
         look(x)
+    with FunctionMode():
+        look(x)
     torch.vmap(look)(x)
     torch.func.jvp(look, (x,), (x,))
     torch.func.grad(lambda v: look(v).sum())(x)
     torch.jit.trace(look, (x,), check_trace=False)
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
         look(x)
-    assert len(seen) >= 6 and all(seen)
+    assert len(seen) >= 7 and all(seen)
     assert not ops._observed()
 
 
