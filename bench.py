@@ -107,13 +107,17 @@ def dominant_kernel(model: MimiModel, name: str, batch: int, samples: int, nq: i
     ms = start.elapsed_time(stop) / iters
     del graph
     achieved = flops / (ms * 1e-3) / 1e12
+    # The fp16 tiles take three products per operand pair, the bf16 ones six;
+    # both matrix-core types have one dense peak.
+    products, kind = (3, "fp16") if "gemm_h3" in plan else (6, "bf16")
     return {"bound": "mfma", "kernel": f"{plan} ({name}: {row[1]} rows={row[3]} K={row[4]} N={row[5]})",
             "flops_per_launch": flops, "avg_launch_ms": ms, "achieved": round(achieved, 3),
             "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP32_TFLOPS, 4),
             "traffic": None,
-            "note": ("FP32 contraction run as six bf16 MFMA products per operand pair (FP32-accurate); "
+            "note": (f"FP32 contraction run as {products} {kind} MFMA products per operand pair (FP32-accurate); "
                      "achieved counts the algorithmic FP32 FLOPs against the FP32 MFMA peak"),
-            "bf16_mfma_pipe_frac": round(6 * achieved / PEAK_BF16_TFLOPS, 4)}
+            "mfma_products": products,
+            "16bit_mfma_pipe_frac": round(products * achieved / PEAK_BF16_TFLOPS, 4)}
 
 
 def graph_ms(fn, iters: int) -> float:
@@ -156,8 +160,13 @@ def rvq_only(model: MimiModel, audio: torch.Tensor, nq: int, iters: int = 10) ->
     wsb = nat.library().fm_rvq_split_workspace_bytes(M, vq, E)
     ws = torch.empty((wsb + 3) // 4, device=audio.device)
     q = torch.empty((M, 2 * vq), device=audio.device)
+    screened = rt.screen is not None and nat.library().fm_rvq_screen_supported(M, vq, E)
 
-    def enc():
+    def enc():  # as the runtime chooses for this many rows
+        if screened:
+            ops.call("fm_rvq_encode_split_screened", proj, 2 * vq, M, T, vq, E, n_sem, nq - n_sem,
+                     rt.embeds, rt.norms, rt.screen, rt.screen_info, codes, nq * T)
+            return
         ops.call("fm_rvq_encode_split", proj, 2 * vq, M, T, vq, E, n_sem, nq - n_sem,
                  rt.embeds, rt.embeds_t, rt.norms, codes, nq * T, ws, wsb)
 
@@ -177,8 +186,9 @@ def rvq_only(model: MimiModel, audio: torch.Tensor, nq: int, iters: int = 10) ->
             "distance_tflops": round(enc_tf, 3), "distance_frac_fp32_mfma": round(enc_tf / PEAK_FP32_TFLOPS, 4),
             "decode_ms": round(dec_ms, 4), "gather_bytes": gather_bytes,
             "gather_gbs": round(dec_gbs, 1), "gather_frac_hbm": round(dec_gbs / PEAK_HBM_GBS, 4),
-            "note": ("encode time covers every launch of fm_rvq_encode_split (per-codebook distance "
-                     "MFMA + argmin + residual subtract, both chains); FLOPs count 2*M*E*D per codebook")}
+            "note": ("encode time covers every launch of the split encode (per-codebook distance MFMA + "
+                     "argmin + residual subtract, both chains; above 1024 rows an fp16 screen with FP32 "
+                     "decisions, so its rate may pass the FP32 peak); FLOPs count 2*M*E*D per codebook")}
 
 
 TRAFFIC_FILE = REPO / "profiles" / "dec_up4_convt_c2_hbm_traffic.md"
@@ -210,7 +220,7 @@ def dominant_only(iters: int) -> None:
     """Launches of the dominant contraction plus a calibration copy (for --pmc runs)."""
     dev = torch.device("cuda", 0)
     model = MimiModel(MimiConfig(), device=dev, seed=0)
-    op = model.runtime().layer_op(DOMINANT, 1, 240_000)
+    op = model.runtime().layer_op(DOMINANT, 1, 240_000, nat.WEIGHTS_X6 | nat.WEIGHTS_H3)
     src = torch.randn(COPY_BYTES // 4, device=dev)
     dst = torch.empty_like(src)
     for _ in range(iters):

@@ -506,7 +506,10 @@ __global__ __launch_bounds__(NT, 3) void resblock_direct_kernel(
 // tile by one from a bound on it, max |ELU(x)| * K1 * max |w1| + max |b1|
 // (some 2^6 above what it reaches, of fp16's 2^39 range), so neither can
 // overflow and no exchange between the waves is needed.  Accumulators return
-// to the caller's scale in one exact step.
+// to the caller's scale in one exact step.  Two planes of ELU(x) take 33 KB, so
+// four blocks share a CU instead of three, and half the MFMAs go: 60000 rows of
+// 128 channels 30.3 -> 24.5 us; 16 clips of 10 s, 64 channels with the
+// waveform conv 579 -> 483 us, 128 channels 414 -> 321, 256 channels 281 -> 198.
 template <int C, int BM, int WM, int PD, bool WAVE_IN, bool WAVE_OUT, bool FAST_ACT = false, bool H3 = false>
 __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     const float* __restrict__ x, int L, const __bf16* __restrict__ w1x, const float* __restrict__ b1,

@@ -38,7 +38,9 @@ struct RowConvArgs {
 // fragment pair.  A wave takes its k-range in chunks of at most seven steps,
 // reads a chunk's A fragments of its rows first (ELU applied), scales each row
 // by a power of two from them, and adds the chunk's products back at the
-// caller's scale.
+// caller's scale.  Bound by the weights' way through L2 (4 bytes a weight here,
+// 6 in the bf16 form): the decoder's first conv at 250 rows 24.8 -> 21.9 us, the
+// 512-channel k3 conv at 2000 rows 20.1 -> 18.2 us.
 template <int K, int BN, bool X6, int MT, bool H3 = false>
 __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
   // MT 16-row MFMA tiles per block (bf16x6 only): each weight fragment a wave

@@ -1254,7 +1254,10 @@ __global__ __launch_bounds__(512) void row_stream_linear_kernel(
 // exponents, fm_split_weights_h3) and three v_mfma_f32_16x16x32_f16 products
 // per fragment pair.  A wave reads its whole k-range of the 16 rows first, takes
 // a power of two per row from it, and its partial tile returns to the caller's
-// scale as it goes to LDS; the column exponents follow after the sum.
+// scale as it goes to LDS; the column exponents follow after the sum.  A chain of
+// latencies (weight loads, products, cross-wave sum), so halving the MFMAs takes
+// off little (250 rows: qkv 9.1 -> 8.6 us, fc1 9.2 -> 8.5, fc2 10.0 -> 9.6, the
+// output projection 5.0 -> 4.8).
 template <int K, int BN, bool X6 = false, bool UPS = false, bool H3 = false>
 __global__ __launch_bounds__(512) void row16_linear_kernel(
     const float* __restrict__ x, int rows, const float* __restrict__ gamma,

@@ -90,7 +90,10 @@ int fm_split_weights(const float* weight_packed, int rows, int cols, void* plane
  * operand pair, activations split on the fly with a power-of-two scale per
  * row.  The error against float64 is that of FP32 sums (below the bf16x6
  * form's); results differ from it in the last bits, so callers whose codes
- * depend on exact sums keep FM_WEIGHTS_X6 alone.
+ * depend on exact sums keep FM_WEIGHTS_X6 alone.  fm_row_linear and
+ * fm_conv1d_rows (in_channels * kernel 256, 1536 or 3584; else the bf16
+ * form) take the flag together with FM_WEIGHTS_X6, and fm_resblock /
+ * fm_resblock64_conv together with FM_ACT_EXP.
  * No reference counterpart (as fm_split_weights).
  */
 int fm_split_weights_h3(const float* weight_packed, int rows, int cols, void* planes, hipStream_t stream);
@@ -183,14 +186,16 @@ int fm_resblock_supported(int channels);
 int fm_resblock(const float* x, int batch, int length, int channels, const float* w1_packed,
                 const float* b1, const float* w2_packed, const float* b2, int elu_out, float* y,
                 hipStream_t stream);
-/* elu_out: nonzero (other than the FM_WEIGHTS_X6 and FM_ACT_EXP bits)
- * applies the trailing ELU; FM_WEIGHTS_X6 says both packed weights carry
+/* elu_out: nonzero (other than the FM_WEIGHTS_X6, FM_WEIGHTS_H3 and
+ * FM_ACT_EXP bits) applies the trailing ELU; FM_WEIGHTS_X6 says both packed weights carry
  * their fm_split_weights planes (the block then runs on the bf16 matrix
  * cores).  FM_ACT_EXP (with FM_WEIGHTS_X6) evaluates the block's ELUs as
  * e^x - 1 from the hardware exponential: about half the vector instructions,
  * an absolute error of a few 1e-8 near zero instead of a relative one.  For
  * callers held to an absolute bar (the decoder's waveform), not for the
- * encoder, whose codes depend on exact activations. */
+ * encoder, whose codes depend on exact activations.  FM_WEIGHTS_H3 with
+ * FM_ACT_EXP runs the block on the fp16 planes after the bf16 ones (three
+ * products, fm_split_weights_h3); without FM_ACT_EXP it is ignored. */
 
 /*
  * The SEANet encoder's first conv (1 -> 64 channels, kernel 7, causal, no
@@ -217,7 +222,7 @@ int fm_conv_resblock64(const float* wav, int batch, int length, const float* w0_
  * Replaces MimiDecoder's last MimiResnetBlock + ELU + MimiConv1d
  * (model.py:1269-1285).
  */
-/* elu_mid may carry FM_WEIGHTS_X6 and FM_ACT_EXP as in fm_resblock. */
+/* elu_mid may carry FM_WEIGHTS_X6, FM_WEIGHTS_H3 and FM_ACT_EXP as in fm_resblock. */
 size_t fm_resblock64_conv_workspace_bytes(int batch, int length);
 int fm_resblock64_conv(const float* x, int batch, int length, const float* w1_packed,
                        const float* b1, const float* w2_packed, const float* b2, int elu_mid,
