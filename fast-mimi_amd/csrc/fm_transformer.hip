@@ -126,6 +126,12 @@ struct RowTile {
 
   FM_DEVICE void load(int tid, const float* __restrict__ src, long ld, int t0, int t_last,
                       const float* __restrict__ cos_t, const float* __restrict__ sin_t) {
+    load_rows(tid, [&](int t) { return src + (long)t * ld; }, t0, t_last, cos_t, sin_t);
+  }
+  // row_of(t): where row t lies.
+  template <typename RowOf>
+  FM_DEVICE void load_rows(int tid, RowOf row_of, int t0, int t_last, const float* __restrict__ cos_t,
+                           const float* __restrict__ sin_t) {
     okm = 0;
 #pragma unroll
     for (int u = 0; u < N; ++u) {
@@ -133,7 +139,7 @@ struct RowTile {
       const int r = e / (D / 8), d = (e % (D / 8)) * 4;
       const int t = min(t0 + r, t_last);
       okm |= (unsigned)(e < PAIRS && t0 + r <= t_last) << u;
-      const float* row = src + (long)t * ld;
+      const float* row = row_of(t);
       lo[u] = *reinterpret_cast<const floatx4*>(row + d);
       hi[u] = *reinterpret_cast<const floatx4*>(row + d + HALF);
       if (ROPE) {
@@ -168,13 +174,17 @@ struct VTile {
   // does not wait for its loads where it is issued.
   unsigned okm;
   FM_DEVICE void load(int lane, const float* __restrict__ src, long ld, int t0, int t_last) {
+    load_rows(lane, [&](int t) { return src + (long)t * ld; }, t0, t_last);
+  }
+  template <typename RowOf>
+  FM_DEVICE void load_rows(int lane, RowOf row_of, int t0, int t_last) {
     okm = 0;
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       const int e = lane + u * 64;
       const int r = e / (DP / 4), d = (e % (DP / 4)) * 4;
       const int t = min(t0 + r, t_last);
-      v[u] = *reinterpret_cast<const floatx4*>(src + (long)t * ld + min(d, D - 4));
+      v[u] = *reinterpret_cast<const floatx4*>(row_of(t) + min(d, D - 4));
       okm |= (unsigned)(e < CHUNKS && t0 + r <= t_last && d < D) << u;
     }
   }
@@ -381,11 +391,26 @@ __global__ __launch_bounds__(64 * NW) void window_attention_kernel(
 // lane holds in accumulator slot r.  O^T is four 16-dim row tiles (four
 // chains).  The waves' (max, sum, O) are merged through LDS with the factors
 // exp(m_w - M) computed once per query.  ROPE: Q and K rotate while staging.
-template <bool ROPE, int NW>
+//
+// STREAM: rows 0 .. q_start-1 are a streaming cache's keys / values
+// ([batch][q_start][kv_heads * 64]) and qkv holds the chunk's rows only, and the
+// blocks write the next cache (the last `keep` key / value rows) as they go.  A
+// streamed chunk is bound by its launches (about 9 us of host time each): the
+// operand's assembly was one more per layer (3.3 us on the GPU).  Four 80 ms
+// chunks: encode 2914 -> 2717 us, decode 2310 -> 2091 us.
+struct StreamKV {
+  const float* keys;
+  const float* values;
+  float* next_keys;
+  float* next_values;
+  int keep;
+};
+template <bool ROPE, int NW, bool STREAM = false>
 __global__ __launch_bounds__(64 * NW) void window_attention16_kernel(
     const float* __restrict__ qkv, int ld, int q_off, int k_off, int v_off,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, int T, int q_start,
-    int heads, int kv_heads, int window, float scale, float* __restrict__ out, int ld_out) {
+    int heads, int kv_heads, int window, float scale, float* __restrict__ out, int ld_out, StreamKV kv) {
+  static_assert(!(STREAM && ROPE), "a streamed chunk arrives rotated");
   constexpr int D = 64, QT = 16, NTH = 64 * NW;
   constexpr int PK = D + 4, PVV = D + 4, P = QT + 1;
   constexpr int SLOT = KB * PK + KB * PVV;
@@ -404,16 +429,26 @@ __global__ __launch_bounds__(64 * NW) void window_attention16_kernel(
   const int q = q0 + i;
   const int k_lo = max(0, q0 - window + 1);
   const int k_hi = min(T, q0 + QT) - 1;
-  const float* seq = qkv + b * (long)T * ld;
+  const int cached = STREAM ? q_start : 0;  // rows that qkv does not hold
+  const float* seq = qkv + b * (long)(T - cached) * ld;
   const float* kcol = seq + k_off + hk * D;
   const float* vcol = seq + v_off + hk * D;
+  const int kv_ld = kv_heads * D;
+  const float* kpast = STREAM ? kv.keys + (b * (long)cached * kv_ld + hk * D) : nullptr;
+  const float* vpast = STREAM ? kv.values + (b * (long)cached * kv_ld + hk * D) : nullptr;
+  auto k_row = [&](int t) {
+    return STREAM && t < cached ? kpast + (long)t * kv_ld : kcol + (long)(t - cached) * ld;
+  };
+  auto v_row = [&](int t) {
+    return STREAM && t < cached ? vpast + (long)t * kv_ld : vcol + (long)(t - cached) * ld;
+  };
 
   const int ntiles = (k_hi - k_lo + KB) / KB;
   RowTile<D, 64, ROPE> kr;
   VTile<D, D> vr;
   if (wave < ntiles) {
-    kr.load(lane, kcol, ld, k_lo + wave * KB, k_hi, cos_t, sin_t);
-    vr.load(lane, vcol, ld, k_lo + wave * KB, k_hi);
+    kr.load_rows(lane, k_row, k_lo + wave * KB, k_hi, cos_t, sin_t);
+    vr.load_rows(lane, v_row, k_lo + wave * KB, k_hi);
   }
   float qv[16];  // query i, dims 16g .. 16g+15
   if constexpr (ROPE) {
@@ -431,7 +466,7 @@ __global__ __launch_bounds__(64 * NW) void window_attention16_kernel(
   } else {
     // Each wave reads its query fragments straight from memory: no LDS pass
     // and no block barrier before the key loop.
-    const float* qrow = seq + (long)min(q, T - 1) * ld + q_off + head * D + 16 * g;
+    const float* qrow = seq + (long)(min(q, T - 1) - cached) * ld + q_off + head * D + 16 * g;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const floatx4 t4 = *reinterpret_cast<const floatx4*>(qrow + 4 * t);
@@ -456,8 +491,8 @@ __global__ __launch_bounds__(64 * NW) void window_attention16_kernel(
     vr.store(lane, Vs, PVV);
     wave_lds_fence();
     if (tile + NW < ntiles) {  // next tile's loads overlap this tile's math
-      kr.load(lane, kcol, ld, k0 + NW * KB, k_hi, cos_t, sin_t);
-      vr.load(lane, vcol, ld, k0 + NW * KB, k_hi);
+      kr.load_rows(lane, k_row, k0 + NW * KB, k_hi, cos_t, sin_t);
+      vr.load_rows(lane, v_row, k0 + NW * KB, k_hi);
     }
 
     floatx4 sc[2][2];
@@ -561,6 +596,17 @@ __global__ __launch_bounds__(64 * NW) void window_attention16_kernel(
       den += Lm[w][qi] * f;
     }
     out[(b * (long)(T - q_start) + qg - q_start) * ld_out + head * D + d] = num / den;
+  }
+  if constexpr (STREAM) {
+    // The next cache's rows of this key / value head, shared by the query
+    // blocks of the group's first head.
+    if (head % (heads / kv_heads)) return;
+    for (int e = blockIdx.x * NTH + tid; e < kv.keep * (D / 4); e += gridDim.x * NTH) {
+      const int r = e / (D / 4), d = (e % (D / 4)) * 4, t = T - kv.keep + r;
+      const long o = (b * kv.keep + r) * (long)kv_ld + hk * D + d;
+      *reinterpret_cast<floatx4*>(kv.next_keys + o) = *reinterpret_cast<const floatx4*>(k_row(t) + d);
+      *reinterpret_cast<floatx4*>(kv.next_values + o) = *reinterpret_cast<const floatx4*>(v_row(t) + d);
+    }
   }
 }
 
@@ -1825,6 +1871,40 @@ int fm_window_attention(const float* qkv, int ld_qkv, int q_offset, int k_offset
                                   ld_out, stream);
 }
 
+// Whether a chunk's attention runs on the 16-query kernel (as the same call of
+// fm_window_attention_rows would: the bits are the same), the one with a streaming form.
+int fm_window_attention_stream_supported(int batch, int length, int cached, int heads, int head_dim) {
+  if (head_dim != 64 || batch <= 0 || length <= 0 || cached < 0 || heads <= 0) return 0;
+  if ((long)batch * heads >= 128) return cached > 0 || length > SEQ_MAX;
+  return length < 512;
+}
+
+int fm_window_attention_stream(const float* qkv, int batch, int length, int heads, int kv_heads, const float* keys,
+                               const float* values, int cached, int keep, int window, float scale, float* out,
+                               int ld_out, float* next_keys, float* next_values, hipStream_t stream) {
+  if (!qkv || !out || batch < 0 || length < 0 || cached < 0 || keep < 0 || heads <= 0 || kv_heads <= 0 ||
+      heads % kv_heads || window <= 0 || (cached > 0 && (!keys || !values)) || keep > (long)cached + length ||
+      (keep > 0 && (!next_keys || !next_values)) || (long)cached + length > INT_MAX / 2)
+    return FM_BAD_ARGUMENT;
+  if (batch == 0 || length == 0) return FM_OK;
+  if (!fm_window_attention_stream_supported(batch, length, cached, heads, 64)) return FM_UNSUPPORTED;
+  // Rows are moved as float4s.
+  if (((uintptr_t)qkv | (uintptr_t)keys | (uintptr_t)values | (uintptr_t)next_keys | (uintptr_t)next_values) & 15)
+    return FM_BAD_ARGUMENT;
+  const dim3 grid((length + 15) / 16, heads, batch);
+  const int q_cols = heads * 64, kv_cols = kv_heads * 64;
+  const StreamKV kv{keys, values, next_keys, next_values, keep};
+  // Waves per block as in fm_window_attention_rows.
+#define FM_ATTS(W)                                                                                                   \
+  hipLaunchKernelGGL((window_attention16_kernel<false, W, true>), grid, dim3(64 * W), 0, stream, qkv,                \
+                     q_cols + 2 * kv_cols, 0, q_cols, q_cols + kv_cols, nullptr, nullptr, cached + length, cached,   \
+                     heads, kv_heads, window, scale, out, ld_out, kv)
+  if ((long)grid.x * grid.y * grid.z < 1024) FM_ATTS(8);
+  else FM_ATTS(4);
+#undef FM_ATTS
+  return (int)hipGetLastError();
+}
+
 // Attention for the queries at rows query_start .. length-1 of each sequence;
 // every row 0 .. length-1 is a key/value (rows before query_start hold a KV
 // cache).  out has length - query_start rows per sequence.
@@ -1873,7 +1953,7 @@ int fm_window_attention_rows(const float* qkv, int ld_qkv, int q_offset, int k_o
     // the grid is too small to fill the GPU, four once blocks are plentiful.
     const dim3 g16((length - query_start + 15) / 16, heads, batch);
     const bool eight16 = (long)g16.x * g16.y * g16.z < 1024;
-#define FM_ATT16(R, W)                                                                             hipLaunchKernelGGL((window_attention16_kernel<R, W>), g16, dim3(64 * W), 0, stream, qkv, ld_qkv,                      q_offset, k_offset, v_offset, cos_table, sin_table, length, query_start,                           heads, kv_heads, window, scale, out, ld_out)
+#define FM_ATT16(R, W)                                                                             hipLaunchKernelGGL((window_attention16_kernel<R, W>), g16, dim3(64 * W), 0, stream, qkv, ld_qkv,                      q_offset, k_offset, v_offset, cos_table, sin_table, length, query_start,                           heads, kv_heads, window, scale, out, ld_out, StreamKV{})
     if (cos_table) {
       if (eight16) FM_ATT16(true, 8);
       else FM_ATT16(true, 4);

@@ -83,6 +83,8 @@ _SIGNATURES = {
     "fm_upsample_depthwise": ([_P, _I, _I, _I, _P, _I, _I, _P, _P], _I),
     "fm_stream_append": ([_P, _P, _I, _I, _I, _I, _I, _P, _P, _P], _I),
     "fm_kv_append": ([_P, _I, _I, _I, _I, _P, _P, _I, _I, _P, _P, _P, _P], _I),
+    "fm_window_attention_stream_supported": ([_I, _I, _I, _I, _I], _I),
+    "fm_window_attention_stream": ([_P, _I, _I, _I, _I, _P, _P, _I, _I, _I, _F, _P, _I, _P, _P, _P], _I),
     "fm_copy_buffers": ([_P, _P, _S, _P, _P, _S, _P], _I),
     "fm_resblock_supported": ([_I], _I),
     "fm_resblock": ([_P, _I, _I, _I, _P, _P, _P, _P, _I, _P, _P], _I),

@@ -55,6 +55,7 @@ SPECS = {
     "fm_upsample_depthwise": "in:x i:batch i:length i:channels in:weight i:kernel i:stride out:y",
     "fm_stream_append": "in:context in:x i:batch i:pad i:length i:channels i:replicate out:buf out:next",
     "fm_kv_append": "in:qkv i:q_cols i:kv_cols i:batch i:length in:keys in:values i:cached i:keep out:comb out:next_keys out:next_values",
+    "fm_window_attention_stream": "in:qkv i:batch i:length i:heads i:kv_heads in:keys in:values i:cached i:keep i:window f:scale out:out i:ld_out out:next_keys out:next_values",
     "fm_copy_buffers": "in:src0 out:dst0 i:bytes0 in:src1 out:dst1 i:bytes1",
 }
 

@@ -626,6 +626,30 @@ class MimiRuntime:
         ctx = cache.update(x, idx)
         return torch.cat((ctx, x), dim=1) if ctx.shape[1] else x
 
+    def _attend_stream(self, q3, kv, li: int, nh: int, nkv: int, hd: int, att) -> bool:
+        """Attention of layer ``li``'s chunk ``q3`` over what ``kv`` retains and
+        the cache's advance in one launch, where one kernel serves both."""
+        B, T, _ = q3.shape
+        kd = nkv * hd
+        key = kv.key_cache[li] if li < len(kv.key_cache) else None
+        value = kv.value_cache[li] if key is not None else None
+        n = 0 if key is None else key.shape[1]
+        if (type(kv) is not MimiKVCache or T == 0 or kv.sliding_window is None
+                or not nat.library().fm_window_attention_stream_supported(B, T, n, nh, hd)):
+            return False
+        if key is not None and not all(type(t) is torch.Tensor and _plain(t, q3, (B, n, kd)) and
+                                       t.data_ptr() % 16 == 0 for t in (key, value)):
+            return False
+        kv._ensure_layer(li)
+        keep = min(n + T, kv.sliding_window - 1)
+        new_k, new_v = (torch.empty((B, keep, kd), device=self.device) for _ in range(2))
+        self._call("fm_window_attention_stream", q3, B, T, nh, nkv, key if n else None, value if n else None, n, keep,
+                   self.config.sliding_window, 1.0 / (hd ** 0.5), att, nh * hd, new_k if keep else None,
+                   new_v if keep else None)
+        kv._cumulative_lengths[li] += T
+        kv.key_cache[li], kv.value_cache[li] = new_k, new_v
+        return True
+
     def _attention_rows(self, q3, kv, li: int, qd: int, kd: int):
         """(operand, cached rows) of layer ``li``'s attention over the chunk
         ``q3`` [B, T, qd + 2 kd] and what ``kv`` retains, the cache advanced."""
@@ -699,10 +723,12 @@ class MimiRuntime:
                 self._call("fm_apply_rope", qkv, M, qkv.shape[1], qd + kd, hd,
                            cos, sin, T)
             ld = qkv.shape[1]
-            comb, n = self._attention_rows(qkv.view(B, T, ld), kv, li, qd, kd)
-            self._call("fm_window_attention_rows", comb, ld, 0, qd, qd + kd, None, None,
-                       B, n + T, n, nh, nkv, hd, cfg.sliding_window, 1.0 / (hd ** 0.5),
-                       att, qd)
+            q3 = qkv.view(B, T, ld)
+            if not self._attend_stream(q3, kv, li, nh, nkv, hd, att):
+                comb, n = self._attention_rows(q3, kv, li, qd, kd)
+                self._call("fm_window_attention_rows", comb, ld, 0, qd, qd + kd, None, None,
+                           B, n + T, n, nh, nkv, hd, cfg.sliding_window, 1.0 / (hd ** 0.5),
+                           att, qd)
             if fused:
                 self._row_linear(att, M, lay.wo, nat.EPI_RES_SCALE, residual=h, scale=lay.ls1, out=h)
                 ff = self._row_linear(h, M, lay.w1, nat.EPI_GELU, ln=lay.ln2)

@@ -498,6 +498,24 @@ int fm_kv_append(const float* qkv, int q_cols, int kv_cols, int batch, int lengt
                  float* next_values, hipStream_t stream);
 
 /*
+ * fm_kv_append and fm_window_attention_rows (head_dim 64, keys already rotated)
+ * in one launch, with the same results: qkv [batch][length][(heads + 2 *
+ * kv_heads) * 64] holds the chunk's rows, keys / values [batch][cached][kv_heads
+ * * 64] the cache (NULL when cached is 0); out has length rows per sequence;
+ * next_keys / next_values [batch][keep][kv_heads * 64] (other memory than keys
+ * / values) receive the last keep key / value rows.  Pointers of qkv, keys,
+ * values and the next ones 16-byte aligned.  Supported where
+ * fm_window_attention_stream_supported(...) != 0, else FM_UNSUPPORTED.
+ * Replaces MimiKVCache.update (model.py:363-518) and the cached attention
+ * (model.py:1870-1961).
+ */
+int fm_window_attention_stream_supported(int batch, int length, int cached, int heads, int head_dim);
+int fm_window_attention_stream(const float* qkv, int batch, int length, int heads, int kv_heads,
+                               const float* keys, const float* values, int cached, int keep, int window,
+                               float scale, float* out, int ld_out, float* next_keys, float* next_values,
+                               hipStream_t stream);
+
+/*
  * Copies bytes0 bytes from src0 to dst0 and bytes1 from src1 to dst1 (device
  * memory, buffers not overlapping; a zero size skips its pair) in one launch
  * on `stream`.  No reference counterpart: the hipGraph runner uses it to move

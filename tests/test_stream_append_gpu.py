@@ -52,6 +52,31 @@ def test_key_value_cache(rt, B, qd, kd, window, lengths):
         assert fast.get_seq_length() == slow.get_seq_length()
 
 
+@pytest.mark.parametrize("B,nh,nkv,lengths", [(1, 8, 8, (2, 2, 240, 17, 2)), (2, 8, 2, (15, 16, 300, 1)), (1, 2, 1, (511, 33)),
+                                              (17, 8, 8, (3, 2)), (3, 4, 4, (250, 600, 4))])
+def test_attention_advances_the_cache(rt, B, nh, nkv, lengths):
+    """One launch gives the attention's and the caches' bits of the two before it."""
+    window = rt.config.sliding_window
+    one, two = MimiKVCache(0, window), MimiKVCache(0, window)
+    qd, kd = 64 * nh, 64 * nkv
+    g = torch.Generator().manual_seed(B + nh)
+    for n in lengths:
+        q3 = torch.randn(B, n, qd + 2 * kd, generator=g).to(DEV)
+        a, b = (torch.full((B * n, qd), float("nan"), device=DEV) for _ in range(2))
+        if not rt._attend_stream(q3, one, 0, nh, nkv, 64, a):
+            comb, past = rt._attention_rows(q3, one, 0, qd, kd)
+            rt._call("fm_window_attention_rows", comb, qd + 2 * kd, 0, qd, qd + kd, None, None, B, past + n, past, nh,
+                     nkv, 64, window, 0.125, a, qd)
+        else:
+            assert n < 512
+        comb, past = rt._attention_rows(q3, two, 0, qd, kd)
+        rt._call("fm_window_attention_rows", comb, qd + 2 * kd, 0, qd, qd + kd, None, None, B, past + n, past, nh, nkv,
+                 64, window, 0.125, b, qd)
+        assert torch.equal(a, b)
+        assert torch.equal(one.key_cache[0], two.key_cache[0]) and torch.equal(one.value_cache[0], two.value_cache[0])
+        assert one.get_seq_length() == two.get_seq_length()
+
+
 def test_foreign_cache_tensors(rt):
     """Strided context and key tensors, as a caller may put there, still serve;
     a context of another shape is refused as before."""
