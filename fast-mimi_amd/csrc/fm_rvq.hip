@@ -1637,11 +1637,14 @@ int fm_rvq_prepare_screen(const float* embeds, const float* norms, int entries, 
   return (int)hipGetLastError();
 }
 
-// Above 1024 rows, where the step launches sum a dot product as one chain (as
-// the exact stage does) and take 34 us a step at 2000 rows, 100 us at 8000;
-// below, they split the codebook over more CUs than there are 32-row blocks.
+// Where the step launches sum a dot product as one chain, as the exact stage
+// does: with 2048 entries above 1024 rows (34 us a step at 2000 rows, 100 us at
+// 8000), with fewer entries from more rows on.  Below, they split the codebook
+// and the dims over more CUs than there are 32-row blocks, and their partial
+// sums round otherwise.
 int fm_rvq_screen_supported(int rows, int dim, int entries) {
-  return rows > 1024 && dim == 256 && entries > 0 && entries % 32 == 0 && entries <= SCREEN_ENTRIES;
+  return rows > 0 && dim == 256 && entries > 0 && entries % 32 == 0 && entries <= SCREEN_ENTRIES &&
+         rvq_plan(rows, dim, entries).kp == 1;
 }
 
 int fm_rvq_encode_split_screened(const float* x, int ld_x, int rows, int rows_per_batch, int dim, int entries,

@@ -426,8 +426,10 @@ int fm_rvq_encode_split_noalloc(const float* x, int ld_x, int rows, int rows_per
  * fm_rvq_encode_split as a screened search for many rows: approximate fp16
  * distances pick the entries that can be nearest, and their FP32 distances
  * decide, so the codes are fm_rvq_encode_split's bit for bit.  Supported where
- * fm_rvq_screen_supported(rows, dim, entries) != 0 (above 1024 rows, 256-dim
- * codebooks of at most 2048 entries, a multiple of 32), else FM_UNSUPPORTED.
+ * fm_rvq_screen_supported(rows, dim, entries) != 0 (256-dim codebooks of at
+ * most 2048 entries, a multiple of 32, over rows enough that
+ * ceil(rows / 32) * ceil(entries / 64) exceeds 1024: above 1024 rows with 2048
+ * entries, above 2048 with 1024), else FM_UNSUPPORTED.
  * planes / info come from fm_rvq_prepare_screen over the same `count` =
  * n_semantic + n_acoustic codebooks: [count][16][entries][16] fp16 (count *
  * entries * 512 bytes, at most 2 GiB) and 8 bytes per codebook.

@@ -117,3 +117,19 @@ def test_gemm_plan_query_is_host_only():
     assert isinstance(nat.last_gemm_plan(), str)
     with pytest.raises(nat.NativeError, match="bad argument"):
         nat.check(nat.library().fm_gemm_last_plan(None, 0), "fm_gemm_last_plan")
+
+
+def test_screened_search_only_where_the_step_launches_sum_one_chain():
+    """The screened search decides by one FMA chain over a row's 256 dims.  The
+    step launches do so too once 64-entry chunks of every 32-row block exceed
+    1024 blocks; below that they sum two or four partial chains, whose near-ties
+    round otherwise, so those sizes are refused (host only)."""
+    if not nat.LIBRARY_PATH.is_file():
+        pytest.skip("library not built")
+    supported = nat.library().fm_rvq_screen_supported
+    for rows, entries in ((1100, 1024), (2000, 1024), (2048, 1024), (1031, 1984), (1024, 2048), (2000, 512), (4096, 512),
+                          (8000, 128), (1031, 96), (16384, 96), (1031, 32), (32768, 32)):
+        assert not supported(rows, 256, entries), (rows, entries)
+    for rows, entries in ((1025, 2048), (1025, 2016), (1057, 1984), (2049, 1024), (4097, 512), (16385, 128), (16385, 96),
+                          (32769, 32), (8000, 2048)):
+        assert supported(rows, 256, entries), (rows, entries)

@@ -39,8 +39,8 @@ def books(emb):
 
 
 @pytest.mark.parametrize("B,T,nsem,n,e", [(1, 1025, 1, 8, 2048), (16, 125, 1, 8, 2048), (3, 2700, 1, 32, 2048),
-                                          (1, 1100, 2, 5, 1024), (2, 600, 0, 3, 2048), (2, 600, 3, 3, 2048),
-                                          (1, 1031, 1, 4, 96), (1, 1031, 1, 2, 32), (1, 8300, 1, 3, 2048),
+                                          (1, 2100, 2, 5, 1024), (2, 600, 0, 3, 2048), (2, 600, 3, 3, 2048),
+                                          (1, 16400, 1, 4, 96), (1, 32800, 1, 2, 32), (1, 8300, 1, 3, 2048),
                                           (205, 5, 1, 3, 2048)])
 def test_codes_equal_step_launches(B, T, nsem, n, e):
     g = torch.Generator().manual_seed(B * T + n + e)
@@ -50,13 +50,19 @@ def test_codes_equal_step_launches(B, T, nsem, n, e):
     assert torch.equal(encode(x, emb, norms, emb_t, nsem, T, True), want)
 
 
-@pytest.mark.parametrize("kind", ["ties", "cluster", "tiny", "huge", "zero_rows", "bad_rows", "bad_book", "mixed",
-                                  "on_entries", "zero_book", "offset"])
-def test_hard_inputs(kind):
+HARD = ["ties", "cluster", "tiny", "huge", "zero_rows", "bad_rows", "bad_book", "mixed", "on_entries", "zero_book",
+        "offset"]
+
+
+@pytest.mark.parametrize("kind,e,rows", [(k, 2048, 1300) for k in HARD] +
+                         [(k, e, rows) for k in ("cluster", "offset") for e, rows in ((1024, 2049), (512, 4100),
+                                                                                     (32, 32769))])
+def test_hard_inputs(kind, e, rows):
     """Equal and nearly equal entries, rows that are entries, scales near both
-    ends of FP32, zero and non-finite rows and codebooks."""
+    ends of FP32, zero and non-finite rows and codebooks; near-ties also at the
+    fewest rows a smaller codebook is accepted with."""
     g = torch.Generator().manual_seed(len(kind))
-    n, e, rows = 4, 2048, 1300
+    n = 4
     emb = torch.randn(n, e, 256, generator=g) / 16
     x = torch.randn(rows, 512, generator=g)
     if kind == "ties":
@@ -92,15 +98,17 @@ def test_hard_inputs(kind):
 
 
 def test_screen_rejects():
-    """Calls whose FP32 sums the step launches order otherwise (1024 rows or
-    fewer) and shapes without a screened form are refused."""
+    """Calls whose FP32 sums the step launches order otherwise (few rows for the
+    entries) and shapes without a screened form are refused."""
     t = torch.empty(4096, device=DEV)
     p = t.data_ptr()
     lib = nat.library()
-    for rows, dim, e in ((1024, 256, 2048), (2000, 128, 2048), (2000, 256, 2080), (2000, 256, 80), (2000, 256, 0)):
+    for rows, dim, e in ((1024, 256, 2048), (1100, 256, 1024), (1031, 256, 96), (1031, 256, 32), (2000, 128, 2048), (2000, 256, 2080), (2000, 256, 80), (2000, 256, 0)):
         assert not lib.fm_rvq_screen_supported(rows, dim, e)
     with pytest.raises(nat.NativeError, match="unsupported"):
         nat.call("fm_rvq_encode_split_screened", p, 512, 1024, 1024, 256, 2048, 1, 1, p, p, p, p, p, 2048, 0)
+    with pytest.raises(nat.NativeError, match="unsupported"):
+        nat.call("fm_rvq_encode_split_screened", p, 512, 1100, 1100, 256, 1024, 1, 1, p, p, p, p, p, 1024, 0)
     with pytest.raises(nat.NativeError, match="bad argument"):
         nat.call("fm_rvq_encode_split_screened", p, 512, 2000, 2000, 256, 2048, 1, 1, p, p, None, p, p, 2048, 0)
     with pytest.raises(nat.NativeError, match="unsupported"):
