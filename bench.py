@@ -160,7 +160,7 @@ def rvq_only(model: MimiModel, audio: torch.Tensor, nq: int, iters: int = 10) ->
     wsb = nat.library().fm_rvq_split_workspace_bytes(M, vq, E)
     ws = torch.empty((wsb + 3) // 4, device=audio.device)
     q = torch.empty((M, 2 * vq), device=audio.device)
-    screened = rt.screen is not None and nat.library().fm_rvq_screen_supported(M, vq, E)
+    screened = rt.screens(M, nq)
 
     def enc():  # as the runtime chooses for this many rows
         if screened:

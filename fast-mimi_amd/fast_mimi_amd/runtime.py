@@ -740,6 +740,14 @@ class MimiRuntime:
             self._proj(ff, M, lay.w2, nat.EPI_RES_SCALE, residual=h, scale=lay.ls2, out=h)
         return h.reshape(B, T, C)
 
+    def screens(self, rows: int, nq: int) -> bool:
+        """Whether ``rows`` x ``nq`` codebooks run as the screened search: the
+        sizes it is exact for, and fp16 codebooks that one 2 GiB buffer
+        resource reaches (2047 of 2048 entries); else the step launches."""
+        e = self.config.codebook_size
+        return (self.screen is not None and 2 * nq * e * self.vq < 2**31
+                and bool(nat.library().fm_rvq_screen_supported(rows, self.vq, e)))
+
     def quantize(self, h, B, T, nq):
         cfg = self.config
         M = B * T
@@ -748,13 +756,12 @@ class MimiRuntime:
         self._tag = "rvq.encode"
         codes = torch.empty((B, nq, T), dtype=torch.int64, device=self.device)
         n_sem = min(cfg.num_semantic_quantizers, nq)
-        lib = nat.library()
-        if self.screen is not None and lib.fm_rvq_screen_supported(M, vq, cfg.codebook_size):
+        if self.screens(M, nq):
             self._call("fm_rvq_encode_split_screened", proj, 2 * vq, M, T, vq, cfg.codebook_size,
                        n_sem, nq - n_sem, self.embeds, self.norms, self.screen, self.screen_info, codes,
                        nq * T)
             return codes
-        ws_bytes = lib.fm_rvq_split_workspace_bytes(M, vq, cfg.codebook_size)
+        ws_bytes = nat.library().fm_rvq_split_workspace_bytes(M, vq, cfg.codebook_size)
         # Both chains in shared launches (step s of each branch in one grid).
         ws = torch.empty((ws_bytes + 3) // 4, device=self.device)
         self._call("fm_rvq_encode_split", proj, 2 * vq, M, T, vq, cfg.codebook_size,

@@ -133,3 +133,19 @@ def test_screened_search_only_where_the_step_launches_sum_one_chain():
     for rows, entries in ((1025, 2048), (1025, 2016), (1057, 1984), (2049, 1024), (4097, 512), (16385, 128), (16385, 96),
                           (32769, 32), (8000, 2048)):
         assert supported(rows, 256, entries), (rows, entries)
+
+
+def test_screened_search_leaves_what_it_cannot_address():
+    """2048 codebooks of 2048 entries are 2 GiB of fp16 copies: the screened
+    entry refuses them, so the runtime takes the step launches (host only)."""
+    from types import SimpleNamespace
+
+    from fast_mimi_amd.runtime import MimiRuntime
+
+    if not nat.LIBRARY_PATH.is_file():
+        pytest.skip("library not built")
+    rt = SimpleNamespace(config=SimpleNamespace(codebook_size=2048), vq=256, screen=object())
+    assert MimiRuntime.screens(rt, 2000, 2047) and not MimiRuntime.screens(rt, 2000, 2048)
+    assert not MimiRuntime.screens(rt, 1000, 8)
+    assert nat.library().fm_rvq_encode_split_screened(64, 512, 2000, 2000, 256, 2048, 1, 2047, 64, 64, 64, 64, 64,
+                                                      2048, None) == 1002
