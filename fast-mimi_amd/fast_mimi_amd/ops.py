@@ -117,9 +117,12 @@ _POINTERS = {entry: tuple(i for i, item in enumerate(spec.split()) if item[:3] i
 def _observed() -> bool:
     """Whether something watches or transforms operator calls: a dispatch
     mode (tracing, fake tensors), a torch function mode, torch.compile,
-    torch.jit.trace, a functorch transform or the profiler."""
-    return bool(torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch.compiler.is_compiling()
+    torch.jit.trace, a functorch transform or the profiler.  (An execution
+    trace observer without the profiler cannot be asked for: it does not see
+    direct calls.)"""
+    # torch.compile first: it folds this to a constant and could not trace the rest.
+    return bool(torch.compiler.is_compiling()
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or torch._C._get_tracing_state() is not None
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch._C._autograd._profiler_enabled())

@@ -42,6 +42,24 @@ def test_observers_keep_the_operator_path():
     assert not ops._observed()
 
 
+def test_compiled_in_one_graph():
+    """torch.compile traces ops.call as the operator, without a graph break."""
+    graphs = []
+
+    def keep(gm, inputs):
+        graphs.append(gm)
+        return lambda *args: args[-1:]  # (the operator itself needs a GPU)
+
+    def body(src, dst):
+        ops.call("fm_copy_buffers", src, dst, 16, None, None, 0)
+        return dst + 1
+
+    torch._dynamo.reset()
+    torch.compile(body, backend=keep, fullgraph=True)(torch.ones(4), torch.zeros(4))
+    assert len(graphs) == 1
+    assert any("copy_buffers" in str(n.target) for n in graphs[0].graph.nodes if n.op == "call_function")
+
+
 def test_pointer_arguments_follow_the_schema():
     for entry, spec in ops.SPECS.items():
         kinds = [item.split(":")[0] for item in spec.split()]
