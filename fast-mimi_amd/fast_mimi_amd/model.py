@@ -363,7 +363,7 @@ class MimiModel:
     def _on_device(self, t: torch.Tensor, dtype) -> torch.Tensor:
         if t.device != self.device:
             raise ValueError(f"tensor on {t.device}, model on {self.device}")
-        return t.to(dtype).contiguous()
+        return t.to(dtype).contiguous().resolve_neg()
 
     def _graph(self, key, fn, inputs):
         runner = self._graphs.get(key)

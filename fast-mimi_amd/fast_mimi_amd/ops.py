@@ -132,7 +132,8 @@ def call(entry: str, *args) -> None:
     """Run C-ABI entry point ``entry``: through its operator when something
     observes operator calls or a tensor is not a plain one (a subclass, or
     one that requires a gradient), else the C function itself on the current
-    stream, which is all the operator's implementation does.  A streamed 80 ms
+    stream, which is all the operator's implementation does (the runtime
+    resolves lazy negations where tensors come in).  A streamed 80 ms
     chunk is some 85 calls; the dispatcher's way took about 11 us of host time
     each, this one about 4."""
     if not _observed():

@@ -119,8 +119,10 @@ def x6_plan(config: MimiConfig) -> dict[str, bool]:
 
 
 def _plain(t: torch.Tensor, like: torch.Tensor, shape: tuple) -> bool:
-    """A contiguous float32 tensor of ``shape`` on ``like``'s device."""
-    return t.shape == shape and t.dtype == torch.float32 and t.device == like.device and t.is_contiguous()
+    """A contiguous float32 tensor of ``shape`` on ``like``'s device whose
+    memory holds its values (no lazy negation)."""
+    return (t.shape == shape and t.dtype == torch.float32 and t.device == like.device and t.is_contiguous()
+            and not t.is_neg())
 
 
 def rope_tables(config: MimiConfig, length: int) -> tuple[torch.Tensor, torch.Tensor]:

@@ -3,12 +3,14 @@ calls, and a streamed RoPE table is a slice of a longer one (CPU only)."""
 
 from __future__ import annotations
 
+from types import SimpleNamespace
+
 import torch
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
-from fast_mimi_amd import MimiConfig, ops
-from fast_mimi_amd.runtime import rope_tables
+from fast_mimi_amd import MimiConfig, MimiModel, ops
+from fast_mimi_amd.runtime import _plain, rope_tables
 
 
 def test_observers_keep_the_operator_path():
@@ -58,6 +60,17 @@ def test_compiled_in_one_graph():
     torch.compile(body, backend=keep, fullgraph=True)(torch.ones(4), torch.zeros(4))
     assert len(graphs) == 1
     assert any("copy_buffers" in str(n.target) for n in graphs[0].graph.nodes if n.op == "call_function")
+
+
+def test_lazily_negated_inputs_are_resolved():
+    """A tensor with the negative bit holds other values than its memory; the
+    operators resolved it, direct calls pass its address."""
+    x = torch.arange(4.0).view(1, 1, 4)
+    neg = torch._neg_view(x)
+    got = MimiModel._on_device(SimpleNamespace(device=x.device), neg, torch.float32)
+    assert not got.is_neg() and torch.equal(got, -x) and got.data_ptr() != x.data_ptr()
+    assert MimiModel._on_device(SimpleNamespace(device=x.device), x, torch.float32).data_ptr() == x.data_ptr()
+    assert _plain(x, x, (1, 1, 4)) and not _plain(neg, x, (1, 1, 4))
 
 
 def test_pointer_arguments_follow_the_schema():
