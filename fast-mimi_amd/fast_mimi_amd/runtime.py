@@ -451,7 +451,8 @@ class MimiRuntime:
         tabs = self._stream_tabs[-1] if self._stream_tabs else None
         if tabs is None or tabs[0].shape[0] < end:
             if torch.cuda.is_current_stream_capturing():
-                raise RuntimeError("RoPE tables must be prepared before graph capture")
+                c, s = self._rope_tables(end)  # as prepare(end) made it, or an error
+                return c[past:], s[past:]
             size = 512
             while size < end:
                 size *= 2

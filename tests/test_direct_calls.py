@@ -5,12 +5,13 @@ from __future__ import annotations
 
 from types import SimpleNamespace
 
+import pytest
 import torch
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from fast_mimi_amd import MimiConfig, MimiModel, ops
-from fast_mimi_amd.runtime import _plain, rope_tables
+from fast_mimi_amd.runtime import MimiRuntime, _plain, rope_tables
 
 
 def test_observers_keep_the_operator_path():
@@ -84,3 +85,25 @@ def test_rope_table_prefixes():
     for n in (1, 2, 3, 7, 100, 251, 777, 2047):
         for a, b in zip(whole, rope_tables(MimiConfig(), n)):
             assert torch.equal(a[:n], b)
+
+
+def test_prepared_stream_tables_serve_a_capture(monkeypatch):
+    """While a graph is captured no table can be uploaded: a streamed chunk
+    takes the one prepare() made for its end position."""
+    rt = MimiRuntime.__new__(MimiRuntime)
+    rt.config, rt.device, rt._rope, rt._stream_tabs = MimiConfig(), torch.device("cpu"), {}, []
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    rt.prepare(700)
+    capturing[0] = True
+    whole = rope_tables(rt.config, 700)
+    for got, want in zip(rt._stream_rope(698, 2), whole):
+        assert torch.equal(got, want[698:])
+    with pytest.raises(RuntimeError, match="prepared"):
+        rt._stream_rope(699, 2)
+    capturing[0] = False
+    rt._stream_rope(699, 2)
+    capturing[0] = True
+    assert rt._stream_rope(1000, 24)[0].shape == (24, 64)
+    with pytest.raises(RuntimeError, match="prepared"):
+        rt._stream_rope(1000, 25)
