@@ -436,11 +436,13 @@ class MimiModel:
             # The work is queued behind the range check and the check's answer
             # awaited before the call returns (the decode kernel reads no entry
             # for a code out of range), so the GPU does not idle over a round
-            # trip to the host.  A caller's own cache type may not be undone,
-            # so it waits first.
+            # trip to the host.  What a refused call could not take back waits
+            # first: a caller's own cache type, the graph of a new shape.
             check = _CodesCheck(self, codes)
             ours = type(kv) is MimiKVCache
-            if kv is not None and not ours and check.bad():
+            graph_key = ("dec", tuple(codes.shape), out_len)
+            builds = kv is None and self.use_graphs and graph_key not in self._graphs
+            if (builds or (kv is not None and not ours)) and check.bad():
                 raise IndexError("audio code out of range of the codebook")
             saved = {k: list(v) if isinstance(v, list) else v for k, v in vars(kv).items()} if ours else None
             try:
@@ -448,8 +450,7 @@ class MimiModel:
                     audio = rt.decode(codes, out_len, kv)
                 elif self.use_graphs:
                     rt.prepare(frames * (2 if rt.bottleneck else 1))
-                    audio = self._graph(("dec", tuple(codes.shape), out_len),
-                                        lambda c: rt.decode(c, out_len), (codes,))
+                    audio = self._graph(graph_key, lambda c: rt.decode(c, out_len), (codes,))
                 else:
                     rt.prepare(frames * (2 if rt.bottleneck else 1))
                     audio = rt.decode(codes, out_len)

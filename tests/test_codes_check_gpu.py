@@ -62,6 +62,18 @@ def test_bad_codes_refused_and_state_kept(model, graphs):
     model.use_graphs = True
 
 
+def test_bad_codes_of_a_new_shape_build_nothing(model):
+    """A refused call of a shape seen for the first time captures no graph
+    (each would keep a memory pool)."""
+    before = set(model._graphs)
+    for t in (17, 19):
+        with pytest.raises(IndexError):
+            model.decode(codes(6, t=t) + 2048)
+    assert set(model._graphs) == before
+    model.decode(codes(6, t=17))
+    assert len(model._graphs) == len(before) + 1
+
+
 def test_foreign_cache_is_not_touched(model):
     class Mine(MimiKVCache):
         pass
