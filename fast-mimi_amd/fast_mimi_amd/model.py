@@ -444,7 +444,8 @@ class MimiModel:
             builds = kv is None and self.use_graphs and graph_key not in self._graphs
             if (builds or (kv is not None and not ours)) and check.bad():
                 raise IndexError("audio code out of range of the codebook")
-            saved = {k: list(v) if isinstance(v, list) else v for k, v in vars(kv).items()} if ours else None
+            saved = dict(vars(kv)) if ours else {}
+            held = {k: list(v) for k, v in saved.items() if isinstance(v, list)}
             try:
                 if kv is not None:
                     audio = rt.decode(codes, out_len, kv)
@@ -456,7 +457,9 @@ class MimiModel:
                     audio = rt.decode(codes, out_len)
             finally:
                 if check.bad():
-                    if saved is not None:
+                    for name, items in held.items():
+                        saved[name][:] = items  # the same list objects: callers may hold them
+                    if ours:
                         vars(kv).update(saved)
                     raise IndexError("audio code out of range of the codebook")
         if not return_dict:

@@ -74,6 +74,17 @@ def test_bad_codes_of_a_new_shape_build_nothing(model):
     assert len(model._graphs) == len(before) + 1
 
 
+def test_refused_call_keeps_the_cache_lists(model):
+    """The lists a caller holds of a cache stay the cache's own."""
+    kv = MimiKVCache(2)
+    model.decode(codes(3, t=2), decoder_past_key_values=kv)
+    keys, values, lengths = kv.key_cache, kv.value_cache, kv._cumulative_lengths
+    with pytest.raises(IndexError):
+        model.decode(codes(4, t=2) + 2048, decoder_past_key_values=kv)
+    assert kv.key_cache is keys and kv.value_cache is values and kv._cumulative_lengths is lengths
+    assert kv.get_seq_length() == 4 and keys[0].shape[1] == 4
+
+
 def test_foreign_cache_is_not_touched(model):
     class Mine(MimiKVCache):
         pass
