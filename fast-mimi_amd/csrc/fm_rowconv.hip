@@ -38,7 +38,8 @@ struct RowConvArgs {
 // fragment pair.  A wave takes its k-range in chunks of at most seven steps,
 // reads a chunk's A fragments of its rows first (ELU applied), scales each row
 // by a power of two from them, and adds the chunk's products back at the
-// caller's scale.  Bound by the weights' way through L2 (4 bytes a weight here,
+// caller's scale (row and column exponents in one step, so that sums near FP32's
+// upper end do not overflow on the way).  Bound by the weights' way through L2 (4 bytes a weight here,
 // 6 in the bf16 form): the decoder's first conv at 250 rows 24.8 -> 21.9 us, the
 // 512-channel k3 conv at 2000 rows 20.1 -> 18.2 us.
 template <int K, int BN, bool X6, int MT, bool H3 = false>
@@ -100,6 +101,9 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
     };
 #pragma unroll
     for (int u = 0; u < R; ++u) load_unit(u, u);
+    int ce[NT];  // this lane's columns' weight exponents
+#pragma unroll
+    for (int j = 0; j < NT; ++j) ce[j] = reinterpret_cast<const int*>(wh + 2 * PL)[n0 + 16 * j + li];
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) {
       floatx4 ah[MT][CS][2];
@@ -157,7 +161,7 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
           const int e = -__shfl(se[mt], 4 * g + r, 64);
 #pragma unroll
           for (int j = 0; j < NT; ++j)
-            acc[mt][j][r] = __fadd_rn(acc[mt][j][r], __builtin_amdgcn_ldexpf(part[mt][j][r], e));
+            acc[mt][j][r] = __fadd_rn(acc[mt][j][r], __builtin_amdgcn_ldexpf(part[mt][j][r], e - ce[j]));
         }
     }
   } else if constexpr (X6) {
@@ -299,9 +303,6 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
     float v = red[er * PR + ec + c];
 #pragma unroll
     for (int q = 1; q < NWV; ++q) v = __fadd_rn(v, red[(q * BM + er) * PR + ec + c]);
-    if constexpr (H3)
-      v = __builtin_amdgcn_ldexpf(
-          v, -reinterpret_cast<const int*>(p.w + (long)p.N * K + 5L * p.N * K / 2)[n0 + ec + c]);
     if (p.bias) v = __fadd_rn(v, p.bias[(n0 + ec + c) % p.bias_len]);
     if (p.flags & FM_EPI_RES_ADD) v = __fadd_rn(p.res[m * p.N + n0 + ec + c], v);
     if (p.flags & FM_EPI_ELU) v = fm_elu(v);

@@ -1300,7 +1300,8 @@ __global__ __launch_bounds__(512) void row_stream_linear_kernel(
 // exponents, fm_split_weights_h3) and three v_mfma_f32_16x16x32_f16 products
 // per fragment pair.  A wave reads its whole k-range of the 16 rows first, takes
 // a power of two per row from it, and its partial tile returns to the caller's
-// scale as it goes to LDS; the column exponents follow after the sum.  A chain of
+// scale as it goes to LDS: row and column exponents in one step (in two, sums
+// near FP32's upper end overflow on the way).  A chain of
 // latencies (weight loads, products, cross-wave sum), so halving the MFMAs takes
 // off little (250 rows: qkv 9.1 -> 8.6 us, fc1 9.2 -> 8.5, fc2 10.0 -> 9.6, the
 // output projection 5.0 -> 4.8).
@@ -1384,12 +1385,10 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
   const bool rope = BN == 64 && cos_t && n0 < rope_cols;
   const bool res_scale = flags & FM_EPI_RES_SCALE;
   float e_res[OPT], e_scale[OPT], e_cos[OPT], e_sin[OPT];
-  int e_col[OPT];  // H3: the columns' weight exponents
   auto fetch_epilogue = [&]() {
 #pragma unroll
     for (int c = 0; c < OPT; ++c) {
       const int n = n0 + ec + c;
-      if constexpr (H3) e_col[c] = reinterpret_cast<const int*>(wp + (long)N * K)[n];
       e_res[c] = res_scale ? res[mc * N + n] : 0.0f;
       e_scale[c] = res_scale ? scale[n] : 0.0f;
       e_cos[c] = rope ? cos_t[(long)tpos * 64 + ec + c] : 0.0f;
@@ -1413,7 +1412,6 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
       float v = red[er * PR + ec + c];
 #pragma unroll
       for (int q = 1; q < NWV; ++q) v = __fadd_rn(v, red[(q * BM + er) * PR + ec + c]);
-      if constexpr (H3) v = __builtin_amdgcn_ldexpf(v, -e_col[c]);
       out[c] = v;
     }
     if (rope || UPS) {
@@ -1499,6 +1497,9 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
           ah[st][h] = *reinterpret_cast<const floatx4*>(As + li * PA + kw0 + 32 * st + 8 * g + 4 * h);
     }
     fetch_epilogue();
+    int ce[NT];  // this lane's columns' weight exponents
+#pragma unroll
+    for (int j = 0; j < NT; ++j) ce[j] = reinterpret_cast<const int*>(wh + 2 * PL)[n0 + 16 * j + li];
     const int se = h3_row_exp16(ah);
     const float sc = __builtin_amdgcn_ldexpf(1.0f, se);
     __builtin_amdgcn_sched_barrier(0);
@@ -1521,7 +1522,7 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
     for (int r = 0; r < 4; ++r) {
       const int e = -__shfl(se, 4 * g + r, 64);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j][r] = __builtin_amdgcn_ldexpf(acc[j][r], e);
+      for (int j = 0; j < NT; ++j) acc[j][r] = __builtin_amdgcn_ldexpf(acc[j][r], e - ce[j]);
     }
     reduce_and_store(acc);
     return;

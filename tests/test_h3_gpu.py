@@ -348,3 +348,32 @@ def test_conv1d_rows(B, cin, cout, k, L, flags):
     with pytest.raises(nat.NativeError, match="unsupported"):
         nat.call("fm_conv1d_rows", xd.data_ptr(), B, L, cin, wp.data_ptr(), layer.b.data_ptr(), cout, cout, k, 1, 0,
                  nat.WEIGHTS_H3, rd.data_ptr(), y.data_ptr(), stream())
+
+
+@pytest.mark.parametrize("kind,k,n,rows", [("row", 512, 1536, 26), ("row", 512, 512, 250), ("row", 2048, 512, 13),
+                                           ("conv", 7, 1024, 26), ("conv", 7, 1024, 265), ("conv", 3, 256, 2000),
+                                           ("conv", 1, 512, 40)])
+@pytest.mark.parametrize("weight_exp", [0, -60, -100])
+def test_few_rows_reach_the_ends_of_fp32(kind, k, n, rows, weight_exp):
+    """Results of 2^100 and more, to which every partial product belongs, stay
+    finite whatever the weights' own scale: a weight row's exponent (13 and up,
+    more for small weights) must not meet a partial sum alone."""
+    g = torch.Generator().manual_seed(rows + n)
+    cin = k if kind == "row" else 256 if k == 1 else 512
+    taps = 1 if kind == "row" else k
+    x = torch.randn(1, cin, rows, generator=g) * 2.0 ** (112 if weight_exp == 0 else 120)
+    w = torch.randn(n, cin, taps, generator=g) / math.sqrt(cin * taps) * 2.0 ** weight_exp
+    layer = _Conv(w.to(DEV), torch.zeros(n, device=DEV))
+    wp, _ = with_planes(layer.w)
+    xd = x.transpose(1, 2).contiguous().to(DEV)
+    y = torch.full((1, rows, n), float("nan"), device=DEV)
+    if kind == "row":
+        nat.call("fm_row_linear", xd.data_ptr(), rows, k, None, None, 1e-5, wp.data_ptr(), n, FLAGS, None, None, None,
+                 None, 0, 1, y.data_ptr(), stream())
+    else:
+        nat.call("fm_conv1d_rows", xd.data_ptr(), 1, rows, cin, wp.data_ptr(), layer.b.data_ptr(), n, n, k, 1, 0, FLAGS,
+                 None, y.data_ptr(), stream())
+    torch.cuda.synchronize()
+    want = causal_conv1d(x.double(), w.double(), torch.zeros(n, dtype=torch.float64))
+    close_dot(y.cpu().transpose(1, 2), want, causal_conv1d(x.double().abs(), w.double().abs(),
+                                                           torch.zeros(n, dtype=torch.float64)))
