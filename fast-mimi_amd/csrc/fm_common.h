@@ -6,6 +6,7 @@
 #include <climits>
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #define FM_DEVICE __device__ __forceinline__
 
@@ -164,6 +165,31 @@ FM_DEVICE void split2(floatx4 lo, floatx4 hi, float sc, halfx8& h0, halfx8& h1) 
 FM_DEVICE int h3_exp_for(float m, int to) {
   const int f = (int)(__builtin_bit_cast(unsigned, m) >> 23) & 255;
   return m > 0.0f ? min(max(127 + to + 127 - f, 1), 253) - 127 : 0;
+}
+
+// The largest m >= 0 of each aligned group of 16, 32 or 64 lanes, in all of
+// them (compared as integers: float maxima would canonicalise every operand):
+// within 16 lanes on DPP operands, across them by row swaps.
+template <int LANES>
+FM_DEVICE float lanes_max(float m) {
+  static_assert(LANES == 16 || LANES == 32 || LANES == 64, "whole DPP rows");
+  auto dpp = [](int v, auto ctrl) {
+    return __builtin_amdgcn_update_dpp(0, v, decltype(ctrl)::value, 0xf, 0xf, true);
+  };
+  int u = __builtin_bit_cast(int, m);
+  u = max(u, dpp(u, std::integral_constant<int, 0xb1>{}));   // lane ^ 1
+  u = max(u, dpp(u, std::integral_constant<int, 0x4e>{}));   // lane ^ 2
+  u = max(u, dpp(u, std::integral_constant<int, 0x141>{}));  // mirrored within 8 lanes
+  u = max(u, dpp(u, std::integral_constant<int, 0x140>{}));  // mirrored within 16 lanes
+  if constexpr (LANES >= 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    u = max((int)r[0], (int)r[1]);
+  }
+  if constexpr (LANES == 64) {
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    u = max((int)r[0], (int)r[1]);
+  }
+  return __builtin_bit_cast(float, u);
 }
 
 // A 16-row wave fragment of the few-row h3 kernels: S 32-deep k steps, lane (row

@@ -500,16 +500,21 @@ __global__ __launch_bounds__(NT, 3) void resblock_direct_kernel(
 // per-CU address path, not the MFMAs, then limits: 1.55x slower).
 //
 // H3: the same block on fp16 weights (fm_split_weights_h3) with three products
-// per operand pair and two planes per operand.  ELU(x) is scaled by one power
-// of two per block, from the block's largest magnitude (into [2^13, 2^14):
-// a value's error is 2^-23 of it or 2^-39 of that largest one); the hidden
-// tile by one from a bound on it, max |ELU(x)| * K1 * max |w1| + max |b1|
-// (some 2^6 above what it reaches, of fp16's 2^39 range), so neither can
-// overflow and no exchange between the waves is needed.  Accumulators return
-// to the caller's scale in one exact step.  Two planes of ELU(x) take 33 KB, so
-// four blocks share a CU instead of three, and half the MFMAs go: 60000 rows of
-// 128 channels 30.3 -> 24.5 us; 16 clips of 10 s, 64 channels with the
-// waveform conv 579 -> 483 us, 128 channels 414 -> 321, 256 channels 281 -> 198.
+// per operand pair and two planes per operand.  Each row of ELU(x) is scaled by
+// its own power of two, from its largest magnitude (into [2^13, 2^14): a
+// value's error is 2^-23 of it or 2^-39 of that largest one); each hidden row
+// by one from a bound on it, (the largest magnitudes of its three input rows)
+// * C * max |w1| + max |b1| (some 2^6 above what it reaches, of fp16's 2^39
+// range), so neither can overflow and no exchange between the waves is needed.
+// A tap's products are summed at its input row's scale and join the others at
+// the loudest one's, so a row's result depends on its own three input rows
+// alone.  Accumulators return to the caller's scale in one exact step.  Two
+// planes of ELU(x) take 33 KB, so four blocks share a CU instead of three, and
+// half the MFMAs go: 60000 rows of 128 channels
+// 31.1 -> 25.7 us; 16 clips of 10 s, 64 channels 616 -> 512 us (486 with the
+// waveform conv), 128 channels 432 -> 345, 256 channels 359 -> 276.  (One scale
+// for a block's rows measured 507, 478, 341 and 270 us there, but took bits
+// from quiet rows beside a loud one.)
 template <int C, int BM, int WM, int PD, bool WAVE_IN, bool WAVE_OUT, bool FAST_ACT = false, bool H3 = false>
 __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     const float* __restrict__ x, int L, const __bf16* __restrict__ w1x, const float* __restrict__ b1,
@@ -531,7 +536,9 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
   __shared__ __attribute__((aligned(16))) char smem[NP * XPLANE > EBYTES ? NP * XPLANE : EBYTES];
   __shared__ float wins[WAVE_IN ? BM + 8 : 1];  // WAVE_IN: waveform samples t0-8 .. t0+BM-1
 
-  __shared__ float topS[4];  // H3: each wave's largest |ELU(x)|
+  // H3: each staged row's largest |ELU(x)| and each hidden row's exponent.
+  __shared__ float topS[H3 ? XR : 1];
+  __shared__ __attribute__((aligned(16))) int expS[H3 ? BM : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, lcol = lane & 31;
@@ -643,22 +650,18 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
   };
 #pragma unroll
   for (int d = 0; d < PD; ++d) load_unit(d, ring[d]);
-  // H3: row exponents of the two weights (after their planes), the block's
-  // scale 2^sx and the hidden tile's 2^sh.
+  // H3: row exponents of the two weights (after their planes), the smallest of
+  // w1's (|w1| < 2^(14 - emin)) and the largest |b1|.
   const int* e1 = reinterpret_cast<const int*>(w1x + 2 * HC * K1);
   const int* e2 = reinterpret_cast<const int*>(w2x + 2 * C * HC);
-  int sx = 0, sh = 0;
+  int emin = 127;
+  float bmax = 0.0f;
+  // The scale of a row of ELU(x) as its exponent field (h3_exp_for(top, 13) +
+  // 127; a row of zeros takes the largest).
+  auto row_field = [](float top) {
+    return min(max(127 + 13 + 127 - (int)(__builtin_bit_cast(unsigned, top) >> 23), 1), 253);
+  };
   if constexpr (H3) {
-    float top = 0.0f, bmax = 0.0f;
-    int emin = 127;
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        xv[u][e] = act(xv[u][e]);
-        const float m = fabsf(xv[u][e]);
-        top = fmaxf(top, m < INFINITY ? m : 0.0f);  // a non-finite value spoils its own outputs only
-      }
 #pragma unroll
     for (int n = 0; n < (HC + 63) / 64; ++n) {
       const int i = min(lane + 64 * n, HC - 1);
@@ -667,26 +670,30 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      top = fmaxf(top, __shfl_xor(top, o, 64));
       emin = min(emin, __shfl_xor(emin, o, 64));
       bmax = fmaxf(bmax, __shfl_xor(bmax, o, 64));
     }
-    if (lane == 0) topS[wave] = top;
-    __syncthreads();
-    top = fmaxf(fmaxf(topS[0], topS[1]), fmaxf(topS[2], topS[3]));
-    sx = h3_exp_for(top, 13);
-    // |w1| < 2^(14 - emin): the bound in [2^14, 2^15).
-    sh = h3_exp_for(__builtin_amdgcn_ldexpf(top * K1, 14 - emin) + bmax, 14);
+    emin = __builtin_amdgcn_readfirstlane(emin);  // (scalar registers: the vector ones are all taken)
+    bmax = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, bmax)));
   }
-  const float scx = __builtin_amdgcn_ldexpf(1.0f, sx), sch = __builtin_amdgcn_ldexpf(1.0f, sh);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int c = tid + u * NT;
+    float top = 0.0f;
+    if constexpr (H3) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xv[u][e] = act(xv[u][e]);
+        top = fmaxf(top, fabsf(xv[u][e]));  // (a non-finite value spoils every output that reads its row)
+      }
+      top = lanes_max<C / 4>(top);  // the lanes of one row
+    }
     if (c >= CH) continue;
     const int r = c / (C / 4), k = (c % (C / 4)) * 4;
     if constexpr (H3) {
+      topS[r] = top;  // (the same from every lane of the row: no branch)
       halfx4 p0, p1;
-      split2(xv[u], scx, p0, p1);
+      split2(xv[u], __builtin_bit_cast(float, row_field(top) << 23), p0, p1);
       char* dst = smem + chunk(r, k >> 3, C * 2) + (k & 4) * 2;
       *reinterpret_cast<halfx4*>(dst) = p0;
       *reinterpret_cast<halfx4*>(dst + XPLANE) = p1;
@@ -719,6 +726,20 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     for (int r = 0; r < 16; ++r) acc1[i][r] = 0.0f;
   frag8 xf[2][NP][2];
   load_x(0, xf[0]);
+  // H3: a tap's sum is taken alone, then joins acc1[0] at the scale of the
+  // loudest of the position's three input rows (exponent sx).
+  constexpr int TU = C / 32;  // units per tap
+  constexpr bool DELAY = C == 64;
+  // What the taps' exponents lie above sx (0 .. 252) and sx + 127, a byte each
+  // in one register: four would spill.
+  unsigned exps = 0;
+  if constexpr (H3) {
+    const int s0 = row_field(topS[prow]), s1 = row_field(topS[prow + 1]), s2 = row_field(topS[prow + 2]);
+    const int sx = min(min(s0, s1), s2);
+    exps = (unsigned)(s0 - sx) | (unsigned)(s1 - sx) << 8 | (unsigned)(s2 - sx) << 16 | (unsigned)sx << 24;
+  }
+  // (2^-150 and less of a tap's sum vanish beside the loudest row's.)
+  auto tap_scale = [&](int tap) { return __builtin_amdgcn_ldexpf(1.0f, -(int)(exps >> 8 * tap & 255)); };
 #pragma unroll
   for (int u = 0; u < T1; ++u) {
     if (u + 1 < T1) load_x(u + 1, xf[(u + 1) & 1]);
@@ -727,9 +748,10 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       if constexpr (H3) {
-        acc1[0] = fm_mfma32_f16(w[1][s], a[0][s], acc1[0]);
-        acc1[1] = fm_mfma32_f16(w[0][s], a[0][s], acc1[1]);
-        acc1[0] = fm_mfma32_f16(w[0][s], a[1][s], acc1[0]);
+        floatx16& acc = acc1[u >= TU];
+        acc = fm_mfma32_f16(w[1][s], a[0][s], acc);
+        acc = fm_mfma32_f16(w[0][s], a[1][s], acc);
+        acc = fm_mfma32_f16(w[0][s], a[0][s], acc);
       } else {
         acc1[0] = fm_mfma32_bf16(w[1][s], a[1][s], acc1[0]);
         acc1[1] = fm_mfma32_bf16(w[2][s], a[0][s], acc1[1]);
@@ -741,6 +763,33 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     }
     if (u + PD < T) load_unit(u + PD, ring[u % PD]);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (H3) {
+      if (DELAY ? u == TU : u == TU - 1) {  // tap 0; where registers allow, while tap 1's products run
+        const float sc = tap_scale(0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc1[0][r] *= sc;
+        asm volatile("" : "+v"(acc1[0]));
+      }
+      if (u == 2 * TU - 1 || u == T1 - 1) {
+        const float sc = tap_scale(u == T1 - 1 ? 2 : 1);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          acc1[0][r] = fmaf(acc1[1][r], sc, acc1[0][r]);  // (an exact product)
+          acc1[1][r] = 0.0f;
+        }
+        // (Kept here: sunk below the last tap, three taps' sums would spill.)
+        asm volatile("" : "+v"(acc1[0]));
+      }
+    }
+  }
+  const int sx = (int)(exps >> 24) - 127;
+  float sch = 1.0f;  // H3: the hidden row's scale; its exponent goes to expS
+  if constexpr (H3) {
+    // The bound in [2^14, 2^15).
+    const float top = topS[prow] + topS[prow + 1] + topS[prow + 2];
+    const int sh = h3_exp_for(__builtin_amdgcn_ldexpf(top * C, 14 - emin) + bmax, 14);
+    sch = __builtin_amdgcn_ldexpf(1.0f, sh);
+    if (wc == 0 && h == 0) expS[prow] = sh;
   }
   __syncthreads();  // every wave is done with the ELU(x) planes
   {
@@ -755,8 +804,7 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
         const int es[4] = {en.x, en.y, en.z, en.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          v[e] = act(__fadd_rn(__builtin_amdgcn_ldexpf(__fadd_rn(acc1[0][4 * g + e], acc1[1][4 * g + e]),
-                                                       -(es[e] + sx)), bb[e]));
+          v[e] = act(__fadd_rn(__builtin_amdgcn_ldexpf(acc1[0][4 * g + e], -(es[e] + sx)), bb[e]));
         halfx4 p0, p1;
         split2(v, sch, p0, p1);
         *reinterpret_cast<halfx4*>(dst) = p0;
@@ -797,6 +845,8 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
       }
   }
   // 1x1 conv: acc[position][output channel], two 32-wide column tiles.
+  int hrow = prow;
+  if constexpr (H3) asm volatile("" : "+v"(hrow));  // (addresses kept from the k3 conv would spill)
   floatx16 acc2[FN2];
 #pragma unroll
   for (int j = 0; j < FN2; ++j)
@@ -809,7 +859,7 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     for (int pl = 0; pl < NP; ++pl)
 #pragma unroll
       for (int s = 0; s < 2; ++s)
-        a[pl][s] = *reinterpret_cast<const frag8*>(smem + pl * HPLANE + chunk(prow, kt * 4 + 2 * s + h, HC * 2));
+        a[pl][s] = *reinterpret_cast<const frag8*>(smem + pl * HPLANE + chunk(hrow, kt * 4 + 2 * s + h, HC * 2));
 #pragma unroll
     for (int j = 0; j < FN2; ++j) {
       const int u = T1 + kt * FN2 + j;
@@ -836,9 +886,10 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
   if constexpr (H3) {
 #pragma unroll
     for (int j = 0; j < FN2; ++j) {
-      const int e = -(e2[wc * 64 + j * 32 + lcol] + sh);
+      const int e = e2[wc * 64 + j * 32 + lcol];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc2[j][r] = __builtin_amdgcn_ldexpf(acc2[j][r], e);
+      for (int r = 0; r < 16; ++r)
+        acc2[j][r] = __builtin_amdgcn_ldexpf(acc2[j][r], -(e + expS[wr * 32 + fm_mfma32_row(r, lane)]));
     }
   }
   if constexpr (WAVE_OUT) {

@@ -195,7 +195,12 @@ int fm_resblock(const float* x, int batch, int length, int channels, const float
  * callers held to an absolute bar (the decoder's waveform), not for the
  * encoder, whose codes depend on exact activations.  FM_WEIGHTS_H3 with
  * FM_ACT_EXP runs the block on the fp16 planes after the bf16 ones (three
- * products, fm_split_weights_h3); without FM_ACT_EXP it is ignored. */
+ * products, fm_split_weights_h3); without FM_ACT_EXP it is ignored.  Each input
+ * row then has its own power-of-two scale and each hidden row one from a bound
+ * on it ((the largest |ELU(x)| of its three input rows) * channels * max |w1| +
+ * max |b1|, 2^14 of it at most): an element keeps 2^-23 of itself or 2^-39 of
+ * its row's largest (of that bound, for a hidden element), whatever the other
+ * rows hold. */
 
 /*
  * The SEANet encoder's first conv (1 -> 64 channels, kernel 7, causal, no

@@ -247,6 +247,64 @@ def test_resblock(C, B, L, kind):
     assert err <= 1.1 * was + 1e-7 * want.norm()
 
 
+def run_block(x, w1, b1, w2, b2):
+    """fm_resblock on the fp16 planes: [B, C, L] on the CPU."""
+    B, C, L = x.shape
+    c1, c2 = _Conv(w1.to(DEV), b1.to(DEV)), _Conv(w2.to(DEV), b2.to(DEV))
+    (w1p, _), (w2p, _) = with_planes(c1.w), with_planes(c2.w)
+    xd = x.transpose(1, 2).contiguous().to(DEV)
+    y = torch.full_like(xd, float("nan"))
+    nat.call("fm_resblock", xd.data_ptr(), B, L, C, w1p.data_ptr(), c1.b.data_ptr(), w2p.data_ptr(), c2.b.data_ptr(),
+             FLAGS | nat.ACT_EXP, y.data_ptr(), stream())
+    torch.cuda.synchronize()
+    return y.cpu().transpose(1, 2)
+
+
+@pytest.mark.parametrize("C,B,L", [(64, 1, 300), (64, 2, 127), (128, 1, 131), (128, 2, 64), (256, 1, 97), (256, 3, 5)])
+@pytest.mark.parametrize("outlier", [False, True])
+def test_resblock_rows_keep_their_own_accuracy(C, B, L, outlier):
+    """Rows from 1e-12 to 1e12 side by side, each held to its own sums:
+    positive inputs and first weights keep both ELUs exact, so only the
+    contractions' 1e-5 of the sum of magnitudes is allowed (the residual's
+    rounding, 2^-24, is within it).  ``outlier``: one hidden channel 1e4 above
+    the others, whose second weights weigh it down again; the others then keep
+    2^-39 * 2^6 * 1e4 = 1.2e-6 of what they are."""
+    g = torch.Generator().manual_seed(C + L)
+    x = torch.rand(B, C, L, generator=g) + 0.1
+    x *= 10.0 ** (24 * torch.rand(B, 1, L, generator=g) - 12)
+    x[:, :, L // 2:L // 2 + 4] = 0
+    w1 = (torch.rand(C // 2, C, 3, generator=g) + 0.1) / (3 * C)
+    w2 = torch.randn(C, C // 2, 1, generator=g) / math.sqrt(C // 2)
+    if outlier:
+        w1[1] *= 1e4
+        w2[:, 1] *= 1e-4
+    zero1, zero2 = torch.zeros(C // 2), torch.zeros(C)
+    want, absref = block_reference(*(t.double() for t in (x, w1, zero1, w2, zero2)))
+    close_dot(run_block(x, w1, zero1, w2, zero2), want, absref)
+
+
+@pytest.mark.parametrize("C,L", [(64, 300), (128, 150), (256, 70)])
+def test_resblock_rows_are_independent(C, L):
+    """A loud, an infinite and a NaN row change the rows that read them (its own
+    and the next two) and no bit of any other, before or after."""
+    g = torch.Generator().manual_seed(C)
+    x = torch.randn(1, C, L, generator=g)
+    w1, b1 = torch.randn(C // 2, C, 3, generator=g) / math.sqrt(3 * C), 0.1 * torch.randn(C // 2, generator=g)
+    w2, b2 = torch.randn(C, C // 2, 1, generator=g) / math.sqrt(C // 2), 0.1 * torch.randn(C, generator=g)
+    plain = run_block(x, w1, b1, w2, b2)
+    loud = x.clone()
+    rows = (0, 20, L // 2, L - 1)
+    loud[:, :, 0] *= 1e7
+    loud[:, :, 20] *= 1e20
+    loud[:, 3, L // 2] = float("inf")
+    loud[:, 5, L - 1] = float("nan")
+    got = run_block(loud, w1, b1, w2, b2)
+    own = torch.ones(L, dtype=torch.bool)
+    for r in rows:
+        own[r:r + 3] = False
+    assert torch.equal(got[..., own], plain[..., own])
+
+
 @pytest.mark.parametrize("B,L,y_len", [(1, 1000, 1000), (2, 129, 100), (3, 33, 33), (1, 1, 1)])
 def test_resblock64_conv(B, L, y_len):
     """The decoder's last block and waveform conv on fp16 weights."""
