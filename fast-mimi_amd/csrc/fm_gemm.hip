@@ -1940,21 +1940,31 @@ void record_plan(int id, bool elu, long tiles, int splits) {
 void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tiles, int& splits) {
   const long t128 = tile_count(M, p.N, kH3);
   const bool k32 = p.C_in % 32 == 0 && p.K % 32 == 0, k64 = p.C_in % 64 == 0 && p.K % 64 == 0;
-  // Smallest power-of-two split that reaches 320 blocks, >= min_k deep.
-  auto fewest = [&](long t, int most, int min_k) {
-    int sp = 1;
-    while (workspace && sp < most && t * sp < 320 && p.K / (2 * sp) >= min_k) sp *= 2;
-    return sp;
+  // K splits: a block for every CU, at least 128 deep, and from K = 1024 on up
+  // to the 512 blocks that are resident at once (both tiles that split hold
+  // two per CU), at least 256 deep.  Never more than are resident: a nearly
+  // empty second round and larger partials cost more than the unsplit tile
+  // (us, blocks in brackets; 160 rows x 1536 x 1024: 17.7 (576), 14.0 (288);
+  // 1030 x 512 x 2048: 32.1 (544), 23.7 (408); 1500 x 1536 x 1024: 41.0 (576),
+  // 32.0 (432); 3000 x 1536 x 1024: 61.4 (576), 48.7 (288); 4600 x 512 x 2048:
+  // 60.6 (576), 47.0 (432); 1700 x 640 x 512: 22.6 (540), 15.5 (270)).  At K =
+  // 512 a second block per CU does not pay for its partials (1250 x 640: 13.4
+  // unsplit, 15.5 in 400 blocks).
+  auto splits_for = [&](long t) {
+    if (!workspace) return 1;
+    const long one = std::min({16L, 256 / t, p.K / 128L});
+    const long two = p.K >= 1024 ? std::min({8L, 512 / t, p.K / 256L}) : 1L;
+    return (int)std::max({one, two, 1L});
   };
   splits = 1;
   if (!k32 || t128 > 512) {
     cfg = kH3;
   } else if (p.K >= 1024 ? t128 >= 64 : t128 >= 192) {
     // Long K: 64 tiles x 8 splits 30 us against 77 us unsplit (250 rows of
-    // the stride-8 upsampling), 192 x 2 40 against 43, 256 x 2 109 against
-    // 129, 128 x 4 (fc2 at 4000 rows) 43 against 78.
+    // the stride-8 upsampling), 180 x 2 37 against 43, 256 x 2 72 against
+    // 87, 128 x 4 (fc2 at 4000 rows) 43 against 78.
     cfg = kH3K32;
-    if (p.K >= 1024) splits = fewest(t128, 8, 256);
+    if (p.K >= 1024) splits = splits_for(t128);
   } else if (!k64) {
     cfg = kH3Small;
   } else {
@@ -1964,7 +1974,7 @@ void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tile
     // fc1, 576 tiles: 20.7 us, 64x128 23.4).
     const long t64 = tile_count(M, p.N, kH3Tiny);
     cfg = t64 > 512 ? kH3Tiny32 : kH3Tiny;
-    if (p.K >= 512) splits = fewest(t64, 16, 128);
+    if (p.K >= 512) splits = splits_for(t64);
   }
   tiles = tile_count(M, p.N, cfg);
 }

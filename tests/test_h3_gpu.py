@@ -108,6 +108,26 @@ def test_linear_tiles(rows, k, n, plan, ws):
               res.double().abs() + scale.double().abs() * (x.double().abs() @ w.double().abs().t()))
 
 
+@pytest.mark.parametrize("rows,k,n,plan", [
+    (160, 1024, 1536, "tiles=72 splits=4"), (1030, 2048, 512, "tiles=136 splits=3"), (250, 2048, 4096, "tiles=64 splits=8"),
+    (1500, 1024, 1536, "tiles=144 splits=3"), (3000, 1024, 1536, "tiles=288 splits=1"), (4600, 2048, 512, "tiles=144 splits=3"),
+    (8200, 2048, 512, "tiles=260 splits=1"), (8192, 2048, 512, "tiles=256 splits=2"), (776, 512, 640, "tiles=130 splits=1"),
+    (1700, 512, 640, "tiles=270 splits=1"), (400, 512, 640, "tiles=70 splits=3"), (1, 2048, 512, "tiles=8 splits=16"),
+    (1000, 1536, 256, "tiles=64 splits=6"), (8300, 1536, 256, "tiles=130 splits=3"), (100, 1088, 512, "tiles=16 splits=6"),
+])
+def test_splits_stay_resident(rows, k, n, plan, ws):
+    """K splits never put more blocks into a launch than the chip holds at once
+    (two per CU), any number of splits adds up, and short last splits too."""
+    tiles, splits = (int(item.split("=")[1]) for item in plan.split())
+    assert splits == 1 or tiles * splits <= 512
+    g = torch.Generator().manual_seed(rows + k)
+    x = torch.randn(rows, k, generator=g).to(DEV)
+    w, _ = with_planes((torch.randn(n, k, generator=g) / math.sqrt(k)).to(DEV))
+    got = linear(x, w, ws)
+    assert "gemm_h3_kernel" in nat.last_gemm_plan() and plan in nat.last_gemm_plan(), nat.last_gemm_plan()
+    close_dot(got, x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t())
+
+
 @pytest.mark.parametrize("rows,k,n", [(200, 512, 256), (2500, 512, 1536), (2500, 512, 512), (70000, 128, 128), (1100, 512, 2048)])
 def test_row_scales(rows, k, n, ws):
     """Rows from 1e-30 to 1e30 side by side, rows that start with zeros, rows
