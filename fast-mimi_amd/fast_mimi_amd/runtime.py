@@ -210,17 +210,6 @@ class MimiRuntime:
             self.screen_info = torch.empty((len(prefixes), 2), dtype=torch.int32, device=device)
             ops.call("fm_rvq_prepare_screen", self.embeds, self.norms, e, d, len(prefixes), self.screen,
                      self.screen_info)
-        # Fragment-packed copies of the projection weights for the few-row kernels,
-        # keyed by the row-major weight's device address.
-        self._packed: dict[int, torch.Tensor] = {}
-        lib = nat.library()
-        for w in [m for lay in self.enc_tf + self.dec_tf for m in (lay.wqkv, lay.wo, lay.w1, lay.w2)] + \
-                [self.w_in, self.w_out]:
-            n, k = w.shape
-            if lib.fm_row_linear_supported(k, n):
-                pw = torch.empty_like(w)
-                ops.call("fm_pack_row_weights", w, n, k, pw)
-                self._packed[w.data_ptr()] = pw
         # Convolution and large-row projection weights carry their bf16x6
         # planes: W^T followed by [3][N][K] bf16 in one buffer.
         self._x6: dict[int, torch.Tensor] = {}
@@ -238,6 +227,17 @@ class MimiRuntime:
                 wx = self._x6[w.data_ptr()] = self._with_planes(w, h3)
                 if h3 and wx is not w:
                     self._h3.add(w.data_ptr())
+        # Fragment-packed copies of the projection weights that the few-row kernels
+        # read in FP32, keyed by the row-major weight's device address.
+        self._packed: dict[int, torch.Tensor] = {}
+        lib = nat.library()
+        for w in [m for lay in self.enc_tf + self.dec_tf for m in (lay.wqkv, lay.wo, lay.w1, lay.w2)] + \
+                [self.w_in, self.w_out]:
+            n, k = w.shape
+            if lib.fm_row_linear_supported(k, n) and self._row_planes(w) is None:
+                pw = torch.empty_like(w)
+                ops.call("fm_pack_row_weights", w, n, k, pw)
+                self._packed[w.data_ptr()] = pw
         # Which layers took planes, checked against the declared plan (a layer
         # without planes would silently run its FP32 kernels instead).
         self.x6_layers = {name: bool(layer.flags & nat.WEIGHTS_X6) for name, layer in self._named_conv_layers()}
@@ -290,7 +290,9 @@ class MimiRuntime:
         """``w`` [N, K] (FP32 W^T) as the first N*K floats of a buffer that
         continues with its three bf16 planes (``fm_split_weights``) and, with
         ``h3``, its fp16 planes (``fm_split_weights_h3``); ``w`` itself when K
-        is not a multiple of 16."""
+        is not a multiple of 16.  (A decoder weight's bf16 planes, 6 bytes a
+        weight, serve what the fp16 kernels do not take: under 32 columns, other
+        depths of the few-row convolutions, planes beyond a 2 GiB buffer.)"""
         rows, cols = w.shape
         if cols % 16:
             return w
@@ -375,6 +377,17 @@ class MimiRuntime:
             return self._row_linear(x, rows, w, flags, residual, scale, out)
         return self._linear(x, rows, w, flags, residual, scale, out)
 
+    def _row_planes(self, w):
+        """The planes a few-row projection runs on, or None for its FP32
+        fragment-packed kernel.  16-bit matrix cores where they measured faster
+        at 250 rows: the fp16 planes of the decoder's projections always; bf16x6
+        for the wide 512-deep ones (qkv 7.5 vs 9.4 us, fc1 7.7 vs 9.6 us), while
+        the output projection (3.5 vs 3.4 us) and the streamed fc2 (8.1 vs 8.1
+        us) keep the FP32 kernel."""
+        n, k = w.shape
+        planes = w.data_ptr() in self._h3 or (k == 512 and n >= 1024)
+        return self._x6.get(w.data_ptr()) if planes else None
+
     def _row_linear(self, x, rows, w, flags=0, residual=None, scale=None, out=None, ln=None,
                     rope=None):
         """Transformer projection with LayerNorm prologue / RoPE epilogue fused."""
@@ -383,13 +396,8 @@ class MimiRuntime:
         g, b = (ln[0], ln[1]) if ln is not None else (None, None)
         cos, sin, rope_cols, per_seq = rope if rope is not None else (None, None, 0, 1)
         few = rows <= _ROW16_MAX_ROWS
-        # 16-bit matrix cores where they measured faster at 250 rows: the fp16
-        # planes of the decoder's projections always; bf16x6 for the wide
-        # 512-deep ones (qkv 7.5 vs 9.4 us, fc1 7.7 vs 9.6 us), while the
-        # output projection (3.5 vs 3.4 us) and the streamed fc2 (8.1 vs 8.1
-        # us) keep the FP32 fragment-packed kernel.
         h3 = w.data_ptr() in self._h3
-        wx = self._x6.get(w.data_ptr()) if few and (h3 or (k == 512 and n >= 1024)) else None
+        wx = self._row_planes(w) if few else None
         packed = self._packed.get(w.data_ptr()) if few else None
         if wx is not None:  # 16-row blocks on the 16-bit matrix cores
             name, wp, flags = "fm_row_linear", wx, flags | nat.WEIGHTS_X6 | (nat.WEIGHTS_H3 if h3 else 0)

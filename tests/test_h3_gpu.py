@@ -16,6 +16,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from fast_mimi_amd import MimiModel
 from fast_mimi_amd import _native as nat
 from fast_mimi_amd.config import MimiConfig
 from fast_mimi_amd.runtime import _Conv, _ConvT, rope_tables
@@ -455,3 +456,20 @@ def test_few_rows_reach_the_ends_of_fp32(kind, k, n, rows, weight_exp):
     want = causal_conv1d(x.double(), w.double(), torch.zeros(n, dtype=torch.float64))
     close_dot(y.cpu().transpose(1, 2), want, causal_conv1d(x.double().abs(), w.double().abs(),
                                                            torch.zeros(n, dtype=torch.float64)))
+
+
+def test_every_packed_copy_is_read():
+    """A few-row round trip reads each fragment-packed projection the runtime
+    keeps: none beside the 16-bit planes that replace it."""
+    model = MimiModel(MimiConfig(num_hidden_layers=2), device=DEV, use_graphs=False)
+    rt = model.runtime()
+    read = set()
+
+    def call(name, *args):
+        if name.startswith("fm_row_linear_packed"):
+            read.add(args[6 if name == "fm_row_linear_packed" else 3].data_ptr())
+        return type(rt)._call(rt, name, *args)
+
+    rt._call = call
+    model.decode(model.encode(torch.randn(1, 1, 24_000, device=DEV)).audio_codes)
+    assert rt._packed and {t.data_ptr() for t in rt._packed.values()} == read
