@@ -1912,8 +1912,8 @@ const char* kernel_name(int id, bool elu) {
     case 19: return elu ? "gemm_x6d_kernel<192,128,6,2,2,true>" : "gemm_x6d_kernel<192,128,6,2,2,false>";
     case 20: return "gemm_x6d_kernel<128,128,4,2,2,false,2>";
     case 22: return "gemm_x6d_kernel<192,128,6,2,2,false,2>";
-    case 24: return elu ? "gemm_h3_kernel<128,128,2,2,1,4,true>" : "gemm_h3_kernel<128,128,2,2,1,4,false>";
-    case 25: return elu ? "gemm_h3_kernel<128,128,4,2,2,4,true>" : "gemm_h3_kernel<128,128,4,2,2,4,false>";
+    case 24: return elu ? "gemm_h3_kernel<128,128,4,1,1,4,true>" : "gemm_h3_kernel<128,128,2,2,1,4,false>";
+    case 25: return elu ? "gemm_h3_kernel<128,128,4,1,2,2,true>" : "gemm_h3_kernel<128,128,4,2,2,4,false>";
     case 26: return elu ? "gemm_h3_kernel<64,128,2,2,2,3,true>" : "gemm_h3_kernel<64,128,2,2,2,3,false>";
     case 27: return elu ? "gemm_h3_kernel<64,64,2,2,4,2,true>" : "gemm_h3_kernel<64,64,2,2,4,2,false>";
     case 28: return elu ? "gemm_h3_kernel<64,64,2,2,2,4,true>" : "gemm_h3_kernel<64,64,2,2,2,4,false>";
@@ -1939,10 +1939,11 @@ void record_plan(int id, bool elu, long tiles, int splits) {
 // 16 x 1536 x 1024: 15.7 -> 10.
 void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tiles, int& splits) {
   const long t128 = tile_count(M, p.N, kH3);
+  const bool elu = p.flags & FM_ELU_IN;
   const bool k32 = p.C_in % 32 == 0 && p.K % 32 == 0, k64 = p.C_in % 64 == 0 && p.K % 64 == 0;
   // K splits: a block for every CU, at least 128 deep, and from K = 1024 on up
   // to the 512 blocks that are resident at once (both tiles that split hold
-  // two per CU), at least 256 deep.  Never more than are resident: a nearly
+  // two per CU), at least min_k deep.  Never more than are resident: a nearly
   // empty second round and larger partials cost more than the unsplit tile
   // (us, blocks in brackets; 160 rows x 1536 x 1024: 17.7 (576), 14.0 (288);
   // 1030 x 512 x 2048: 32.1 (544), 23.7 (408); 1500 x 1536 x 1024: 41.0 (576),
@@ -1950,21 +1951,23 @@ void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tile
   // 60.6 (576), 47.0 (432); 1700 x 640 x 512: 22.6 (540), 15.5 (270)).  At K =
   // 512 a second block per CU does not pay for its partials (1250 x 640: 13.4
   // unsplit, 15.5 in 400 blocks).
-  auto splits_for = [&](long t) {
+  auto splits_for = [&](long t, long min_k) {
     if (!workspace) return 1;
     const long one = std::min({16L, 256 / t, p.K / 128L});
-    const long two = p.K >= 1024 ? std::min({8L, 512 / t, p.K / 256L}) : 1L;
+    const long two = p.K >= 1024 ? std::min({8L, 512 / t, p.K / min_k}) : 1L;
     return (int)std::max({one, two, 1L});
   };
   splits = 1;
   if (!k32 || t128 > 512) {
     cfg = kH3;
-  } else if (p.K >= 1024 ? t128 >= 64 : t128 >= 192) {
+  } else if (p.K >= 1024 ? t128 >= (elu ? 36 : 64) : t128 >= 192) {
     // Long K: 64 tiles x 8 splits 30 us against 77 us unsplit (250 rows of
     // the stride-8 upsampling), 180 x 2 37 against 43, 256 x 2 72 against
-    // 87, 128 x 4 (fc2 at 4000 rows) 43 against 78.
+    // 87, 128 x 4 (fc2 at 4000 rows) 43 against 78.  With ELU on load, which
+    // the smaller tiles evaluate twice, from fewer tiles on: 512 channels, k3,
+    // 3000 rows 30 us against 40 in 64x64 tiles.
     cfg = kH3K32;
-    if (p.K >= 1024) splits = splits_for(t128);
+    if (p.K >= 1024) splits = splits_for(t128, elu ? 192 : 256);
   } else if (!k64) {
     cfg = kH3Small;
   } else {
@@ -1974,7 +1977,7 @@ void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tile
     // fc1, 576 tiles: 20.7 us, 64x128 23.4).
     const long t64 = tile_count(M, p.N, kH3Tiny);
     cfg = t64 > 512 ? kH3Tiny32 : kH3Tiny;
-    if (p.K >= 512) splits = splits_for(t64);
+    if (p.K >= 512) splits = splits_for(t64, 256);
   }
   tiles = tile_count(M, p.N, cfg);
 }
@@ -2002,11 +2005,15 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
   const bool big_ok = p.N % 4 == 0 && !(p.bias && p.bias_len % 4);
   const TileCfg big = p.N >= 128 ? kBigSquare : kBigTile;
   const long big_tiles = tile_count(M, p.N, big);
+  // (With ELU on load and long K, the bf16x6 tile over 1300-2300 rows of 256
+  // columns: 1800 rows 22.7 us against 26.6, 2000 rows 24.8 against 27.0.)
+  const bool h3_elu_gap = (p.flags & FM_ELU_IN) && (p.flags & FM_WEIGHTS_X6) && workspace && big_ok && p.K >= 1024 &&
+                          M >= 1024 && tile_count(M, p.N, kH3) >= 20 && tile_count(M, p.N, kH3) < 36;
   // fp16 planes: the h3 tiles take every such contraction they can address
   // (weight planes and a tile's rows behind 32-bit buffer offsets) with
-  // columns enough to fill a fragment.
+  // columns enough to fill a fragment, that gap excepted.
   const bool h3 = (p.flags & FM_WEIGHTS_H3) && !(p.flags & FM_REPLICATE) && p.C_in % 16 == 0 && p.K % 16 == 0 &&
-                  p.N >= 32 && 4L * p.K * p.N <= 0x7fffffffL && 257L * p.N * 4 <= 0x7fffffffL;
+                  p.N >= 32 && 4L * p.K * p.N <= 0x7fffffffL && 257L * p.N * 4 <= 0x7fffffffL && !h3_elu_gap;
   if (h3) {
     pick_h3(M, p, workspace != nullptr, cfg, tiles, splits);
   } else if (!fast) {
@@ -2248,10 +2255,14 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
       hipLaunchKernelGGL((gemm_x6d_kernel<192, 128, 6, 2, 2, false, 2>), grid, dim3(768), 0, s, p,
                          reinterpret_cast<const __bf16*>(p.w + (long)p.N * p.K));
       break;
-#define FM_H3(BM_, BN_, WM_, WN_, KS_, WPE_, ROPE_)                                                          \
-  if (p.flags & FM_ELU_IN)                                                                                   \
-    hipLaunchKernelGGL((gemm_h3_kernel<BM_, BN_, WM_, WN_, KS_, WPE_, true>), grid, dim3(64 * WM_ * WN_), 0, \
-                       s, p, wh);                                                                            \
+// ELU on load (E*): in the 128x128 tiles four waves of 32 x 128, so each A
+// element's ELU and split run once (512 -> 256 channels, k3: 32000 rows 143 ->
+// 107 us, 64000 rows 267 -> 208, 16000 rows 82 -> 67, against waves that share rows;
+// bf16x6 142, 278, 95).
+#define FM_H3(BM_, BN_, WM_, WN_, KS_, WPE_, ROPE_, EWM_, EWN_, EWPE_)                                          \
+  if (p.flags & FM_ELU_IN)                                                                                      \
+    hipLaunchKernelGGL((gemm_h3_kernel<BM_, BN_, EWM_, EWN_, KS_, EWPE_, true>), grid, dim3(64 * EWM_ * EWN_), 0, \
+                       s, p, wh);                                                                               \
   else if (ROPE_ && (p.flags & FM_EPI_ROPE))                                                                 \
     hipLaunchKernelGGL((gemm_h3_kernel<BM_, BN_, WM_, WN_, KS_, WPE_, false, ROPE_>), grid,                  \
                        dim3(64 * WM_ * WN_), 0, s, p, wh);                                                   \
@@ -2261,12 +2272,12 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
     case 24:
       if (M * p.N * 4 > (256L << 20) && !p.partial && !(p.flags & (FM_ELU_IN | FM_EPI_ROPE)))
         hipLaunchKernelGGL((gemm_h3_kernel<128, 128, 2, 2, 1, 4, false, false, true>), grid, dim3(256), 0, s, p, wh);
-      else FM_H3(128, 128, 2, 2, 1, 4, true);
+      else FM_H3(128, 128, 2, 2, 1, 4, true, 4, 1, 4);
       break;
-    case 25: FM_H3(128, 128, 4, 2, 2, 4, true); break;
-    case 26: FM_H3(64, 128, 2, 2, 2, 3, true); break;
-    case 27: FM_H3(64, 64, 2, 2, 4, 2, false); break;
-    case 28: FM_H3(64, 64, 2, 2, 2, 4, false); break;
+    case 25: FM_H3(128, 128, 4, 2, 2, 4, true, 4, 1, 2); break;
+    case 26: FM_H3(64, 128, 2, 2, 2, 3, true, 2, 2, 3); break;
+    case 27: FM_H3(64, 64, 2, 2, 4, 2, false, 2, 2, 2); break;
+    case 28: FM_H3(64, 64, 2, 2, 2, 4, false, 2, 2, 4); break;
 #undef FM_H3
     case 7: hipLaunchKernelGGL((gemm_mid_kernel<64, 64, 1>), grid, dim3(NTHREADS), 0, s, p); break;
     case 8: hipLaunchKernelGGL((gemm_mid_kernel<32, 32, 4>), grid, dim3(NTHREADS), 0, s, p); break;

@@ -129,6 +129,30 @@ def test_splits_stay_resident(rows, k, n, plan, ws):
     close_dot(got, x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t())
 
 
+@pytest.mark.parametrize("rows,plan", [
+    (1, "gemm_h3_kernel<64,64,2,2,4,2,true> tiles=4 splits=12"), (1100, "gemm_h3_kernel<64,64,2,2,4,2,true> tiles=72 splits=6"),
+    (1300, "gemm_x6d_kernel<"), (2176, "gemm_x6d_kernel<"), (2177, "gemm_h3_kernel<128,128,4,1,2,2,true> tiles=36 splits=8"),
+    (8161, "gemm_h3_kernel<128,128,4,1,2,2,true> tiles=128 splits=4"), (32700, "gemm_h3_kernel<128,128,4,1,2,2,true> tiles=512 splits=1"),
+    (32800, "gemm_h3_kernel<128,128,4,1,1,4,true> tiles=514 splits=1"),
+])
+def test_elu_on_load_tiles(rows, plan, ws):
+    """The 512-channel residual block's k3 conv (256 columns, ELU on load) over
+    its tiles and the gap that stays on the bf16 form."""
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, 512, generator=g).to(DEV)
+    wt = torch.randn(256, 3 * 512, generator=g).to(DEV) / math.sqrt(1536)
+    w, _ = with_planes(wt)
+    b = torch.randn(256, generator=g).to(DEV)
+    y = torch.full((rows, 256), float("nan"), device=DEV)
+    nat.call("fm_conv1d", x.data_ptr(), 1, rows, 512, w.data_ptr(), b.data_ptr(), 256, 3, 1, 0, FLAGS | nat.ELU_IN, None,
+             y.data_ptr(), rows, ws.data_ptr(), WS_BYTES, stream())
+    torch.cuda.synchronize()
+    assert plan in nat.last_gemm_plan(), nat.last_gemm_plan()
+    a = F.pad(F.elu(x.double()), (0, 0, 2, 0))
+    taps = torch.cat([a[j:j + rows] for j in range(3)], 1)
+    close_dot(y, taps @ wt.double().t() + b.double(), taps.abs() @ wt.double().abs().t() + b.double().abs())
+
+
 @pytest.mark.parametrize("rows,k,n", [(200, 512, 256), (2500, 512, 1536), (2500, 512, 512), (70000, 128, 128), (1100, 512, 2048)])
 def test_row_scales(rows, k, n, ws):
     """Rows from 1e-30 to 1e30 side by side, rows that start with zeros, rows
