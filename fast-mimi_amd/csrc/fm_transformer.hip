@@ -1719,7 +1719,14 @@ int fm_row_linear(const float* x, int rows, int in_features, const float* ln_gam
     const float* planes = weight + (long)out_features * in_features;
     const dim3 g64(out_features / 64, (rows + 15) / 16), g32(out_features / 32, (rows + 15) / 16);
     const bool wide = rope_cos || (long)(out_features / 32) * ((rows + 15) / 16) > 512;
-    if (flags & FM_WEIGHTS_H3) {
+    // fp16 planes, but for the wide 512-deep projections while their blocks are
+    // at most one per CU: there nothing hides the step that scales the rows
+    // (us, fp16 / bf16: qkv with RoPE 5.23 / 5.15 at 26 rows, 5.49 / 5.38 at 160,
+    // 7.41 / 7.57 at 200; fc1 4.3 / 4.1 at 26 rows, 4.5 / 4.2 at 64, 5.63 / 5.58 at
+    // 65, 5.82 / 5.92 at 128).
+    const bool few_blocks = in_features == 512 && out_features >= 1024 &&
+                            (long)(out_features / (wide ? 64 : 32)) * ((rows + 15) / 16) <= 256;
+    if ((flags & FM_WEIGHTS_H3) && !few_blocks) {
       const float* h3 = planes + 3L * out_features * in_features / 2;
 #define FM_R16H3(KK, BN, G)                                                                                       \
   hipLaunchKernelGGL((row16_linear_kernel<KK, BN, true, false, true>), G, dim3(512), 0, stream, x, rows, ln_gamma, \

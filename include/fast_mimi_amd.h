@@ -91,9 +91,11 @@ int fm_split_weights(const float* weight_packed, int rows, int cols, void* plane
  * row.  The error against float64 is that of FP32 sums (below the bf16x6
  * form's); results differ from it in the last bits, so callers whose codes
  * depend on exact sums keep FM_WEIGHTS_X6 alone.  fm_row_linear and
- * fm_conv1d_rows (in_channels * kernel 256, 1536 or 3584; else the bf16
- * form) take the flag together with FM_WEIGHTS_X6, and fm_resblock /
- * fm_resblock64_conv together with FM_ACT_EXP.
+ * fm_conv1d_rows take the flag together with FM_WEIGHTS_X6, and fm_resblock /
+ * fm_resblock64_conv together with FM_ACT_EXP.  Where the bf16 form is the
+ * faster one (fm_conv1d_rows with in_channels * kernel other than 1536 and 3584
+ * and at some row counts of those, fm_row_linear's 512-deep projections of 1024
+ * and more columns at few rows), a call with both flags runs that form.
  * No reference counterpart (as fm_split_weights).
  */
 int fm_split_weights_h3(const float* weight_packed, int rows, int cols, void* planes, hipStream_t stream);

@@ -497,3 +497,36 @@ def test_every_packed_copy_is_read():
     rt._call = call
     model.decode(model.encode(torch.randn(1, 1, 24_000, device=DEV)).audio_codes)
     assert rt._packed and {t.data_ptr() for t in rt._packed.values()} == read
+
+
+@pytest.mark.parametrize("kind,k,n,rows,fp16", [
+    ("conv", 1, 512, 26, False), ("conv", 1, 512, 2000, False),                               # K = 256
+    ("conv", 3, 256, 26, True), ("conv", 3, 256, 1008, True), ("conv", 3, 256, 1024, False),  # K = 1536: two-tile blocks
+    ("conv", 3, 256, 1040, True),
+    ("conv", 7, 1024, 26, True), ("conv", 7, 1024, 256, True), ("conv", 7, 1024, 257, False),  # K = 3584: 64 columns
+    ("row", 512, 2048, 1, False), ("row", 512, 2048, 64, False), ("row", 512, 2048, 65, True),
+    ("row", 512, 1536, 80, False), ("row", 512, 1536, 81, True), ("row", 512, 512, 1, True), ("row", 2048, 512, 1, True),
+    ("rope", 512, 1536, 160, False), ("rope", 512, 1536, 161, True),
+])
+def test_few_rows_take_the_faster_form(kind, k, n, rows, fp16):
+    """With both plane sets the call is the bf16 form bit for bit where that one
+    is the faster, and the fp16 form elsewhere."""
+    g = torch.Generator().manual_seed(rows + n)
+    cin = k if kind != "conv" else 256 if k == 1 else 512
+    taps = k if kind == "conv" else 1
+    x = torch.randn(rows, cin, generator=g).to(DEV)
+    w, _ = with_planes(torch.randn(n, cin * taps, generator=g).to(DEV))
+    cos, sin = (t.to(DEV) for t in rope_tables(MimiConfig(), rows))
+    out = []
+    for flags in (FLAGS, nat.WEIGHTS_X6):
+        y = torch.full((rows, n), float("nan"), device=DEV)
+        if kind == "conv":
+            nat.call("fm_conv1d_rows", x.data_ptr(), 1, rows, cin, w.data_ptr(), None, 0, n, k, 1, 0, flags, None,
+                     y.data_ptr(), stream())
+        else:
+            rope = (cos.data_ptr(), sin.data_ptr(), 1024) if kind == "rope" else (None, None, 0)
+            nat.call("fm_row_linear", x.data_ptr(), rows, cin, None, None, 1e-5, w.data_ptr(), n, flags, None, None,
+                     *rope, rows, y.data_ptr(), stream())
+        torch.cuda.synchronize()
+        out.append(y)
+    assert torch.isfinite(out[0]).all() and torch.equal(*out) != fp16
