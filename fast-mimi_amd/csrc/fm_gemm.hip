@@ -1941,21 +1941,19 @@ void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tile
   const long t128 = tile_count(M, p.N, kH3);
   const bool elu = p.flags & FM_ELU_IN;
   const bool k32 = p.C_in % 32 == 0 && p.K % 32 == 0, k64 = p.C_in % 64 == 0 && p.K % 64 == 0;
-  // K splits: a block for every CU, at least 128 deep, and from K = 1024 on up
-  // to the 512 blocks that are resident at once (both tiles that split hold
-  // two per CU), at least min_k deep.  Never more than are resident: a nearly
-  // empty second round and larger partials cost more than the unsplit tile
-  // (us, blocks in brackets; 160 rows x 1536 x 1024: 17.7 (576), 14.0 (288);
-  // 1030 x 512 x 2048: 32.1 (544), 23.7 (408); 1500 x 1536 x 1024: 41.0 (576),
-  // 32.0 (432); 3000 x 1536 x 1024: 61.4 (576), 48.7 (288); 4600 x 512 x 2048:
-  // 60.6 (576), 47.0 (432); 1700 x 640 x 512: 22.6 (540), 15.5 (270)).  At K =
-  // 512 a second block per CU does not pay for its partials (1250 x 640: 13.4
-  // unsplit, 15.5 in 400 blocks).
-  auto splits_for = [&](long t, long min_k) {
-    if (!workspace) return 1;
-    const long one = std::min({16L, 256 / t, p.K / 128L});
-    const long two = p.K >= 1024 ? std::min({8L, 512 / t, p.K / min_k}) : 1L;
-    return (int)std::max({one, two, 1L});
+  // K splits, at least min_k deep: doubled until 320 blocks, but no further than
+  // the 512 that are resident at once (both tiles that split hold two per CU);
+  // where the doubling would pass them, the fewest splits that reach 320.  Past
+  // them a nearly empty second round and larger partials cost more than the
+  // splits give (us, blocks in brackets; 1500 x 1536 x 1024: 41.0 (576), 32.0
+  // (432); 3000 x 1536 x 1024: 61.4 (576), 48.7 (288); 1030 x 512 x 2048: 32.1
+  // (544), 23.7 (408); 1700 x 640 x 512: 22.6 (540), 15.5 (270); an eight-layer
+  // transformer at 2100 rows, 68 tiles for fc2: 1274 (544), 1193 (476), 1161
+  // (340); at 2560 rows, 80 tiles: 1256 (480), 1233 (400), 1233 (320)).
+  auto splits_for = [&](long t, int most, int min_k) {
+    int sp = 1;
+    while (workspace && sp < most && t * sp < 320 && p.K / (2 * sp) >= min_k) sp *= 2;
+    return t * sp > 512 && sp > 1 ? (int)std::min((320 + t - 1) / t, 512 / t) : sp;
   };
   splits = 1;
   if (!k32 || t128 > 512) {
@@ -1967,7 +1965,7 @@ void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tile
     // the smaller tiles evaluate twice, from fewer tiles on: 512 channels, k3,
     // 3000 rows 30 us against 40 in 64x64 tiles.
     cfg = kH3K32;
-    if (p.K >= 1024) splits = splits_for(t128, elu ? 192 : 256);
+    if (p.K >= 1024) splits = splits_for(t128, 8, elu ? 192 : 256);
   } else if (!k64) {
     cfg = kH3Small;
   } else {
@@ -1977,7 +1975,7 @@ void pick_h3(long M, const GemmArgs& p, bool workspace, TileCfg& cfg, long& tile
     // fc1, 576 tiles: 20.7 us, 64x128 23.4).
     const long t64 = tile_count(M, p.N, kH3Tiny);
     cfg = t64 > 512 ? kH3Tiny32 : kH3Tiny;
-    if (p.K >= 512) splits = splits_for(t64, 256);
+    if (p.K >= 512) splits = splits_for(t64, 16, 128);
   }
   tiles = tile_count(M, p.N, cfg);
 }

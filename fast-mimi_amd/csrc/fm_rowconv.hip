@@ -92,6 +92,9 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
     const _Float16* wh = reinterpret_cast<const _Float16*>(p.w + (long)p.N * K + 3L * p.N * K / 2);
     const long PL = (long)p.N * K;
     const _Float16* wbh = wh + ((long)((kw0 >> 4) + (g >> 1)) * p.N + n0 + li) * 16 + 8 * (g & 1);
+    int ce[NT];  // this lane's columns' weight exponents, read ahead of the ring
+#pragma unroll
+    for (int j = 0; j < NT; ++j) ce[j] = reinterpret_cast<const int*>(wh + 2 * PL)[n0 + 16 * j + li];
     halfx8 bu[R][NT];
     auto load_unit = [&](int buf, int u) {
 #pragma unroll
@@ -101,9 +104,6 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
     };
 #pragma unroll
     for (int u = 0; u < R; ++u) load_unit(u, u);
-    int ce[NT];  // this lane's columns' weight exponents
-#pragma unroll
-    for (int j = 0; j < NT; ++j) ce[j] = reinterpret_cast<const int*>(wh + 2 * PL)[n0 + 16 * j + li];
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) {
       floatx4 ah[MT][CS][2];
@@ -362,17 +362,20 @@ int fm_conv1d_rows(const float* x, int batch, int length, int in_channels, const
   // 21.1 us at C2; with fewer blocks the CUs left idle cost more than the
   // halved weight reads save).
   const bool two = !wide && (long)(out_channels / 32) * row_blocks >= 512;
-  // The decoder's depths on fp16 planes, in the same blocks, but for the forms
-  // where the bf16 planes measured faster (us, fp16 / bf16): K = 256, a step or
-  // two of products per wave (250 rows 3.7 / 3.5, 2000 rows 9.2 / 9.1); K = 3584
-  // in 64-column blocks, which take every register and spill (257-272 rows
-  // 30.4 / 26.9); K = 1536 in two-tile blocks (1024 rows 11.9 / 11.6).
-  if ((flags & FM_WEIGHTS_H3) && ((K == 1536 && !two) || (K == 3584 && !wide))) {
+  // The decoder's depths on fp16 planes, in the same blocks, but for K = 3584 in
+  // 64-column blocks: those take every register and spill (257-272 rows 28.5 us
+  // on fp16 planes, 26.6 on bf16).
+  if ((flags & FM_WEIGHTS_H3) && (K == 256 || K == 1536 || (K == 3584 && !wide))) {
 #define FM_ROWCONVH3(KK, BN, MT, G) hipLaunchKernelGGL((row16_conv_kernel<KK, BN, true, MT, true>), G, dim3(512), 0, stream, p)
-    if (K == 1536 && wide) FM_ROWCONVH3(1536, 64, 2, grid64);
-    else if (K == 1536) FM_ROWCONVH3(1536, 32, 1, grid);
+#define FM_ROWCONVH3K(KK)                         \
+  if (two) FM_ROWCONVH3(KK, 32, 2, grid32r);      \
+  else if (wide) FM_ROWCONVH3(KK, 64, 2, grid64); \
+  else FM_ROWCONVH3(KK, 32, 1, grid)
+    if (K == 256) { FM_ROWCONVH3K(256); }
+    else if (K == 1536) { FM_ROWCONVH3K(1536); }
     else if (two) FM_ROWCONVH3(3584, 32, 2, grid32r);
     else FM_ROWCONVH3(3584, 32, 1, grid);
+#undef FM_ROWCONVH3K
 #undef FM_ROWCONVH3
     return (int)hipGetLastError();
   }

@@ -1300,7 +1300,7 @@ __global__ __launch_bounds__(512) void row_stream_linear_kernel(
 // exponents, fm_split_weights_h3) and three v_mfma_f32_16x16x32_f16 products
 // per fragment pair.  A wave reads its whole k-range of the 16 rows first, takes
 // a power of two per row from it, and its partial tile returns to the caller's
-// scale as it goes to LDS: row and column exponents in one step (in two, sums
+// scale as it is summed: row and column exponents in one step (in two, sums
 // near FP32's upper end overflow on the way).  A chain of
 // latencies (weight loads, products, cross-wave sum), so halving the MFMAs takes
 // off little (250 rows: qkv 9.1 -> 8.6 us, fc1 9.2 -> 8.5, fc2 10.0 -> 9.6, the
@@ -1385,10 +1385,14 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
   const bool rope = BN == 64 && cos_t && n0 < rope_cols;
   const bool res_scale = flags & FM_EPI_RES_SCALE;
   float e_res[OPT], e_scale[OPT], e_cos[OPT], e_sin[OPT];
+  int e_col[OPT];  // H3: the columns' weight exponents
+  // H3: each wave's exponent of each row.
+  __shared__ __attribute__((aligned(16))) int row_exp[H3 ? BM : 1][NWV];
   auto fetch_epilogue = [&]() {
 #pragma unroll
     for (int c = 0; c < OPT; ++c) {
       const int n = n0 + ec + c;
+      if constexpr (H3) e_col[c] = reinterpret_cast<const int*>(wp + (long)N * K)[n];
       e_res[c] = res_scale ? res[mc * N + n] : 0.0f;
       e_scale[c] = res_scale ? scale[n] : 0.0f;
       e_cos[c] = rope ? cos_t[(long)tpos * 64 + ec + c] : 0.0f;
@@ -1409,9 +1413,16 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
     float out[OPT];
 #pragma unroll
     for (int c = 0; c < OPT; ++c) {
-      float v = red[er * PR + ec + c];
+      // H3: each partial sum returns to the caller's scale here, by its wave's row
+      // exponent and the column's in one step.
+      auto part = [&](int q) {
+        const float v = red[(q * BM + er) * PR + ec + c];
+        if constexpr (H3) return __builtin_amdgcn_ldexpf(v, -(row_exp[er][q] + e_col[c]));
+        else return v;
+      };
+      float v = part(0);
 #pragma unroll
-      for (int q = 1; q < NWV; ++q) v = __fadd_rn(v, red[(q * BM + er) * PR + ec + c]);
+      for (int q = 1; q < NWV; ++q) v = __fadd_rn(v, part(q));
       out[c] = v;
     }
     if (rope || UPS) {
@@ -1497,10 +1508,8 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
           ah[st][h] = *reinterpret_cast<const floatx4*>(As + li * PA + kw0 + 32 * st + 8 * g + 4 * h);
     }
     fetch_epilogue();
-    int ce[NT];  // this lane's columns' weight exponents
-#pragma unroll
-    for (int j = 0; j < NT; ++j) ce[j] = reinterpret_cast<const int*>(wh + 2 * PL)[n0 + 16 * j + li];
     const int se = h3_row_exp16(ah);
+    if (g == 0) row_exp[li][wave] = se;
     const float sc = __builtin_amdgcn_ldexpf(1.0f, se);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1517,12 +1526,6 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
       for (int pl = 0; pl < 2; ++pl)
         if (2 * st + pl + R < NU) load_unit((2 * st + pl) % R, 2 * st + pl + R);
       __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int e = -__shfl(se, 4 * g + r, 64);
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j][r] = __builtin_amdgcn_ldexpf(acc[j][r], e - ce[j]);
     }
     reduce_and_store(acc);
     return;
@@ -1719,14 +1722,7 @@ int fm_row_linear(const float* x, int rows, int in_features, const float* ln_gam
     const float* planes = weight + (long)out_features * in_features;
     const dim3 g64(out_features / 64, (rows + 15) / 16), g32(out_features / 32, (rows + 15) / 16);
     const bool wide = rope_cos || (long)(out_features / 32) * ((rows + 15) / 16) > 512;
-    // fp16 planes, but for the wide 512-deep projections while their blocks are
-    // at most one per CU: there nothing hides the step that scales the rows
-    // (us, fp16 / bf16: qkv with RoPE 5.23 / 5.15 at 26 rows, 5.49 / 5.38 at 160,
-    // 7.41 / 7.57 at 200; fc1 4.3 / 4.1 at 26 rows, 4.5 / 4.2 at 64, 5.63 / 5.58 at
-    // 65, 5.82 / 5.92 at 128).
-    const bool few_blocks = in_features == 512 && out_features >= 1024 &&
-                            (long)(out_features / (wide ? 64 : 32)) * ((rows + 15) / 16) <= 256;
-    if ((flags & FM_WEIGHTS_H3) && !few_blocks) {
+    if (flags & FM_WEIGHTS_H3) {
       const float* h3 = planes + 3L * out_features * in_features / 2;
 #define FM_R16H3(KK, BN, G)                                                                                       \
   hipLaunchKernelGGL((row16_linear_kernel<KK, BN, true, false, true>), G, dim3(512), 0, stream, x, rows, ln_gamma, \

@@ -380,9 +380,8 @@ class MimiRuntime:
     def _row_planes(self, w):
         """The planes a few-row projection runs on, or None for its FP32
         fragment-packed kernel.  16-bit matrix cores where they measured faster
-        at 250 rows: all of the decoder's projections, whose fp16 planes the
-        kernel takes where they are the faster; bf16x6 for the encoder's wide
-        512-deep ones (qkv 7.5 vs 9.4 us, fc1 7.7 vs 9.6 us), while
+        at 250 rows: the fp16 planes of the decoder's projections always;
+        bf16x6 for the encoder's wide 512-deep ones (qkv 7.5 vs 9.4 us, fc1 7.7 vs 9.6 us), while
         the output projection (3.5 vs 3.4 us) and the streamed fc2 (8.1 vs 8.1
         us) keep the FP32 kernel."""
         n, k = w.shape

@@ -93,9 +93,9 @@ int fm_split_weights(const float* weight_packed, int rows, int cols, void* plane
  * depend on exact sums keep FM_WEIGHTS_X6 alone.  fm_row_linear and
  * fm_conv1d_rows take the flag together with FM_WEIGHTS_X6, and fm_resblock /
  * fm_resblock64_conv together with FM_ACT_EXP.  Where the bf16 form is the
- * faster one (fm_conv1d_rows with in_channels * kernel other than 1536 and 3584
- * and at some row counts of those, fm_row_linear's 512-deep projections of 1024
- * and more columns at few rows), a call with both flags runs that form.
+ * faster one (fm_conv1d_rows with in_channels * kernel other than 256, 1536 and
+ * 3584 and at some row counts of 3584; fm_conv1d with FM_ELU_IN at some), a
+ * call with both flags runs that form.
  * No reference counterpart (as fm_split_weights).
  */
 int fm_split_weights_h3(const float* weight_packed, int rows, int cols, void* planes, hipStream_t stream);
