@@ -510,11 +510,15 @@ __global__ __launch_bounds__(NT, 3) void resblock_direct_kernel(
 // the loudest one's, so a row's result depends on its own three input rows
 // alone.  Accumulators return to the caller's scale in one exact step.  Two
 // planes of ELU(x) take 33 KB, so four blocks share a CU instead of three, and
-// half the MFMAs go: 60000 rows of 128 channels
-// 31.1 -> 25.7 us; 16 clips of 10 s, 64 channels 616 -> 512 us (486 with the
-// waveform conv), 128 channels 432 -> 345, 256 channels 359 -> 276.  (One scale
-// for a block's rows measured 507, 478, 341 and 270 us there, but took bits
-// from quiet rows beside a loud one.)
+// half the MFMAs go: 60000 rows of 128 channels 31.2 -> 25.8 us; 16 clips of
+// 10 s, 64 channels 626 -> 523 us (495 with the waveform conv), 128 channels
+// 435 -> 350, 256 channels 358 -> 280.  (One scale for a block's rows measured
+// 516, 484, 345 and 274 us there, but took bits from quiet rows beside a loud
+// one.)  A unit's small products are issued before its large ones: rounded into
+// a sum still small, they leave the error against float64 at 0.95 / 0.86 / 0.74
+// of the bf16 form's (64 / 128 / 256 channels).  A second accumulator for them
+// lowers it to 0.93 / 0.76 / 0.63, but without registers for a second set of
+// input fragments takes 3% more time.
 template <int C, int BM, int WM, int PD, bool WAVE_IN, bool WAVE_OUT, bool FAST_ACT = false, bool H3 = false>
 __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     const float* __restrict__ x, int L, const __bf16* __restrict__ w1x, const float* __restrict__ b1,
@@ -745,14 +749,19 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     if (u + 1 < T1) load_x(u + 1, xf[(u + 1) & 1]);
     const frag8(&w)[NP][2] = ring[u % PD];
     const frag8(&a)[NP][2] = xf[u & 1];
+    if constexpr (H3) {
+      // The small products first: rounded into a sum still small.
+      floatx16& acc = acc1[u >= TU];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      if constexpr (H3) {
-        floatx16& acc = acc1[u >= TU];
+      for (int s = 0; s < 2; ++s) {
         acc = fm_mfma32_f16(w[1][s], a[0][s], acc);
         acc = fm_mfma32_f16(w[0][s], a[1][s], acc);
-        acc = fm_mfma32_f16(w[0][s], a[0][s], acc);
-      } else {
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) acc = fm_mfma32_f16(w[0][s], a[0][s], acc);
+    } else {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
         acc1[0] = fm_mfma32_bf16(w[1][s], a[1][s], acc1[0]);
         acc1[1] = fm_mfma32_bf16(w[2][s], a[0][s], acc1[1]);
         acc1[0] = fm_mfma32_bf16(w[1][s], a[0][s], acc1[0]);
@@ -864,13 +873,17 @@ __global__ __launch_bounds__(NT, H3 ? 4 : 3) void resblock_x6_kernel(
     for (int j = 0; j < FN2; ++j) {
       const int u = T1 + kt * FN2 + j;
       const frag8(&w)[NP][2] = ring[u % PD];
+      if constexpr (H3) {
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        if constexpr (H3) {
+        for (int s = 0; s < 2; ++s) {
           acc2[j] = fm_mfma32_f16(a[1][s], w[0][s], acc2[j]);
           acc2[j] = fm_mfma32_f16(a[0][s], w[1][s], acc2[j]);
-          acc2[j] = fm_mfma32_f16(a[0][s], w[0][s], acc2[j]);
-        } else {
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) acc2[j] = fm_mfma32_f16(a[0][s], w[0][s], acc2[j]);
+      } else {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
           acc2[j] = fm_mfma32_bf16(a[1][s], w[1][s], acc2[j]);
           acc2[j] = fm_mfma32_bf16(a[2][s], w[0][s], acc2[j]);
           acc2[j] = fm_mfma32_bf16(a[1][s], w[0][s], acc2[j]);
