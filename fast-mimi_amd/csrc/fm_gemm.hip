@@ -1599,6 +1599,21 @@ void gemm_h3_kernel(GemmArgs p, const _Float16* __restrict__ wh) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
+  // SMALL: a1b0 and a0b1 are summed by themselves, so that the sum of the large
+  // products is rounded once per 16 k instead of three times (error against
+  // float64 over the former FP32 or bf16x6 plan's, in one sum / in two: 240 x 256
+  // x 256 1.28 / 0.87, 300 x 1024 x 3584 1.43 / 0.90, 2600 x 256 x 1536 1.48 / 0.92).
+  // The four-blocks-per-CU tiles have no registers for it; the plans they replace
+  // sum as many terms in one chain (0.71-0.80 of their error).
+  constexpr bool SMALL = FM * FN <= 2 || WPE <= 2;
+  floatx16 low[SMALL ? FM : 1][SMALL ? FN : 1];
+#pragma unroll
+  for (int i = 0; i < (SMALL ? FM : 1); ++i)
+#pragma unroll
+    for (int j = 0; j < (SMALL ? FN : 1); ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) low[i][j][r] = 0.0f;
+
   const int lrow = lane & 31, lk = lane >> 5;
   // Per fragment row (lanes l and l + 32 hold one row): its scale 2^s, s, and
   // the magnitude it covers (0: the row has been zero so far).
@@ -1671,7 +1686,10 @@ void gemm_h3_kernel(GemmArgs p, const _Float16* __restrict__ wh) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j) scale_rows(i, 0, acc[i][j]);
+          for (int j = 0; j < FN; ++j) {
+            scale_rows(i, 0, acc[i][j]);
+            if constexpr (SMALL) scale_rows(i, 0, low[i][j]);
+          }
       }
       halfx8 a0[FM], a1[FM], b0[FN], b1[FN];
 #pragma unroll
@@ -1686,11 +1704,20 @@ void gemm_h3_kernel(GemmArgs p, const _Float16* __restrict__ wh) {
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          acc[i][j] = fm_mfma32_f16(a1[i], b0[j], acc[i][j]);
-          acc[i][j] = fm_mfma32_f16(a0[i], b1[j], acc[i][j]);
+          floatx16& lo = SMALL ? low[SMALL ? i : 0][SMALL ? j : 0] : acc[i][j];
+          lo = fm_mfma32_f16(a1[i], b0[j], lo);
+          lo = fm_mfma32_f16(a0[i], b1[j], lo);
           acc[i][j] = fm_mfma32_f16(a0[i], b0[j], acc[i][j]);
         }
     }
+  }
+  if constexpr (SMALL) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = __fadd_rn(acc[i][j][r], low[i][j][r]);
   }
   // Back to the caller's scale: 2^-(s_row + s_column) in one exact step.
   wave_lds_fence();
@@ -2003,10 +2030,10 @@ int run_gemm(GemmArgs p, float* workspace, size_t workspace_bytes, hipStream_t s
   const bool big_ok = p.N % 4 == 0 && !(p.bias && p.bias_len % 4);
   const TileCfg big = p.N >= 128 ? kBigSquare : kBigTile;
   const long big_tiles = tile_count(M, p.N, big);
-  // (With ELU on load and long K, the bf16x6 tile over 1300-2300 rows of 256
-  // columns: 1800 rows 22.7 us against 26.6, 2000 rows 24.8 against 27.0.)
+  // (With ELU on load and long K, the bf16x6 tile over 1024-2176 rows of 256
+  // columns: 1100 rows 22.3 us against 23.1, 1800 rows 22.7 against 26.6.)
   const bool h3_elu_gap = (p.flags & FM_ELU_IN) && (p.flags & FM_WEIGHTS_X6) && workspace && big_ok && p.K >= 1024 &&
-                          M >= 1024 && tile_count(M, p.N, kH3) >= 20 && tile_count(M, p.N, kH3) < 36;
+                          M >= 1024 && tile_count(M, p.N, kH3) < 36;
   // fp16 planes: the h3 tiles take every such contraction they can address
   // (weight planes and a tile's rows behind 32-bit buffer offsets) with
   // columns enough to fill a fragment, that gap excepted.

@@ -126,13 +126,22 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
       }
       int se[MT];
       float sc[MT];
-      floatx4 part[MT][NT];
+      // low: a1b0 and a0b1, summed by themselves (rounded into a small sum) where
+      // that does not spill.
+      constexpr bool SMALL = MT * NT <= 4;
+      floatx4 part[MT][NT], low[SMALL ? MT : 1][SMALL ? NT : 1];
+      auto small = [&](int mt, int j) -> floatx4& {
+        return SMALL ? low[SMALL ? mt : 0][SMALL ? j : 0] : part[mt][j];
+      };
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         se[mt] = h3_row_exp16(ah[mt]);
         sc[mt] = __builtin_amdgcn_ldexpf(1.0f, se[mt]);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) part[mt][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < NT; ++j) {
+          part[mt][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+          if constexpr (SMALL) low[mt][j] = part[mt][j];
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -143,11 +152,11 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
           halfx8 p0v, p1v;
           split2(ah[mt][st][0], ah[mt][st][1], sc[mt], p0v, p1v);
 #pragma unroll
-          for (int j = 0; j < NT; ++j) part[mt][j] = fm_mfma16_f16(p1v, bu[u % R][j], part[mt][j]);
+          for (int j = 0; j < NT; ++j) small(mt, j) = fm_mfma16_f16(p1v, bu[u % R][j], small(mt, j));
 #pragma unroll
           for (int j = 0; j < NT; ++j) part[mt][j] = fm_mfma16_f16(p0v, bu[u % R][j], part[mt][j]);
 #pragma unroll
-          for (int j = 0; j < NT; ++j) part[mt][j] = fm_mfma16_f16(p0v, bu[(u + 1) % R][j], part[mt][j]);
+          for (int j = 0; j < NT; ++j) small(mt, j) = fm_mfma16_f16(p0v, bu[(u + 1) % R][j], small(mt, j));
         }
 #pragma unroll
         for (int pl = 0; pl < 2; ++pl)
@@ -160,8 +169,11 @@ __global__ __launch_bounds__(512) void row16_conv_kernel(RowConvArgs p) {
         for (int r = 0; r < 4; ++r) {
           const int e = -__shfl(se[mt], 4 * g + r, 64);
 #pragma unroll
-          for (int j = 0; j < NT; ++j)
-            acc[mt][j][r] = __fadd_rn(acc[mt][j][r], __builtin_amdgcn_ldexpf(part[mt][j][r], e - ce[j]));
+          for (int j = 0; j < NT; ++j) {
+            float v = part[mt][j][r];
+            if constexpr (SMALL) v = __fadd_rn(v, low[mt][j][r]);
+            acc[mt][j][r] = __fadd_rn(acc[mt][j][r], __builtin_amdgcn_ldexpf(v, e - ce[j]));
+          }
         }
     }
   } else if constexpr (X6) {
@@ -364,18 +376,15 @@ int fm_conv1d_rows(const float* x, int batch, int length, int in_channels, const
   const bool two = !wide && (long)(out_channels / 32) * row_blocks >= 512;
   // The decoder's depths on fp16 planes, in the same blocks, but for K = 3584 in
   // 64-column blocks: those take every register and spill (257-272 rows 28.5 us
-  // on fp16 planes, 26.6 on bf16).
-  if ((flags & FM_WEIGHTS_H3) && (K == 256 || K == 1536 || (K == 3584 && !wide))) {
+  // on fp16 planes, 26.6 on bf16), and for K = 256, so short a sum that the two
+  // pieces' own error shows (2-norm against float64 1.17e-7, bf16 1.12e-7).
+  if ((flags & FM_WEIGHTS_H3) && (K == 1536 || (K == 3584 && !wide))) {
 #define FM_ROWCONVH3(KK, BN, MT, G) hipLaunchKernelGGL((row16_conv_kernel<KK, BN, true, MT, true>), G, dim3(512), 0, stream, p)
-#define FM_ROWCONVH3K(KK)                         \
-  if (two) FM_ROWCONVH3(KK, 32, 2, grid32r);      \
-  else if (wide) FM_ROWCONVH3(KK, 64, 2, grid64); \
-  else FM_ROWCONVH3(KK, 32, 1, grid)
-    if (K == 256) { FM_ROWCONVH3K(256); }
-    else if (K == 1536) { FM_ROWCONVH3K(1536); }
+    if (K == 1536 && two) FM_ROWCONVH3(1536, 32, 2, grid32r);
+    else if (K == 1536 && wide) FM_ROWCONVH3(1536, 64, 2, grid64);
+    else if (K == 1536) FM_ROWCONVH3(1536, 32, 1, grid);
     else if (two) FM_ROWCONVH3(3584, 32, 2, grid32r);
     else FM_ROWCONVH3(3584, 32, 1, grid);
-#undef FM_ROWCONVH3K
 #undef FM_ROWCONVH3
     return (int)hipGetLastError();
   }

@@ -1508,6 +1508,9 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
           ah[st][h] = *reinterpret_cast<const floatx4*>(As + li * PA + kw0 + 32 * st + 8 * g + 4 * h);
     }
     fetch_epilogue();
+    floatx4 low[NT];  // a1b0 and a0b1, summed by themselves (rounded into a small sum)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) low[j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     const int se = h3_row_exp16(ah);
     if (g == 0) row_exp[li][wave] = se;
     const float sc = __builtin_amdgcn_ldexpf(1.0f, se);
@@ -1517,16 +1520,20 @@ __global__ __launch_bounds__(512) void row16_linear_kernel(
       halfx8 p0, p1;
       split2(ah[st][0], ah[st][1], sc, p0, p1);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j] = fm_mfma16_f16(p1, bu[2 * st % R][j], acc[j]);
+      for (int j = 0; j < NT; ++j) low[j] = fm_mfma16_f16(p1, bu[2 * st % R][j], low[j]);
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[j] = fm_mfma16_f16(p0, bu[2 * st % R][j], acc[j]);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j] = fm_mfma16_f16(p0, bu[(2 * st + 1) % R][j], acc[j]);
+      for (int j = 0; j < NT; ++j) low[j] = fm_mfma16_f16(p0, bu[(2 * st + 1) % R][j], low[j]);
 #pragma unroll
       for (int pl = 0; pl < 2; ++pl)
         if (2 * st + pl + R < NU) load_unit((2 * st + pl) % R, 2 * st + pl + R);
       __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[j][r] = __fadd_rn(acc[j][r], low[j][r]);
     reduce_and_store(acc);
     return;
   }

@@ -131,8 +131,8 @@ def test_splits_stay_resident(rows, k, n, plan, ws):
 
 
 @pytest.mark.parametrize("rows,plan", [
-    (1, "gemm_h3_kernel<64,64,2,2,4,2,true> tiles=4 splits=8"), (1100, "gemm_h3_kernel<64,64,2,2,4,2,true> tiles=72 splits=5"),
-    (1300, "gemm_x6d_kernel<"), (2176, "gemm_x6d_kernel<"), (2177, "gemm_h3_kernel<128,128,4,1,2,2,true> tiles=36 splits=8"),
+    (1, "gemm_h3_kernel<64,64,2,2,4,2,true> tiles=4 splits=8"), (1023, "gemm_h3_kernel<64,64,2,2,4,2,true> tiles=64 splits=8"),
+    (1024, "gemm_x6d_kernel<"), (2176, "gemm_x6d_kernel<"), (2177, "gemm_h3_kernel<128,128,4,1,2,2,true> tiles=36 splits=8"),
     (8161, "gemm_h3_kernel<128,128,4,1,2,2,true> tiles=128 splits=4"), (32700, "gemm_h3_kernel<128,128,4,1,2,2,true> tiles=512 splits=1"),
     (32800, "gemm_h3_kernel<128,128,4,1,1,4,true> tiles=514 splits=1"),
 ])
@@ -501,7 +501,7 @@ def test_every_packed_copy_is_read():
 
 
 @pytest.mark.parametrize("kind,k,n,rows,fp16", [
-    ("conv", 1, 512, 26, True), ("conv", 3, 256, 1024, True), ("conv", 7, 1024, 26, True), ("conv", 7, 1024, 256, True),
+    ("conv", 1, 512, 26, False), ("conv", 1, 512, 2000, False), ("conv", 3, 256, 1024, True), ("conv", 7, 1024, 26, True), ("conv", 7, 1024, 256, True),
     ("conv", 7, 1024, 257, False), ("conv", 7, 1024, 272, False), ("row", 512, 2048, 1, True), ("row", 512, 512, 1, True),
     ("row", 2048, 512, 1, True), ("rope", 512, 1536, 1, True), ("rope", 512, 1536, 512, True),
 ])
@@ -527,3 +527,48 @@ def test_few_rows_take_the_faster_form(kind, k, n, rows, fp16):
         torch.cuda.synchronize()
         out.append(y)
     assert torch.isfinite(out[0]).all() and torch.equal(*out) != fp16
+
+
+@pytest.mark.parametrize("kind,rows,k,n", [
+    ("gemm", 240, 256, 256), ("gemm", 6240, 256, 256), ("gemm", 208, 1024, 1536), ("gemm", 1248, 512, 640),
+    ("gemm", 1030, 2048, 512), ("gemm", 2500, 2048, 512), ("gemm", 300, 3584, 1024), ("gemm", 2600, 1536, 256),
+    ("gemm", 9000, 256, 512), ("gemm", 70000, 256, 256), ("elu", 600, 1536, 256), ("elu", 2600, 1536, 256),
+    ("elu", 33000, 1536, 256), ("conv", 26, 256, 512), ("conv", 26, 1536, 256), ("conv", 2000, 1536, 256),
+    ("conv", 26, 3584, 1024), ("conv", 250, 3584, 1024), ("row", 26, 512, 2048), ("row", 250, 512, 1536),
+    ("packed", 26, 512, 512), ("packed", 250, 2048, 512),
+])
+@pytest.mark.parametrize("spread", [0.0, 2.0])
+def test_no_further_from_float64_than_before(kind, rows, k, n, spread, ws):
+    """The 2-norm error of the fp16 form against float64 is at most that of the
+    form it replaces at the same size: the bf16x6 or FP32 plan, and the
+    fragment-packed FP32 kernel ("packed").  ``spread``: rows scaled by e^(2 z)."""
+    g = torch.Generator(device=DEV).manual_seed(rows + k)
+    taps = {"elu": 3, "conv": 1 if k == 256 else k // 512}.get(kind, 1)
+    x = torch.randn(rows, k // taps, device=DEV, generator=g)
+    x *= torch.exp(spread * torch.randn(rows, 1, device=DEV, generator=g))
+    wt = torch.randn(n, k, device=DEV, generator=g) / math.sqrt(k)
+    w, _ = with_planes(wt)
+    packed = torch.empty_like(wt)
+    nat.call("fm_pack_row_weights", wt.data_ptr(), n, k, packed.data_ptr(), stream())
+    errs = []
+    for flags in (FLAGS, nat.WEIGHTS_X6):
+        y = torch.full((rows, n), float("nan"), device=DEV)
+        if kind == "gemm":
+            y = linear(x, w, ws, flags)
+        elif kind == "elu":
+            nat.call("fm_conv1d", x.data_ptr(), 1, rows, k // 3, w.data_ptr(), None, n, 3, 1, 0, flags | nat.ELU_IN, None,
+                     y.data_ptr(), rows, ws.data_ptr(), WS_BYTES, stream())
+        elif kind == "conv":
+            nat.call("fm_conv1d_rows", x.data_ptr(), 1, rows, k // taps, w.data_ptr(), None, 0, n, taps, 1, 0, flags, None,
+                     y.data_ptr(), stream())
+        else:
+            name, wp, f = "fm_row_linear", w, flags
+            if kind == "packed" and flags != FLAGS:
+                name, wp, f = "fm_row_linear_packed", packed, 0
+            nat.call(name, x.data_ptr(), rows, k, None, None, 1e-5, wp.data_ptr(), n, f, None, None, None, None, 0, 1,
+                     y.data_ptr(), stream())
+        torch.cuda.synchronize()
+        a = F.pad(F.elu(x.double()) if kind == "elu" else x.double(), (0, 0, taps - 1, 0))
+        want = torch.cat([a[j:j + rows] for j in range(taps)], 1) @ wt.double().t()
+        errs.append(((y.double() - want).norm() / want.norm()).item())
+    assert errs[0] <= errs[1], f"{errs[0]:.3e} against {errs[1]:.3e}"
