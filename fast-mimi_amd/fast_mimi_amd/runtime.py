@@ -227,17 +227,29 @@ class MimiRuntime:
                 wx = self._x6[w.data_ptr()] = self._with_planes(w, h3)
                 if h3 and wx is not w:
                     self._h3.add(w.data_ptr())
-        # Fragment-packed copies of the projection weights that the few-row kernels
-        # read in FP32, keyed by the row-major weight's device address.
+        # What a few-row projection runs as, keyed by the row-major weight's device
+        # address: (entry point, its weight, its plane flags).  16-bit matrix cores
+        # where they measured faster at 250 rows: the fp16 planes of the decoder's
+        # projections always; bf16x6 for the encoder's wide 512-deep ones (qkv 7.5
+        # vs 9.4 us, fc1 7.7 vs 9.6 us); fragment-packed FP32 for its output
+        # projection (3.5 vs 3.4 us) and fc2 (8.1 vs 8.1 us).
+        self._row_forms: dict[int, tuple] = {}
         self._packed: dict[int, torch.Tensor] = {}
         lib = nat.library()
         for w in [m for lay in self.enc_tf + self.dec_tf for m in (lay.wqkv, lay.wo, lay.w1, lay.w2)] + \
                 [self.w_in, self.w_out]:
             n, k = w.shape
-            if lib.fm_row_linear_supported(k, n) and self._row_planes(w) is None:
-                pw = torch.empty_like(w)
+            if not lib.fm_row_linear_supported(k, n):
+                continue
+            key = w.data_ptr()
+            wx = self._x6.get(key)
+            if wx is not None and (key in self._h3 or (k == 512 and n >= 1024)):
+                self._row_forms[key] = ("fm_row_linear", wx,
+                                        nat.WEIGHTS_X6 | (nat.WEIGHTS_H3 if key in self._h3 else 0))
+            else:
+                pw = self._packed[key] = torch.empty_like(w)
                 ops.call("fm_pack_row_weights", w, n, k, pw)
-                self._packed[w.data_ptr()] = pw
+                self._row_forms[key] = ("fm_row_linear_packed", pw, 0)
         # Which layers took planes, checked against the declared plan (a layer
         # without planes would silently run its FP32 kernels instead).
         self.x6_layers = {name: bool(layer.flags & nat.WEIGHTS_X6) for name, layer in self._named_conv_layers()}
@@ -377,17 +389,6 @@ class MimiRuntime:
             return self._row_linear(x, rows, w, flags, residual, scale, out)
         return self._linear(x, rows, w, flags, residual, scale, out)
 
-    def _row_planes(self, w):
-        """The planes a few-row projection runs on, or None for its FP32
-        fragment-packed kernel.  16-bit matrix cores where they measured faster
-        at 250 rows: the fp16 planes of the decoder's projections always;
-        bf16x6 for the encoder's wide 512-deep ones (qkv 7.5 vs 9.4 us, fc1 7.7 vs 9.6 us), while
-        the output projection (3.5 vs 3.4 us) and the streamed fc2 (8.1 vs 8.1
-        us) keep the FP32 kernel."""
-        n, k = w.shape
-        planes = w.data_ptr() in self._h3 or (k == 512 and n >= 1024)
-        return self._x6.get(w.data_ptr()) if planes else None
-
     def _row_linear(self, x, rows, w, flags=0, residual=None, scale=None, out=None, ln=None,
                     rope=None):
         """Transformer projection with LayerNorm prologue / RoPE epilogue fused."""
@@ -395,16 +396,9 @@ class MimiRuntime:
         y = torch.empty((rows, n), device=self.device) if out is None else out
         g, b = (ln[0], ln[1]) if ln is not None else (None, None)
         cos, sin, rope_cols, per_seq = rope if rope is not None else (None, None, 0, 1)
-        few = rows <= _ROW16_MAX_ROWS
-        h3 = w.data_ptr() in self._h3
-        wx = self._row_planes(w) if few else None
-        packed = self._packed.get(w.data_ptr()) if few else None
-        if wx is not None:  # 16-row blocks on the 16-bit matrix cores
-            name, wp, flags = "fm_row_linear", wx, flags | nat.WEIGHTS_X6 | (nat.WEIGHTS_H3 if h3 else 0)
-        elif packed is not None:
-            name, wp = "fm_row_linear_packed", packed
-        else:
-            name, wp = "fm_row_linear", w
+        form = self._row_forms.get(w.data_ptr()) if rows <= _ROW16_MAX_ROWS else None
+        name, wp, planes = form if form is not None else ("fm_row_linear", w, 0)
+        flags |= planes
         self._call(name, x, rows, k, g, b, self.config.norm_eps,
                    wp, n, flags, residual, scale, cos, sin,
                    rope_cols, per_seq, y)
