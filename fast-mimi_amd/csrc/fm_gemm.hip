@@ -1449,8 +1449,9 @@ void gemm_x6d_kernel(GemmArgs p, const __bf16* __restrict__ w3) {
 // the dropped a1b1 is below 2^-22 |a b| and of either sign.  Half of the
 // bf16x6 form's MFMA work, two planes in LDS instead of three and 28 vector
 // instructions per eight A elements instead of 44; with half as many roundings
-// into the FP32 accumulator its error against float64 is smaller too (rms over
-// the decoder's shapes 1.4-3.6e-7 of the output scale, bf16x6 1.7-4.9e-7).
+// into the FP32 accumulator, and one in six where the small products have their
+// own (SMALL below), its error against float64 is smaller too (rms over the
+// decoder's shapes 0.9-3.6e-7 of the output scale, the former plans' 1.5-4.9e-7).
 // fp16's range is what the scales are for:
 //   * a weight row n (one output column) is scaled by 2^s_n so that its largest
 //     magnitude lies in [2^13, 2^14) (fm_split_weights_h3; s_n is stored);

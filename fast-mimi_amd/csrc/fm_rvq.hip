@@ -922,7 +922,7 @@ __global__ __launch_bounds__(256) void rvq_decode_kernel(const int64_t* codes, i
 // Bound by the fp16 codebook stream, 1 MB per step and CU through the L1 port
 // (about two thirds of a step; the rest is the chain residual -> screen ->
 // candidates -> exact): 8000 rows x 32 codebooks 3.17 ms in step launches ->
-// 0.71 ms, 2000 rows x 8 0.27 -> 0.14 ms.
+// 0.46-0.56 ms, 2000 rows x 8 0.27 -> 0.14 ms.
 constexpr int SCREEN_WAVES = 8;
 constexpr int SCREEN_ENTRIES = 2048;     // 8 waves x 8 tiles x 32 entries: 7-bit tags
 constexpr int SCREEN_PAIRS = 512;        // exact candidates per block and step
