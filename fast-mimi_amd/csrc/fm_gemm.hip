@@ -1604,9 +1604,10 @@ void gemm_h3_kernel(GemmArgs p, const _Float16* __restrict__ wh) {
   // products is rounded once per 16 k instead of three times (error against
   // float64 over the former FP32 or bf16x6 plan's, in one sum / in two: 240 x 256
   // x 256 1.28 / 0.87, 300 x 1024 x 3584 1.43 / 0.90, 2600 x 256 x 1536 1.48 / 0.92).
-  // The four-blocks-per-CU tiles have no registers for it; the plans they replace
-  // sum as many terms in one chain (0.71-0.80 of their error).
-  constexpr bool SMALL = FM * FN <= 2 || WPE <= 2;
+  // Not in the 128x128 tiles of four waves per SIMD, which have no registers for
+  // it or lose 1% to it (a 2500-row transformer 1215 -> 1235 us): the plans those
+  // replace sum as many terms in one chain (one sum: 0.71-0.90 of their error).
+  constexpr bool SMALL = WPE != 4 || FM * FN == 1;
   floatx16 low[SMALL ? FM : 1][SMALL ? FN : 1];
 #pragma unroll
   for (int i = 0; i < (SMALL ? FM : 1); ++i)
